@@ -25,8 +25,7 @@ struct AttnArgs {
   // decode (T == 1): per (sequence, kv head) count of finished chunk blocks;
   // zero on entry, left zero on exit
   unsigned *ctr;
-  // prefill: first position of the rows as the host expects it; it sizes the
-  // key split and nothing else (the kernels read pos)
+  // prefill (launch_attention_prefill): position of the first row
   int plan_pos;
   // decode: every sequence's position is below pos_bound (0: no bound).  Only
   // the chunks below it are launched, and they load their cached rows before
@@ -92,27 +91,24 @@ int launch_rope_cur(const AttnArgs &a, hipStream_t st);
 int launch_attention(const AttnArgs &a, hipStream_t st);
 int attn_check(const AttnArgs &a);
 
-// Prefill attention for one sequence (B = 1) and many rows: RoPE of the rows'
-// q and k into qr [T][q_dim] / kr [T][kv_dim], a flash-attention pass on fp32
-// MFMA (one block per 16 rows and kv head, one wave per query head), then the
-// cache append of the rows.  Needs 4 query heads per kv head and head_dim
-// 128, 256 or 512 (prefill_flash_ok); a.part is not used.
-bool prefill_flash_ok(const AttnArgs &a);
-// Row tiles attending to many keys split their key tiles over several blocks
-// (so that the launch fills the CUs), merged by a second launch.  The split
-// plan follows T, cache_len, n_kv and a.plan_pos; the splits' partials need
-// flash_part_floats(a) floats of fpart (0: no split), never more than
-// flash_part_floats_max(hd).  With a smaller or null fpart the launch does not
-// split.
-struct FlashSplit {
-  int st_tiles;  // key tiles per split
-  int maxs;      // blocks per row tile (1: no split)
-  int n_rt;      // row tiles
-  float *part;   // per block: o [16 rows][4 heads][hd], then (max, sum) [16][4][2]
+// Prefill attention of T rows of one sequence (B = 1) at positions plan_pos ..
+// plan_pos + T - 1 (flash.hip): RoPE, causal attention over the cached keys and
+// the rows' own, and the cache append of the rows.  Any number of query heads
+// per kv head; a.part and a.pos are not used.  buf: flash_bytes(a) bytes of
+// workspace, never more than flash_bytes_max(a) at the same T, whatever the
+// position.
+struct FlashBuf {
+  int base, kbase;        // first row's position; first key of tile 0
+  int nkt, n_qt;          // 32-key tiles; tiles of 64 queries per kv head
+  int st_tiles, maxs;     // key tiles per split, splits per query tile (1: none)
+  int append;             // k_flash_prep appends the rows to the cache
+  _Float16 *q, *k, *v;    // split operands in MFMA fragment order
+  int32_t *qe;            // their exponents, per query
+  int2 *kve;              // and per key tile (k, v)
+  float *part;            // per split block: o [64][hd], then (max, sum) [64][2]
 };
-size_t flash_part_floats(const AttnArgs &a);
-size_t flash_part_floats_max(int hd);
-int launch_attention_prefill(const AttnArgs &a, float *qr, float *kr, float *fpart,
-                             size_t fpart_floats, hipStream_t st);
+size_t flash_bytes(const AttnArgs &a);
+size_t flash_bytes_max(const AttnArgs &a);
+int launch_attention_prefill(const AttnArgs &a, void *buf, size_t buf_bytes, hipStream_t st);
 
 }  // namespace ms

@@ -552,26 +552,6 @@ int launch_attention(const AttnArgs &a, hipStream_t st) {
 }
 
 
-// ------------------------------------------------------------------------------
-// Prefill attention: many rows of one sequence.
-//
-//  k_rope_rows      q and k of every row after RoPE (qr, kr).
-//  k_flash_prefill  one block per (16 rows, kv head), wave g = query head
-//                   h*4 + g.  Keys in tiles of 16: K (row pitch HD + 4) and V
-//                   transposed (V^T, pitch 20) staged in LDS, the next tile's
-//                   loads in registers while the current one computes.
-//                   S = Q K^T and O += P V on v_mfma_f32_16x16x4f32 (fp32
-//                   products, fp32 sums); online softmax with DPP row
-//                   reductions (the 16 keys of a score row sit in one 16-lane
-//                   row of the C fragment).  Keys older than the rows come
-//                   from the cache, the rows' own keys from kr / qkv.
-//  k_cache_append   the rows' k (after RoPE) and v into the cache, after every
-//                   block has read it (a circular window must not lose a key
-//                   an earlier row still needs).
-// The dot product runs over the head dims in the order d = 16u + 4c + r for
-// MFMA step 4u + r and k-group c, the same for q and k, so each lane loads its
-// q as float4 and reads K with one 16-byte LDS load per four steps.
-// ------------------------------------------------------------------------------
 typedef float af32x4 __attribute__((ext_vector_type(4)));
 
 template <int CTRL>
@@ -592,473 +572,6 @@ __device__ inline float row16_sum(float v) {
   v += adpp<0x4E>(v);
   v += adpp<0x141>(v);
   return v + adpp<0x140>(v);
-}
-
-// The same on float4 units (the rotated half of a head a multiple of 4):
-// unit u of a head is four rotation pairs (dims i .. i + 3 and half + i ..,
-// both rotated from one float4 of each half and of the tables) or four dims
-// past the rotary ones (copied).  Same arithmetic per value as rope_apply.
-__global__ __launch_bounds__(256) void k_rope_rows4(AttnArgs args, float *qr, float *kr,
-                                                    int hd) {
-  const AttnP p = load_params(args);
-  const int r = blockIdx.x;
-  const int pos = aldg<int32_t>(p.pos) + r;
-  const int rot = p.apply_rope ? p.rot : 0, half = rot >> 1;
-  const int pq = half >> 2, per = pq + ((hd - rot) >> 2);  // units per head
-  const int nh = p.n_heads + p.n_kv;
-  const float *row = p.qkv + (size_t)r * p.ld;
-  const float *ct = p.cos_t + (size_t)pos * half, *st = p.sin_t + (size_t)pos * half;
-  for (int u = threadIdx.x; u < nh * per; u += 256) {
-    const int head = u / per, j = u - head * per;
-    const bool isq = head < p.n_heads;
-    const int hk = isq ? head : head - p.n_heads;
-    const float *src = row + (isq ? 0 : p.q_dim) + hk * hd;
-    float *dst = isq ? qr + (size_t)r * p.q_dim + hk * hd : kr + (size_t)r * p.kv_dim + hk * hd;
-    if (j < pq) {
-      const int i = 4 * j;
-      const float4 xl = aldg<float4>(src + i), xh = aldg<float4>(src + half + i);
-      const float4 c = aldg<float4>(ct + i), sn = aldg<float4>(st + i);
-      *reinterpret_cast<float4 *>(dst + i) =
-          float4{xl.x * c.x - xh.x * sn.x, xl.y * c.y - xh.y * sn.y, xl.z * c.z - xh.z * sn.z,
-                 xl.w * c.w - xh.w * sn.w};
-      *reinterpret_cast<float4 *>(dst + half + i) =
-          float4{xl.x * sn.x + xh.x * c.x, xl.y * sn.y + xh.y * c.y, xl.z * sn.z + xh.z * c.z,
-                 xl.w * sn.w + xh.w * c.w};
-    } else {
-      const int d = rot + 4 * (j - pq);
-      *reinterpret_cast<float4 *>(dst + d) = aldg<float4>(src + d);
-    }
-  }
-}
-
-__global__ __launch_bounds__(256) void k_rope_rows(AttnArgs args, float *qr, float *kr, int hd) {
-  const AttnP p = load_params(args);
-  const int r = blockIdx.x;
-  const int pos = aldg<int32_t>(p.pos) + r;
-  const int nq = p.q_dim, nall = p.q_dim + p.kv_dim;
-#pragma unroll 4
-  for (int e = threadIdx.x; e < nall; e += 256) {
-    const bool isq = e < nq;
-    const int ee = isq ? e : e - nq;
-    const int head = ee / hd, d = ee - head * hd;
-    RopeIn ri;
-    rope_load(p, r, (isq ? 0 : nq) + head * hd, d, pos, ri);
-    const float v = rope_apply(ri);
-    if (isq)
-      qr[(size_t)r * nq + ee] = v;
-    else
-      kr[(size_t)r * p.kv_dim + ee] = v;
-  }
-}
-
-// DS waves per query head, each with 1/DS of the head dims (its q and o in
-// registers); their partial scores meet in LDS.
-template <int HD, int DS>
-constexpr int flash_lds_floats() {
-  return 16 * (HD + 4) + HD * 20 + 4 * DS * 16 * 20 + (DS > 1 ? 4 * DS * 256 : 0);
-}
-
-template <int HD, int DS>
-__global__ __launch_bounds__(256 * DS) void k_flash_prefill(AttnArgs args, const float *qr,
-                                                            const float *kr, FlashSplit fs) {
-  constexpr int NT = 256 * DS;
-  constexpr int HW = HD / DS;             // head dims per wave
-  constexpr int NU = HW / 16;             // q float4 per lane; O tiles of 16 dims
-  constexpr int KP = HD + 4;              // K row pitch (floats)
-  constexpr int VP = 20;                  // V^T row pitch
-  constexpr int PP = 20;                  // P row pitch
-  constexpr int NF = 16 * HD / 4 / NT;    // float4 of K (and of V) per thread per tile
-  extern __shared__ __align__(16) float fl[];
-  float *Ks = fl;                     // [16][KP]
-  float *VT = Ks + 16 * KP;           // [HD][VP]
-  float *Ps = VT + HD * VP;           // [4 DS][16][PP]
-  float *Sx = Ps + 4 * DS * 16 * PP;  // [4 DS][256] partial scores (DS > 1)
-  const AttnP p = load_params(args);
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
-  const int li = lane & 15, lk = lane >> 4;
-  const int g = wave / DS, hf = wave % DS;
-  // block j = (sp * n_rt + n_rt - 1 - rt) * n_kv + h: key split sp of row
-  // tile rt and kv head h.  Splits in order, the row tiles with the most keys
-  // first, the heads interleaved: the heavy blocks start first and the
-  // round-robin of blocks over the XCDs spreads every kind of block.
-  const int maxs = keep(fs.maxs), stt = keep(fs.st_tiles), n_rt = keep(fs.n_rt);
-  const int j = blockIdx.x;
-  const int h = j % p.n_kv, rt = n_rt - 1 - (j / p.n_kv) % n_rt, sp = j / (p.n_kv * n_rt);
-  const int hq = h * 4 + g;
-  const int d0 = hf * HW;  // first head dim of this wave
-  const int r0 = rt * 16;
-  const int base = aldg<int32_t>(p.pos);
-  const int rlast = min(r0 + 15, p.T - 1);
-  int klo, khi, dummy;
-  key_range(p, base + r0, &klo, &dummy);
-  key_range(p, base + rlast, &dummy, &khi);
-  const int kbeg = klo & ~15;
-  // the last split takes every remaining tile
-  const int nsplit = maxs == 1 ? 1 : min(maxs, ((khi - kbeg) / 16 + stt) / stt);
-  if (sp >= nsplit) return;
-  const int kfirst = kbeg + sp * stt * 16;
-  const int klast = sp == nsplit - 1 ? khi : kbeg + (sp + 1) * stt * 16 - 1;
-
-  // q rows of this wave (A operand, head dims in MFMA order)
-  af32x4 q[NU];
-  {
-    const int row = r0 + li;
-    const float *qp = qr + (size_t)row * p.q_dim + hq * HD + d0 + 4 * lk;
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      q[u] = af32x4{0.f, 0.f, 0.f, 0.f};
-      if (row < p.T) q[u] = aldg<af32x4>(qp + 16 * u);
-    }
-  }
-  // key range of each of this lane's four score rows
-  int rlo[4], rhi[4];
-  bool rok[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int row = r0 + 4 * lk + e;
-    rok[e] = row < p.T;
-    key_range(p, base + row, &rlo[e], &rhi[e]);
-  }
-
-  // K: a wave's lanes take consecutive dims of one key (whole rows, one
-  // float4 LDS store each).  V (VK, head dim 256 and below): lanes take the
-  // 16 keys of four dim quads, so the transposed stores of a wave fall in
-  // different banks; with a wave over the dims of one key, lane l's V^T rows
-  // start 4 l * VP floats apart and each 4-byte store hits a few banks many
-  // times over.  At head dim 512 (the key-fastest deal's V addresses would
-  // spill registers) thread t takes a 4 x 4 block instead: keys 4 (t / (HD /
-  // 4)) .. + 3 of dim quad t % (HD / 4), four coalesced float4 loads, a
-  // transpose in registers and four float4 stores to V^T.  The four-key
-  // groups of V^T row r sit in slot group ^ ((r >> 4) & 3): the 16 lanes of
-  // a store phase (rows 4 d4 + c, 80 bytes apart) then cover 16 distinct
-  // bank quads, and a read of dims 16u .. 16u + 15 uses one rotation.
-  constexpr bool VK = HD <= 256;
-  static_assert(VK || (NF == 4 && NT == 4 * (HD / 4)), "V blocks: 4 keys x 4 dims per thread");
-  // (NT is a multiple of 16: with VK, a thread's V key is the same for every f)
-  const int vkey = tid % 16;
-  af32x4 kreg[NF], vreg[NF];
-  auto tile_load = [&](int k0) {
-    const int vk = k0 + vkey;
-    const float *vrow = nullptr;
-    if (VK && vk <= khi)
-      vrow = vk < base ? p.vc + (size_t)cache_slot(p, vk) * p.kv_dim + h * HD
-                       : p.qkv + (size_t)(vk - base) * p.ld + p.q_dim + p.kv_dim + h * HD;
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      const int idx = tid + NT * f;
-      const int key = idx / (HD / 4), d4 = idx % (HD / 4);
-      const int k = k0 + key;
-      kreg[f] = af32x4{0.f, 0.f, 0.f, 0.f};
-      vreg[f] = af32x4{0.f, 0.f, 0.f, 0.f};
-      if (k <= khi) {
-        if (k < base) {
-          const size_t o = (size_t)cache_slot(p, k) * p.kv_dim + h * HD + 4 * d4;
-          kreg[f] = aldg<af32x4>(p.kc + o);
-        } else {
-          const int rr = k - base;
-          kreg[f] = aldg<af32x4>(kr + (size_t)rr * p.kv_dim + h * HD + 4 * d4);
-        }
-      }
-      if (VK && vrow) vreg[f] = aldg<af32x4>(vrow + 4 * (idx / 16));
-    }
-    if constexpr (!VK) {
-      // V block: keys k0 + 4 (tid / (HD / 4)) + r, dim quad tid % (HD / 4)
-      const int kq = tid / (HD / 4), d4 = tid % (HD / 4);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int k = k0 + 4 * kq + r;
-        vreg[r] = af32x4{0.f, 0.f, 0.f, 0.f};
-        if (k <= khi)
-          vreg[r] = k < base
-                        ? aldg<af32x4>(p.vc + (size_t)cache_slot(p, k) * p.kv_dim + h * HD +
-                                       4 * d4)
-                        : aldg<af32x4>(p.qkv + (size_t)(k - base) * p.ld + p.q_dim +
-                                       p.kv_dim + h * HD + 4 * d4);
-      }
-    }
-  };
-  auto tile_store = [&]() {
-#pragma unroll
-    for (int f = 0; f < NF; ++f) {
-      const int idx = tid + NT * f;
-      const int key = idx / (HD / 4), d4 = idx % (HD / 4);
-      *reinterpret_cast<af32x4 *>(Ks + key * KP + 4 * d4) = kreg[f];
-      if constexpr (VK) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) VT[(4 * (idx / 16) + c) * VP + vkey] = vreg[f][c];
-      }
-    }
-    if constexpr (!VK) {
-      const int kq = tid / (HD / 4), d4 = tid % (HD / 4);
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-        *reinterpret_cast<af32x4 *>(VT + (4 * d4 + c) * VP + 4 * (kq ^ ((d4 >> 2) & 3))) =
-            af32x4{vreg[0][c], vreg[1][c], vreg[2][c], vreg[3][c]};
-    }
-  };
-
-  af32x4 o[NU];
-#pragma unroll
-  for (int u = 0; u < NU; ++u) o[u] = af32x4{0.f, 0.f, 0.f, 0.f};
-  float m[4], l[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    m[e] = -INFINITY;
-    l[e] = 0.f;
-  }
-  float *Pw = Ps + wave * 16 * PP;
-
-  tile_load(kfirst);
-  tile_store();
-  __syncthreads();
-  for (int k0 = kfirst; k0 <= klast; k0 += 16) {
-    const bool more = k0 + 16 <= klast;
-    if (more) tile_load(k0 + 16);
-    // scores over this wave's dims: row 4lk + e, key k0 + li
-    af32x4 sc = af32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      const af32x4 kv = *reinterpret_cast<const af32x4 *>(Ks + li * KP + d0 + 16 * u + 4 * lk);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        sc = __builtin_amdgcn_mfma_f32_16x16x4f32(q[u][r], kv[r], sc, 0, 0, 0);
-    }
-    if constexpr (DS > 1) {
-      // sum the partial scores of the head's DS waves, in wave order (every
-      // wave of the head gets the same bits)
-      *reinterpret_cast<af32x4 *>(Sx + wave * 256 + lane * 4) = sc;
-      __syncthreads();
-      af32x4 t = *reinterpret_cast<const af32x4 *>(Sx + (g * DS) * 256 + lane * 4);
-#pragma unroll
-      for (int w2 = 1; w2 < DS; ++w2)
-        t += *reinterpret_cast<const af32x4 *>(Sx + (g * DS + w2) * 256 + lane * 4);
-      sc = t;
-    }
-    const int key = k0 + li;
-    float pe[4], corr[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const bool ok = rok[e] && key >= rlo[e] && key <= rhi[e];
-      const float x = ok ? sc[e] * p.scale : -INFINITY;
-      const float mn = fmaxf(m[e], row16_max(x));
-      const float msafe = mn == -INFINITY ? 0.f : mn;
-      pe[e] = ok ? expf(x - msafe) : 0.f;
-      corr[e] = m[e] == -INFINITY ? 0.f : expf(m[e] - msafe);
-      l[e] = l[e] * corr[e] + row16_sum(pe[e]);
-      m[e] = mn;
-    }
-#pragma unroll
-    for (int u = 0; u < NU; ++u)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o[u][e] *= corr[e];
-    // P: C layout [row][key] -> LDS -> A layout (this wave only; LDS accesses
-    // of one wave complete in order)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) Pw[(4 * lk + e) * PP + li] = pe[e];
-    __builtin_amdgcn_wave_barrier();
-    const af32x4 pa = *reinterpret_cast<const af32x4 *>(Pw + li * PP + 4 * lk);
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      // (head dim 512: the row's key groups are rotated by ((row >> 4) & 3))
-      const int vs = VK ? lk : lk ^ (((d0 >> 4) + u) & 3);
-      const af32x4 vt =
-          *reinterpret_cast<const af32x4 *>(VT + (d0 + 16 * u + li) * VP + 4 * vs);
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        o[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(pa[r], vt[r], o[u], 0, 0, 0);
-    }
-    __syncthreads();  // every wave is done with this tile (and with Sx)
-    if (more) tile_store();
-    __syncthreads();
-  }
-  if (nsplit == 1) {
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int row = r0 + 4 * lk + e;
-      if (row >= p.T) continue;
-      const float inv = 1.0f / l[e];
-      float *op = p.out + (size_t)row * p.q_dim + hq * HD + d0 + li;
-#pragma unroll
-      for (int u = 0; u < NU; ++u) op[16 * u] = o[u][e] * inv;
-    }
-  } else {
-    // partial of this split: o (unnormalized), max and sum per (row, head)
-    float *pb = keep(fs.part) + (size_t)j * 64 * (HD + 2);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int rl = 4 * lk + e;
-      float *po = pb + (rl * 4 + g) * HD + d0 + li;
-#pragma unroll
-      for (int u = 0; u < NU; ++u) po[16 * u] = o[u][e];
-      if (li == 0 && hf == 0) {
-        float *pm = pb + 64 * HD + (rl * 4 + g) * 2;
-        pm[0] = m[e];
-        pm[1] = l[e];
-      }
-    }
-  }
-}
-
-// Row tiles whose key tiles were split over several blocks: log-sum-exp merge
-// of the splits' partials.  One block per (row tile, kv head, query head of
-// the group); the splits' weights exp(m_s - M) / L of the 16 rows go through
-// LDS, then every thread sums float4 of o over the splits.
-constexpr int kFlashMaxSplits = 32;
-constexpr int kFlashMaxBlocks = 512;  // blocks of a split launch (two per CU)
-
-template <int HD>
-__global__ __launch_bounds__(256) void k_flash_merge(AttnArgs args, FlashSplit fs) {
-  __shared__ float wsh[kFlashMaxSplits][16];
-  const AttnP p = load_params(args);
-  const int maxs = keep(fs.maxs), stt = keep(fs.st_tiles), n_rt = keep(fs.n_rt);
-  const int rt = blockIdx.x, h = blockIdx.y >> 2, g = blockIdx.y & 3;
-  const int r0 = rt * 16;
-  const int base = aldg<int32_t>(p.pos);
-  const int rlast = min(r0 + 15, p.T - 1);
-  int klo, khi, dummy;
-  key_range(p, base + r0, &klo, &dummy);
-  key_range(p, base + rlast, &dummy, &khi);
-  const int kbeg = klo & ~15;
-  const int nsplit = min(maxs, ((khi - kbeg) / 16 + stt) / stt);
-  if (nsplit <= 1) return;
-  // record of split s: block (s * n_rt + n_rt - 1 - rt) * n_kv + h
-  const float *pb = keep(fs.part) + ((size_t)(n_rt - 1 - rt) * p.n_kv + h) * 64 * (HD + 2);
-  const size_t sstride = (size_t)n_rt * p.n_kv * 64 * (HD + 2);
-  const int tid = threadIdx.x;
-  if (tid < 16) {
-    const float *pm = pb + 64 * HD + (tid * 4 + g) * 2;
-    float M = -INFINITY;
-    for (int s2 = 0; s2 < nsplit; ++s2) M = fmaxf(M, pm[s2 * sstride]);
-    float L = 0.f;
-    for (int s2 = 0; s2 < nsplit; ++s2) {
-      const float ms2 = pm[s2 * sstride];
-      const float w = ms2 == -INFINITY ? 0.f : expf(ms2 - M);
-      wsh[s2][tid] = w;
-      L += pm[s2 * sstride + 1] * w;
-    }
-    // rows past T have no keys (L = 0); they are not stored
-    const float inv = L > 0.f ? 1.0f / L : 0.f;
-    for (int s2 = 0; s2 < nsplit; ++s2) wsh[s2][tid] *= inv;
-  }
-  __syncthreads();
-  constexpr int N4 = 16 * HD / 4;
-#pragma unroll 4
-  for (int e = tid; e < N4; e += 256) {
-    const int rl = e / (HD / 4), d = 4 * (e % (HD / 4));
-    const int row = r0 + rl;
-    const float *po = pb + (rl * 4 + g) * HD + d;
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int s2 = 0; s2 < nsplit; ++s2) {
-      const float w = wsh[s2][rl];
-      const float4 v = *reinterpret_cast<const float4 *>(po + s2 * sstride);
-      acc.x += w * v.x;
-      acc.y += w * v.y;
-      acc.z += w * v.z;
-      acc.w += w * v.w;
-    }
-    if (row < p.T) {
-      float *op = p.out + (size_t)row * p.q_dim + (h * 4 + g) * HD + d;
-      op[0] = acc.x;
-      op[1] = acc.y;
-      op[2] = acc.z;
-      op[3] = acc.w;
-    }
-  }
-}
-
-// Split plan of a prefill launch.  Row tile rt (rows at positions
-// plan_pos + 16 rt ...) attends to about min(plan_pos / 16 + rt + 2, bound)
-// key tiles, bound = cache_len / 16 + 2.  Splits of st tiles, st = the launch's
-// tiles / 256 CUs (at least 8), so that the blocks make about one round of
-// the chip; no split unless the longest row tile is a third longer than st.
-// At most kFlashMaxBlocks blocks and kFlashMaxSplits splits per row tile (the
-// last split of a row tile takes every tile left).
-static FlashSplit flash_split_plan(const AttnArgs &a) {
-  FlashSplit fs{};
-  fs.n_rt = (a.T + 15) / 16;
-  fs.maxs = 1;
-  fs.st_tiles = 1 << 30;
-  const long bound = (a.cache_len + 15) / 16 + 1;
-  const long p0 = std::max(0, a.plan_pos);
-  auto tiles = [&](long rt) { return std::min((p0 + rt * 16 + 15) / 16 + 1, bound); };
-  long tot = 0;
-  for (long rt = 0; rt < fs.n_rt; ++rt) tot += tiles(rt);
-  tot *= a.n_kv;
-  const long maxw = tiles(fs.n_rt - 1);
-  long st = std::max(8L, (tot + 255) / 256);
-  if (st * 4 > maxw * 3) return fs;
-  long maxs = std::min<long>((maxw + st - 1) / st, kFlashMaxSplits);
-  maxs = std::min<long>(maxs, kFlashMaxBlocks / ((long)fs.n_rt * a.n_kv));
-  if (maxs <= 1) return fs;
-  st = std::max(st, (maxw + maxs - 1) / maxs);
-  fs.maxs = (int)maxs;
-  fs.st_tiles = (int)st;
-  return fs;
-}
-
-size_t flash_part_floats(const AttnArgs &a) {
-  const FlashSplit fs = flash_split_plan(a);
-  if (fs.maxs <= 1) return 0;
-  return (size_t)a.n_kv * fs.n_rt * fs.maxs * 64 * (a.hd + 2);
-}
-
-size_t flash_part_floats_max(int hd) { return (size_t)kFlashMaxBlocks * 64 * (hd + 2); }
-
-// write_kv_sliding / write_kv_full (gemma4_e4b.mojo:211-249) for the rows
-__global__ __launch_bounds__(256) void k_cache_append(AttnArgs args, const float *kr) {
-  const AttnP p = load_params(args);
-  const int r = blockIdx.x;
-  // a circular cache keeps the last cache_len rows; older rows of the call
-  // would share their slots with later ones
-  if (p.circular && r < p.T - p.cache_len) return;
-  const int pt = aldg<int32_t>(p.pos) + r;
-  if (!p.circular && pt >= p.cache_len) return;  // linear cache full: dropped
-  const size_t cb = (size_t)cache_slot(p, pt) * p.kv_dim;
-  for (int c = threadIdx.x; c < p.kv_dim; c += 256) {
-    p.kc[cb + c] = aldg<float>(kr + (size_t)r * p.kv_dim + c);
-    p.vc[cb + c] = aldg<float>(p.qkv + (size_t)r * p.ld + p.q_dim + p.kv_dim + c);
-  }
-}
-
-bool prefill_flash_ok(const AttnArgs &a) {
-  return a.B == 1 && a.n_kv > 0 && a.n_heads == 4 * a.n_kv &&
-         (a.hd == 128 || a.hd == 256 || a.hd == 512);
-}
-
-int launch_attention_prefill(const AttnArgs &a, float *qr, float *kr, float *fpart,
-                             size_t fpart_floats, hipStream_t st) {
-  if (int rc = attn_check(a)) return rc;
-  MS_CHECK_ARG(prefill_flash_ok(a), "prefill attention: needs B = 1, 4 query heads per kv "
-                                    "head and head_dim 128, 256 or 512");
-  MS_CHECK_ARG(a.qkv && a.pos && a.out && a.kc && a.vc && qr && kr,
-               "prefill attention: missing buffers");
-  FlashSplit fs = flash_split_plan(a);
-  const size_t need = flash_part_floats(a);
-  if (need == 0 || !fpart || fpart_floats < need) fs.maxs = 1;  // no split
-  fs.part = fpart;
-  if (a.hd % 4 == 0 && (!a.apply_rope || a.rot % 8 == 0) && a.ld % 4 == 0 && a.q_dim % 4 == 0 &&
-      a.kv_dim % 4 == 0)
-    hipLaunchKernelGGL(k_rope_rows4, dim3(a.T), dim3(256), 0, st, a, qr, kr, a.hd);
-  else
-    hipLaunchKernelGGL(k_rope_rows, dim3(a.T), dim3(256), 0, st, a, qr, kr, a.hd);
-  const dim3 grid(fs.maxs * fs.n_rt * a.n_kv);
-#define MS_FLASH(HDV, DSV)                                                                \
-  hipLaunchKernelGGL((k_flash_prefill<HDV, DSV>), grid, dim3(256 * DSV),                   \
-                     (flash_lds_floats<HDV, DSV>() * 4), st, a, (const float *)qr,         \
-                     (const float *)kr, fs);                                               \
-  if (fs.maxs > 1)                                                                         \
-  hipLaunchKernelGGL(k_flash_merge<HDV>, dim3(fs.n_rt, a.n_kv * 4), dim3(256), 0, st, a, fs)
-  switch (a.hd) {
-    case 128: MS_FLASH(128, 1); break;
-    case 256: MS_FLASH(256, 2); break;
-    default: MS_FLASH(512, 2); break;
-  }
-#undef MS_FLASH
-  if (a.write_cache)
-    hipLaunchKernelGGL(k_cache_append, dim3(a.T), dim3(256), 0, st, a, (const float *)kr);
-  MS_HIP_TRY(hipGetLastError());
-  return MS_OK;
 }
 
 // ------------------------------------------------------------------------------

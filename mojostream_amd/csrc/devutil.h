@@ -28,6 +28,19 @@ __device__ inline T ldg_nt(const void *p) {
   return __builtin_nontemporal_load((const __attribute__((address_space(1))) T *)p);
 }
 
+// Global memory straight into LDS, 16 bytes per lane: lane l's bytes at base +
+// voff + soff land at dst + 16 l (dst wave-uniform).  As a buffer load: after
+// a global_load_lds the compiler treats every LDS read as out of order (a flat
+// access may return through the LDS) and waits for all of them at each use;
+// after a buffer load it counts them.
+typedef __attribute__((address_space(3))) void lds_void;
+__device__ inline __amdgpu_buffer_rsrc_t buffer_of(const void *p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, bytes, 0x00020000);
+}
+__device__ inline void load_lds16(__amdgpu_buffer_rsrc_t r, void *dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)dst, 16, voff, soff, 0, 0);
+}
+
 // A uniform value passed through an opaque register move: the compiler can no
 // longer turn selects between such values back into an indexed memory access
 // (which would put them in scratch memory or re-read the argument struct).

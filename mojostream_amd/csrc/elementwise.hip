@@ -200,12 +200,12 @@ extern "C" int ms_attention(const ms_layer_desc *L, const float *d_q, const floa
   a.pos_bound = base + T;
   if (int rc = attn_check(a)) return rc;
   const int G = a.n_heads / a.n_kv;
-  // many rows: the flash-attention prefill path (needs no chunk partials, but
-  // buffers for the rows' q and k)
-  const bool flash = T > kGemvMaxM && prefill_flash_ok(a);
-  const size_t qkv_f = (size_t)T * ld;
-  const size_t fsplit_f = flash ? flash_part_floats(a) : 0;
-  const size_t part_f = flash ? (size_t)T * (L->q_dim + L->kv_dim) + fsplit_f
+  // many rows: the flash-attention prefill path (its workspace in place of the
+  // chunk partials), 256-byte aligned after the rows
+  const bool flash = T > kGemvMaxM;
+  const size_t qkv_f = ((size_t)T * ld + 63) & ~(size_t)63;
+  const size_t flash_b = flash ? flash_bytes(a) : 0;
+  const size_t part_f = flash ? flash_b / 4
                               : attn_part_floats(1, a.n_kv, a.n_chunks, T, G, a.hd);
   const size_t need = (qkv_f + part_f) * 4 + 64 + (size_t)a.n_kv * 4;
   void *buf = nullptr;
@@ -227,10 +227,7 @@ extern "C" int ms_attention(const ms_layer_desc *L, const float *d_q, const floa
   a.pos = dpos;
   a.ctr = ctr;
   if (flash) {
-    float *fsplit = part + (size_t)T * (L->q_dim + L->kv_dim);
-    if (int rc = launch_attention_prefill(a, part, part + (size_t)T * L->q_dim,
-                                          fsplit_f ? fsplit : nullptr, fsplit_f, st))
-      return rc;
+    if (int rc = launch_attention_prefill(a, part, flash_b, st)) return rc;
   } else if (int rc = launch_attention(a, st)) {
     return rc;
   }

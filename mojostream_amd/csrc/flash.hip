@@ -1,0 +1,713 @@
+// Prefill attention: many rows of one sequence, causal GQA over the cached
+// keys and the rows' own (semantics in attention.hip).
+//
+// Operands in two fp16 parts.  A value y = x 2^-e (e per query, per 32-key
+// tile of K and of V, chosen so that the largest |y| lies in [2^13, 2^14)) is
+// held as hi = fp16(y) and lo = fp16(y - hi): 2^-24 relative, what an fp32
+// value carries, down to 2^-38 of the largest, below which the parts are
+// fixed point.  A product takes three v_mfma_f32_16x16x32_f16 (hi hi, hi lo,
+// lo hi; lo lo is below 2^-24 of the product) with fp32 sums.  On gfx950 one
+// fp32 16x16x4 MFMA takes as long as a fp16 16x16x32: three of the latter do
+// the work of eight of the former.
+//
+//  k_flash_prep   q and k after RoPE, v, and the cached keys the rows attend
+//                 to, split and written in MFMA fragment order (lane l of a
+//                 fragment owns the 16 bytes at 16 l), so that the flash
+//                 kernel copies whole tiles straight into LDS and reads every
+//                 fragment without bank conflicts.  Where the rows are the
+//                 sequence's first it also appends them to the cache; where
+//                 older keys were read k_cache_append does it afterwards (a
+//                 circular cache must not lose a key that a block still
+//                 reads).
+//  k_flash        one block per (64 queries of a kv head, key split).  The
+//                 queries of a kv head are numbered row * G + g: any number G
+//                 of query heads per kv head fills the MFMA tiles.  Wave w
+//                 owns queries 16w .. 16w + 15 with its q in registers and
+//                 computes S^T = K Q^T and O^T = V^T P^T: a lane then holds
+//                 one query's scores (keys 4 (l / 16) + e of each 16-key
+//                 half tile), which are the B operand of the second product
+//                 as they are (V^T is stored with the same key order), and the
+//                 softmax needs two lane swaps a tile.
+//  k_flash_merge  log-sum-exp merge of the key splits.
+//
+// Measured (E4B, 2048 rows; the fp32 MFMA kernel before it): sliding layer 45
+// + 13 (prep) against 135 + 17 us (RoPE and append launches), full layer 190 + 32
+// + 14 (merge) against 515 + 29; 14B class, 1000 rows, one layer: 62 + 16
+// against 5.0 ms of chunk launches.  Bound by the fragment reads and MFMAs of one
+// wave per SIMD; a short prompt by latency (77 rows: 10.5 + 7.4 against 22.5 +
+// 9.5 us).
+#include <algorithm>
+#include <cmath>
+
+#include "attention.h"
+#include "devutil.h"
+
+namespace ms {
+namespace {
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef float f4 __attribute__((ext_vector_type(4)));
+typedef int i2 __attribute__((ext_vector_type(2)));
+
+constexpr int kQB = 64;   // queries per block: 16 per wave
+constexpr int kKT = 32;   // keys per tile
+constexpr int kFlashMaxSplits = 32;
+constexpr int kFlashMaxBlocks = 512;  // blocks of a split launch
+constexpr int kPBits = 14;            // P is scaled by 2^14 before its split
+
+// First and last key that the row at position pos attends to.
+__host__ __device__ inline void key_span(int circular, int clamp, int cache_len, int pos, int *lo,
+                                         int *hi) {
+  *lo = circular && pos - cache_len + 1 > 0 ? pos - cache_len + 1 : 0;
+  *hi = !circular && clamp && pos > cache_len - 1 ? cache_len - 1 : pos;
+}
+
+// Key tiles [*t0, *t1] of query tile qt.
+__host__ __device__ inline void tile_span(const AttnArgs &a, const FlashBuf &f, int qt, int *t0,
+                                          int *t1) {
+  const int G = a.n_heads / a.n_kv, circ = a.cache_kind == MS_CACHE_CIRCULAR;
+  const int r0 = qt * kQB / G;
+  const int r1 = (qt * kQB + kQB - 1) / G < a.T - 1 ? (qt * kQB + kQB - 1) / G : a.T - 1;
+  int lo, hi, d;
+  key_span(circ, a.clamp, a.cache_len, f.base + r0, &lo, &d);
+  key_span(circ, a.clamp, a.cache_len, f.base + r1, &d, &hi);
+  *t0 = (lo - f.kbase) / kKT;
+  *t1 = (hi - f.kbase) / kKT;
+}
+
+__host__ __device__ inline int split_count(const FlashBuf &f, int nt) {
+  const int n = (nt + f.st_tiles - 1) / f.st_tiles;
+  return f.maxs == 1 ? 1 : (n < f.maxs ? n : f.maxs);
+}
+
+// |x| for the tile's scale; what is not finite does not set it
+__device__ inline float fin_abs(float x) {
+  const float v = fabsf(x);
+  return v < INFINITY ? v : 0.f;
+}
+// e with 2^-e * m in [2^13, 2^14); 0 for m = 0
+__device__ inline int scale_exp(float m) {
+  return m > 0.f ? __builtin_amdgcn_frexp_expf(m) - 14 : 0;
+}
+// hi and lo of x[0..7] 2^-e to dst and dst + 512 (halves)
+__device__ inline void store_split(const float *x, int e, _Float16 *dst) {
+  h8 hi, lo;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float y = ldexpf(x[j], -e);
+    hi[j] = (_Float16)y;
+    lo[j] = (_Float16)(y - (float)hi[j]);
+  }
+  *reinterpret_cast<h8 *>(dst) = hi;
+  *reinterpret_cast<h8 *>(dst + 512) = lo;
+}
+
+// Dims d0 .. d0 + 7 of a head row at src, after RoPE at position pos where
+// `rope` is set (pairs (i, i + half) over the first rot dims;
+// kernels.mojo:579-595).
+__device__ inline void load_rope8(const AttnArgs &a, const float *src, int d0, bool rope, int pos,
+                                  float *x) {
+  const int rot = a.apply_rope ? a.rot : 0, half = rot >> 1;
+  const bool r = rope && d0 < rot, low = d0 < half;
+  const f4 x0 = ldg<f4>(src + d0), x1 = ldg<f4>(src + d0 + 4);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) x[j] = j < 4 ? x0[j] : x1[j - 4];
+  if (rot == 0) return;
+  if (half % 8 == 0) {
+    // the eight dims lie in one half of the rotary dims or past them; what is
+    // not rotated loads its own values and the first table entries
+    const int pd = !r ? d0 : low ? d0 + half : d0 - half;
+    const size_t ti = !r ? 0 : (size_t)pos * half + (low ? d0 : d0 - half);
+    const f4 y0 = ldg<f4>(src + pd), y1 = ldg<f4>(src + pd + 4);
+    const f4 c0 = ldg<f4>(a.cos_t + ti), c1 = ldg<f4>(a.cos_t + ti + 4);
+    const f4 s0 = ldg<f4>(a.sin_t + ti), s1 = ldg<f4>(a.sin_t + ti + 4);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float y = j < 4 ? y0[j] : y1[j - 4], c = j < 4 ? c0[j] : c1[j - 4],
+                  s = j < 4 ? s0[j] : s1[j - 4];
+      const float t = low ? x[j] * c - y * s : y * s + x[j] * c;
+      x[j] = r ? t : x[j];
+    }
+    return;
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const int d = d0 + j, i = d < half ? d : d - half;
+    if (!rope || d >= rot) continue;
+    const float y = ldg<float>(src + (d < half ? d + half : i));
+    const float c = ldg<float>(a.cos_t + (size_t)pos * half + i);
+    const float s = ldg<float>(a.sin_t + (size_t)pos * half + i);
+    x[j] = d < half ? x[j] * c - y * s : y * s + x[j] * c;
+  }
+}
+
+// Blocks 0 .. nkt * n_kv - 1: K and V of one 32-key tile of a kv head; the
+// rest: 32 queries of a kv head each.  A thread takes one piece of eight dims
+// of a key or query (two at head dim 512) and one of eight keys of a dim of
+// V.  Latency and instruction fetch bound: one piece per thread keeps the code
+// at a tenth of four pieces', which ran 20 us on 77 rows, all of it cold code.
+template <int HD>
+constexpr int prep_threads() {
+  return HD < 256 ? 4 * HD : 1024;
+}
+template <int HD>
+__global__ __launch_bounds__(prep_threads<HD>()) void k_flash_prep(AttnArgs a, FlashBuf f) {
+  constexpr int NT = prep_threads<HD>();
+  constexpr int NP = 4 * HD / NT;  // pieces per thread
+  constexpr int PK = HD / 8;       // threads per key or query
+  constexpr int KS = HD / 32;      // 32-dim MFMA steps
+  __shared__ const float *krow[kKT], *vrow[kKT];
+  __shared__ int kslot[kKT], kind[kKT];  // kind: 0 no key, 1 cached, 2 one of the rows
+  __shared__ float red[2][16];
+  const int tid = threadIdx.x;
+  const int G = a.n_heads / a.n_kv;
+  int blk = blockIdx.x;
+  if (blk >= f.nkt * a.n_kv) {
+    // ---- queries
+    blk -= f.nkt * a.n_kv;
+    const int h = blk % a.n_kv;
+    const size_t nq = (size_t)f.n_qt * kQB;
+#pragma unroll 1
+    for (int i = 0; i < NP; ++i) {
+      const int q = blk / a.n_kv * 32 + (tid + NT * i) / PK, d8 = (tid + NT * i) % PK;
+      const int row = q / G, head = h * G + q - row * G;
+      const bool ok = row < a.T;
+      float x[8], m = 0.f;
+      load_rope8(a, a.qkv + (ok ? (size_t)row * a.ld + head * HD : 0), 8 * d8, ok, f.base + row,
+                 x);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        x[j] = ok ? x[j] : 0.f;
+        m = fmaxf(m, fin_abs(x[j]));
+      }
+#pragma unroll
+      for (int o = 1; o < PK; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+      const int e = scale_exp(m);
+      if (d8 == 0) f.qe[h * nq + q] = e;
+      store_split(x, e, f.q + (h * nq + (q & ~15)) * HD * 2 + (d8 >> 2) * 1024 +
+                            ((d8 & 3) * 16 + (q & 15)) * 8);
+    }
+    return;
+  }
+  // ---- keys and values.  A key's row lies in the cache before base (a full
+  // linear cache holds none past its end), then among the rows.
+  const int h = blk % a.n_kv, kt = blk / a.n_kv;
+  const size_t hc = (size_t)h * HD;
+  if (tid < kKT) {
+    const int k = f.kbase + kt * kKT + tid, r = k - f.base;
+    const bool circ = a.cache_kind == MS_CACHE_CIRCULAR;
+    const int slot = circ ? k % a.cache_len : k;
+    const int kd = r >= 0 ? (r < a.T ? 2 : 0) : (slot < a.cache_len ? 1 : 0);
+    const float *kr = a.qkv + (kd == 2 ? (size_t)r * a.ld + a.q_dim + hc : 0);
+    krow[tid] = kd == 1 ? a.kc + (size_t)slot * a.kv_dim + hc : kr;
+    vrow[tid] = kd == 1 ? a.vc + (size_t)slot * a.kv_dim + hc : kd == 2 ? kr + a.kv_dim : kr;
+    kind[tid] = kd;
+    // write_kv_sliding / write_kv_full (gemma4_e4b.mojo:211-249): a circular
+    // cache keeps the last cache_len rows, a full linear one drops the rest
+    kslot[tid] = kd == 2 && (circ ? r >= a.T - a.cache_len : slot < a.cache_len) ? slot : -1;
+  }
+  __syncthreads();
+  float x[NP][8], v[NP][8], mk = 0.f, mv = 0.f;
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    // V piece (dim, lk): keys 4 lk + 0..3 and 16 + 4 lk + 0..3
+    const int dim = (tid + NT * i) % HD, lk = (tid + NT * i) / HD;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[i][j] = ldg<float>(vrow[4 * lk + (j & 3) + 4 * (j & 4)] + dim);
+    const int kk = (tid + NT * i) / PK, d8 = (tid + NT * i) % PK;
+    load_rope8(a, krow[kk], 8 * d8, kind[kk] == 2, f.kbase + kt * kKT + kk, x[i]);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      x[i][j] = kind[kk] ? x[i][j] : 0.f;
+      v[i][j] = kind[4 * lk + (j & 3) + 4 * (j & 4)] ? v[i][j] : 0.f;
+      mk = fmaxf(mk, fin_abs(x[i][j]));
+      mv = fmaxf(mv, fin_abs(v[i][j]));
+    }
+  }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    mk = fmaxf(mk, __shfl_xor(mk, o, 64));
+    mv = fmaxf(mv, __shfl_xor(mv, o, 64));
+  }
+  if ((tid & 63) == 0) {
+    red[0][tid >> 6] = mk;
+    red[1][tid >> 6] = mv;
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int w = 0; w < NT / 64; ++w) {
+    mk = fmaxf(mk, red[0][w]);
+    mv = fmaxf(mv, red[1][w]);
+  }
+  const int ek = scale_exp(mk), ev = scale_exp(mv);
+  if (tid == 0) f.kve[h * f.nkt + kt] = int2{ek, ev};
+  const size_t tile = ((size_t)h * f.nkt + kt) * HD * 64;  // halves per tile and operand
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    const int dim = (tid + NT * i) % HD, lk = (tid + NT * i) / HD;
+    const int kk = (tid + NT * i) / PK, d8 = (tid + NT * i) % PK;
+    store_split(x[i], ek, f.k + tile + ((kk >> 4) * KS + (d8 >> 2)) * 1024 +
+                              ((d8 & 3) * 16 + (kk & 15)) * 8);
+    store_split(v[i], ev, f.v + tile + (dim >> 4) * 1024 + (lk * 16 + (dim & 15)) * 8);
+    if (!f.append) continue;
+    if (kslot[kk] >= 0) {
+      float *d = a.kc + (size_t)kslot[kk] * a.kv_dim + hc + 8 * d8;
+      *reinterpret_cast<f4 *>(d) = f4{x[i][0], x[i][1], x[i][2], x[i][3]};
+      *reinterpret_cast<f4 *>(d + 4) = f4{x[i][4], x[i][5], x[i][6], x[i][7]};
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int s = kslot[4 * lk + (j & 3) + 4 * (j & 4)];
+      if (s >= 0) a.vc[(size_t)s * a.kv_dim + hc + dim] = v[i][j];
+    }
+  }
+}
+
+// The rows' k (after RoPE) and v into the cache, once every key was read.
+__global__ __launch_bounds__(256) void k_cache_append(AttnArgs a, int base) {
+  const int r = blockIdx.x, pos = base + r;
+  const bool circ = a.cache_kind == MS_CACHE_CIRCULAR;
+  if (circ ? r < a.T - a.cache_len : pos >= a.cache_len) return;
+  const size_t cb = (size_t)(circ ? pos % a.cache_len : pos) * a.kv_dim;
+  const float *row = a.qkv + (size_t)r * a.ld + a.q_dim;
+  for (int c = 8 * threadIdx.x; c < a.kv_dim; c += 8 * 256) {
+    const int d = c % a.hd;
+    float o[8];
+    load_rope8(a, row + (c - d), d, true, pos, o);
+    *reinterpret_cast<f4 *>(a.kc + cb + c) = f4{o[0], o[1], o[2], o[3]};
+    *reinterpret_cast<f4 *>(a.kc + cb + c + 4) = f4{o[4], o[5], o[6], o[7]};
+    const float *v = row + a.kv_dim + c;
+    *reinterpret_cast<f4 *>(a.vc + cb + c) = ldg<f4>(v);
+    *reinterpret_cast<f4 *>(a.vc + cb + c + 4) = ldg<f4>(v + 4);
+  }
+}
+
+// Maximum over the lanes l, l ^ 16, l ^ 32, l ^ 48.
+__device__ inline float max_rows(float v) {
+  unsigned x = __float_as_uint(v);
+  auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  x = __float_as_uint(v);
+  r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// e^d for d <= 0: d log2(e) in two parts, so that the exponential of a large
+// |d| keeps fp32's accuracy.
+__device__ inline float exp_neg(float d) {
+  constexpr float kL = 0x1.715476p+0f, kLlo = 0x1.4ae0cp-26f, kLn2 = 0x1.62e43p-1f;
+  const float t = d * kL;
+  const float r = __builtin_fmaf(d, kLlo, __builtin_fmaf(d, kL, -t));
+  const float e = __builtin_amdgcn_exp2f(t);
+  // (d = -inf, a masked key, would make r a NaN; a NaN d stays one)
+  return d < -104.f ? 0.f : __builtin_fmaf(e, r * kLn2, e);
+}
+
+// Instruction order of a product phase of `reads` fragment reads feeding `mfmas`
+// MFMAs: eight reads ahead, then four per six MFMAs.  (Left to itself the
+// compiler reads each fragment right before its use and waits for it; with one
+// wave per SIMD nothing else covers that.)
+template <int READS, int MFMAS>
+__device__ inline void interleave() {
+  constexpr int kMfma = 0x008, kRead = 0x100;
+  __builtin_amdgcn_sched_group_barrier(kRead, 8, 0);
+#pragma unroll
+  for (int i = 8; i < READS; i += 4) {
+    __builtin_amdgcn_sched_group_barrier(kMfma, 6, 0);
+    __builtin_amdgcn_sched_group_barrier(kRead, 4, 0);
+  }
+  __builtin_amdgcn_sched_group_barrier(kMfma, MFMAS, 0);
+}
+
+// vmcnt(n), every other counter free
+template <int N>
+__device__ inline void wait_loads() {
+  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+  asm volatile("" ::: "memory");
+}
+__device__ inline void block_sync() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// Head dims up to 256 keep two K and two V tiles in LDS (DB): the scores of
+// tile t + 1 are computed beside the softmax and P V of tile t, one barrier a
+// tile.  At 512 one tile of each fits (128 KiB): V(t) arrives during the
+// scores, K(t + 1) during P V.
+template <int HD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD <= 256 ? 2 : 1, HD <= 256 ? 2 : 1)))
+void k_flash(AttnArgs a, FlashBuf f) {
+  constexpr int KS = HD / 32, DT = HD / 16;
+  constexpr int TB = HD * 128;         // bytes of a K or V tile
+  constexpr bool DB = HD <= 256;
+  constexpr int NLD = TB / 4096;       // 1 KiB loads per wave and tile
+  extern __shared__ __align__(16) uint8_t lds[];
+  uint8_t *kb = lds, *vb = lds + (DB ? 2 : 1) * TB;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int li = lane & 15, lk = lane >> 4;
+  const int G = a.n_heads / a.n_kv, circ = a.cache_kind == MS_CACHE_CIRCULAR;
+  // block (split, query tile, kv head), the tiles with the most keys first and
+  // the heads interleaved: heavy blocks start first, and the round-robin of
+  // blocks over the XCDs spreads every kind of block
+  const int j = blockIdx.x;
+  const int h = j % a.n_kv, qt = f.n_qt - 1 - (j / a.n_kv) % f.n_qt, sp = j / (a.n_kv * f.n_qt);
+  int t0, t1;
+  tile_span(a, f, qt, &t0, &t1);
+  const int nsplit = split_count(f, t1 - t0 + 1);
+  if (sp >= nsplit) return;
+  t0 += sp * f.st_tiles;
+  if (sp < nsplit - 1) t1 = t0 + f.st_tiles - 1;
+
+  const size_t nq = (size_t)f.n_qt * kQB;
+  const int qi = qt * kQB + wave * 16 + li, row = qi / G;
+  const bool valid = row < a.T;
+  int lo, hi;
+  key_span(circ, a.clamp, a.cache_len, f.base + row, &lo, &hi);
+  lo = valid ? lo - f.kbase : 1;
+  hi = valid ? hi - f.kbase : 0;
+  const int qe = ldg<int32_t>(f.qe + h * nq + qi);
+  h8 qh[KS], ql[KS];
+  {
+    const _Float16 *qp = f.q + (h * nq + qt * kQB + wave * 16) * HD * 2 + lane * 8;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      qh[s] = ldg<h8>(qp + s * 1024);
+      ql[s] = ldg<h8>(qp + s * 1024 + 512);
+    }
+  }
+  const __amdgpu_buffer_rsrc_t kg =
+      buffer_of(reinterpret_cast<const uint8_t *>(f.k) + (size_t)h * f.nkt * TB, f.nkt * TB);
+  const __amdgpu_buffer_rsrc_t vg =
+      buffer_of(reinterpret_cast<const uint8_t *>(f.v) + (size_t)h * f.nkt * TB, f.nkt * TB);
+  // tile t of a K or V array into LDS: this wave's NLD kilobytes
+  const int voff = wave * (NLD * 1024) + lane * 16;
+  auto issue = [&](const __amdgpu_buffer_rsrc_t src, int t, uint8_t *dst) {
+#pragma unroll
+    for (int i = 0; i < NLD; ++i)
+      load_lds16(src, dst + (wave * NLD + i) * 1024, voff, t * TB + i * 1024);
+  };
+  // S^T of the tile at kt: s[u], keys 16 u + 4 lk + e of query li
+  auto scores = [&](const uint8_t *kt, f4 *s) {
+    f4 x[2];  // the small products, added last
+#pragma unroll
+    for (int u = 0; u < 2; ++u) s[u] = x[u] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int d = 0; d < KS; ++d)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const h8 kh = *reinterpret_cast<const h8 *>(kt + (u * KS + d) * 2048 + lane * 16);
+        const h8 kl = *reinterpret_cast<const h8 *>(kt + (u * KS + d) * 2048 + 1024 + lane * 16);
+        s[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[d], s[u], 0, 0, 0);
+        x[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[d], x[u], 0, 0, 0);
+        x[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[d], x[u], 0, 0, 0);
+      }
+    interleave<4 * KS, 6 * KS>();
+#pragma unroll
+    for (int u = 0; u < 2; ++u) s[u] += x[u];
+  };
+  f4 o[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) o[d] = f4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  int E = -(1 << 20);  // o is in units of 2^(E - 14), E the largest V exponent so far
+  // exponents of tile t's K and V, loaded through a vector register: scalar
+  // loads in flight would turn every wait for an LDS read into one for all
+  auto exps = [&](int t) {
+    int z;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(z));
+    return ldg<i2>(f.kve + h * f.nkt + t + z);
+  };
+  // softmax of the scores of tile t against the running maximum: p in its two
+  // parts, o and l rescaled
+  auto softmax = [&](int t, const i2 kve, const f4 *s, h8 &ph, h8 &pl) {
+    const int ke = __builtin_amdgcn_readfirstlane(kve.x);
+    const int ve = __builtin_amdgcn_readfirstlane(kve.y);
+    const float sf = ldexpf(a.scale, qe + ke);
+    const int k0 = t * kKT;
+    float x[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = s[i >> 2][i & 3] * sf;
+    if (!__all(lo <= k0 && hi >= k0 + kKT - 1)) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int k = k0 + 16 * (i >> 2) + 4 * lk + (i & 3);
+        x[i] = k >= lo && k <= hi ? x[i] : -INFINITY;
+      }
+    }
+    float mt = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
+                     fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+    const float mn = fmaxf(m, max_rows(mt));
+    const float safe = mn == -INFINITY ? 0.f : mn;
+    if (ve > E || __any(mn != m)) {
+      const int En = ve > E ? ve : E;
+      const float c = m == -INFINITY ? 0.f : exp_neg(m - safe);
+      const float oc = ldexpf(c, E - En);
+      l *= c;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) o[d] *= oc;
+      m = mn;
+      E = En;
+    }
+    const int pe = kPBits + ve - E;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float p = exp_neg(x[i] - safe);
+      l += p;
+      const float y = ldexpf(p, pe);
+      ph[i] = (_Float16)y;
+      pl[i] = (_Float16)(y - (float)ph[i]);
+    }
+  };
+  // O^T += V^T P^T
+  auto pv = [&](const uint8_t *vt, const h8 ph, const h8 pl) {
+#pragma unroll
+    for (int d = 0; d < DT; d += 4) {
+      h8 vh[4], vl[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        vh[i] = *reinterpret_cast<const h8 *>(vt + (d + i) * 2048 + lane * 16);
+        vl[i] = *reinterpret_cast<const h8 *>(vt + (d + i) * 2048 + 1024 + lane * 16);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        o[d + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[i], ph, o[d + i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        o[d + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[i], pl, o[d + i], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        o[d + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[i], ph, o[d + i], 0, 0, 0);
+    }
+    interleave<2 * DT, 3 * DT>();
+  };
+
+  h8 ph, pl;
+  if constexpr (DB) {
+    i2 e = exps(t0);
+    issue(kg, t0, kb);
+    issue(vg, t0, vb);
+    wait_loads<0>();
+    block_sync();
+    if (t0 < t1) issue(kg, t0 + 1, kb + TB);
+    f4 s[2];
+    scores(kb, s);
+    for (int t = t0, b = 0; t <= t1; ++t, b ^= 1) {
+      // K(t + 1) and V(t) have landed, and no wave still reads the buffers
+      // that the next loads fill
+      wait_loads<0>();
+      block_sync();
+      const i2 en = exps(t < t1 ? t + 1 : t);
+      if (t + 2 <= t1) issue(kg, t + 2, kb + b * TB);
+      if (t + 1 <= t1) issue(vg, t + 1, vb + (b ^ 1) * TB);
+      f4 sn[2];
+      scores(kb + (b ^ 1) * TB, sn);  // past the last tile: not used
+      softmax(t, e, s, ph, pl);
+      pv(vb + b * TB, ph, pl);
+      s[0] = sn[0];
+      s[1] = sn[1];
+      e = en;
+    }
+  } else {
+    issue(kg, t0, kb);
+    for (int t = t0; t <= t1; ++t) {
+      const i2 e = exps(t);
+      issue(vg, t, vb);
+      wait_loads<NLD>();
+      block_sync();
+      f4 s[2];
+      scores(kb, s);
+      block_sync();
+      if (t < t1) issue(kg, t + 1, kb);
+      softmax(t, e, s, ph, pl);
+      if (t < t1) wait_loads<NLD>();
+      else wait_loads<0>();
+      block_sync();
+      pv(vb, ph, pl);
+      block_sync();
+    }
+  }
+  // the query's sum over its four lanes
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (nsplit == 1) {
+    if (!valid) return;
+    const float w = 1.0f / l;
+    float *op = a.out + (size_t)row * a.q_dim + (h * G + qi - row * G) * HD + 4 * lk;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      f4 v;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = ldexpf(o[d][e], E - kPBits) * w;
+      *reinterpret_cast<f4 *>(op + 16 * d) = v;
+    }
+    return;
+  }
+  // partial of this split: o, then (max, sum), per query
+  float *pb = f.part + (size_t)j * kQB * (HD + 2);
+  float *po = pb + (wave * 16 + li) * HD + 4 * lk;
+#pragma unroll
+  for (int d = 0; d < DT; ++d) {
+    f4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = ldexpf(o[d][e], E - kPBits);
+    *reinterpret_cast<f4 *>(po + 16 * d) = v;
+  }
+  if (lk == 0) {
+    float *pm = pb + kQB * HD + (wave * 16 + li) * 2;
+    pm[0] = m;
+    pm[1] = l;
+  }
+}
+
+// 16 queries of a query tile whose keys were split: weights e^(m_s - M) / L
+// through LDS, then float4 sums over the splits.
+template <int HD>
+__global__ __launch_bounds__(256) void k_flash_merge(AttnArgs a, FlashBuf f) {
+  __shared__ float wsh[kFlashMaxSplits][16];
+  const int qt = blockIdx.x >> 2, qs = (blockIdx.x & 3) * 16, h = blockIdx.y;
+  const int G = a.n_heads / a.n_kv;
+  int t0, t1;
+  tile_span(a, f, qt, &t0, &t1);
+  const int nsplit = split_count(f, t1 - t0 + 1);
+  if (nsplit <= 1) return;
+  const size_t rec = (size_t)kQB * (HD + 2);
+  const float *pb = f.part + ((size_t)(f.n_qt - 1 - qt) * a.n_kv + h) * rec;
+  const size_t ss = (size_t)f.n_qt * a.n_kv * rec;
+  const int tid = threadIdx.x;
+  if (tid < 16) {
+    const float *pm = pb + kQB * HD + (qs + tid) * 2;
+    float M = -INFINITY, L = 0.f;
+    for (int s = 0; s < nsplit; ++s) M = fmaxf(M, pm[s * ss]);
+    for (int s = 0; s < nsplit; ++s) {
+      const float w = pm[s * ss] == -INFINITY ? 0.f : expf(pm[s * ss] - M);
+      wsh[s][tid] = w;
+      L += pm[s * ss + 1] * w;
+    }
+    const float inv = L > 0.f ? 1.0f / L : 0.f;  // (queries past the last row)
+    for (int s = 0; s < nsplit; ++s) wsh[s][tid] *= inv;
+  }
+  __syncthreads();
+#pragma unroll 4
+  for (int e = tid; e < 16 * HD / 4; e += 256) {
+    const int q = e / (HD / 4), d = 4 * (e % (HD / 4));
+    const int qi = qt * kQB + qs + q, row = qi / G;
+    const float *po = pb + (qs + q) * HD + d;
+    f4 acc = f4{0.f, 0.f, 0.f, 0.f};
+    for (int s = 0; s < nsplit; ++s) acc += wsh[s][q] * ldg<f4>(po + s * ss);
+    if (row < a.T)
+      *reinterpret_cast<f4 *>(a.out + (size_t)row * a.q_dim + (h * G + qi - row * G) * HD + d) =
+          acc;
+  }
+}
+
+// Splits of st key tiles, st = the launch's tiles over the CUs' block slots
+// (at least 4), so that the blocks make about one round of the chip; no split
+// unless the longest query tile is a third longer than st.
+void split_plan(const AttnArgs &a, FlashBuf *f) {
+  f->maxs = 1;
+  f->st_tiles = 1 << 30;
+  long tot = 0, maxw = 0;
+  for (int qt = 0; qt < f->n_qt; ++qt) {
+    int t0, t1;
+    tile_span(a, *f, qt, &t0, &t1);
+    tot += t1 - t0 + 1;
+    maxw = std::max<long>(maxw, t1 - t0 + 1);
+  }
+  tot *= a.n_kv;
+  const long slots = a.hd <= 128 ? 512 : 256;
+  long st = std::max(4L, (tot + slots - 1) / slots);
+  if (st * 4 > maxw * 3) return;
+  long maxs = std::min<long>((maxw + st - 1) / st, kFlashMaxSplits);
+  maxs = std::min<long>(maxs, kFlashMaxBlocks / ((long)f->n_qt * a.n_kv));
+  if (maxs <= 1) return;
+  st = std::max(st, (maxw + maxs - 1) / maxs);
+  f->maxs = (int)maxs;
+  f->st_tiles = (int)st;
+}
+
+size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
+
+// Sizes and, with a buffer, pointers of a launch: T rows at position base.
+FlashBuf flash_view(const AttnArgs &a, int base, void *buf, size_t *bytes) {
+  FlashBuf f{};
+  const int G = a.n_heads / a.n_kv, circ = a.cache_kind == MS_CACHE_CIRCULAR;
+  int lo, hi, d;
+  key_span(circ, a.clamp, a.cache_len, base, &lo, &d);
+  key_span(circ, a.clamp, a.cache_len, base + a.T - 1, &d, &hi);
+  f.base = base;
+  f.kbase = lo & ~(kKT - 1);
+  f.nkt = (hi - f.kbase) / kKT + 1;
+  f.n_qt = (a.T * G + kQB - 1) / kQB;
+  split_plan(a, &f);
+  const size_t nq = (size_t)a.n_kv * f.n_qt * kQB, nk = (size_t)a.n_kv * f.nkt * kKT;
+  uint8_t *p = static_cast<uint8_t *>(buf);
+  size_t off = 0;
+  auto take = [&](size_t b) {
+    uint8_t *r = p + off;
+    off += up256(b);
+    return r;
+  };
+  f.q = reinterpret_cast<_Float16 *>(take(nq * a.hd * 4));
+  f.k = reinterpret_cast<_Float16 *>(take(nk * a.hd * 4));
+  f.v = reinterpret_cast<_Float16 *>(take(nk * a.hd * 4));
+  f.qe = reinterpret_cast<int32_t *>(take(nq * 4));
+  f.kve = reinterpret_cast<int2 *>(take((size_t)a.n_kv * f.nkt * 8));
+  f.part = reinterpret_cast<float *>(
+      take(f.maxs > 1 ? (size_t)f.maxs * f.n_qt * a.n_kv * kQB * (a.hd + 2) * 4 : 0));
+  *bytes = off;
+  return f;
+}
+
+template <int HD>
+void launch_hd(const AttnArgs &a, const FlashBuf &f, hipStream_t st) {
+  constexpr int lds = HD * 128 * (HD <= 256 ? 4 : 2);
+  hipLaunchKernelGGL(k_flash_prep<HD>, dim3((f.nkt + 2 * f.n_qt) * a.n_kv),
+                     dim3(prep_threads<HD>()), 0, st, a, f);
+  hipLaunchKernelGGL(k_flash<HD>, dim3(f.maxs * f.n_qt * a.n_kv), dim3(256), lds, st, a, f);
+  if (f.maxs > 1)
+    hipLaunchKernelGGL(k_flash_merge<HD>, dim3(f.n_qt * 4, a.n_kv), dim3(256), 0, st, a, f);
+}
+
+}  // namespace
+
+size_t flash_bytes(const AttnArgs &a) {
+  size_t b = 0;
+  (void)flash_view(a, a.plan_pos, nullptr, &b);
+  return b;
+}
+
+size_t flash_bytes_max(const AttnArgs &a) {
+  // the most keys: a full window or cache before the rows; the most blocks
+  const int G = a.n_heads / a.n_kv;
+  const size_t nq = (size_t)a.n_kv * ((a.T * G + kQB - 1) / kQB) * kQB;
+  const size_t keys = a.cache_kind == MS_CACHE_CIRCULAR ? (size_t)a.cache_len + a.T : a.cache_len;
+  const size_t nk = (size_t)a.n_kv * (keys + 2 * kKT);
+  return nq * a.hd * 4 + 2 * nk * a.hd * 4 + nq * 4 + nk + 8 * 256 +
+         (size_t)kFlashMaxBlocks * kQB * (a.hd + 2) * 4;
+}
+
+int launch_attention_prefill(const AttnArgs &a, void *buf, size_t buf_bytes, hipStream_t st) {
+  if (int rc = attn_check(a)) return rc;
+  MS_CHECK_ARG(a.B == 1 && a.plan_pos >= 0 && a.qkv && a.out && a.kc && a.vc && buf,
+               "prefill attention: one sequence, its position and its buffers");
+  MS_CHECK_ARG(a.ld % 4 == 0 && (!a.apply_rope || (a.cos_t && a.sin_t)),
+               "prefill attention: row stride or RoPE tables");
+  size_t need = 0;
+  FlashBuf f = flash_view(a, a.plan_pos, buf, &need);
+  MS_CHECK_ARG(buf_bytes >= need, "prefill attention: workspace too small");
+  f.append = a.write_cache && f.kbase == 0 && f.base == 0;
+  switch (a.hd) {
+    case 64: launch_hd<64>(a, f, st); break;
+    case 128: launch_hd<128>(a, f, st); break;
+    case 256: launch_hd<256>(a, f, st); break;
+    default: launch_hd<512>(a, f, st); break;
+  }
+  if (a.write_cache && !f.append)
+    hipLaunchKernelGGL(k_cache_append, dim3(a.T), dim3(256), 0, st, a, f.base);
+  MS_HIP_TRY(hipGetLastError());
+  return MS_OK;
+}
+
+}  // namespace ms

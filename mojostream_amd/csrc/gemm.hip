@@ -52,8 +52,6 @@ constexpr int kStages = 3;               // K steps resident in LDS
 constexpr int kGemmLds = kStages * kStage;  // 60 KiB
 constexpr int kLoads = 5;                // direct loads per thread per K step
 
-typedef __attribute__((address_space(3))) void lds_void;
-
 // LDS position of 16-byte chunk c of A limb row r: c ^ a_swz(r).  The rows
 // one A fragment read touches are r0 + 0..15; a 16-byte read goes in phases
 // of 8 lanes over 32 banks of 4 bytes (128 bytes per phase), so rows

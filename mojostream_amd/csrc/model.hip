@@ -115,13 +115,10 @@ struct ms_model {
   float *qkv = nullptr, *attn_part = nullptr;
   float *rope_cur = nullptr;  // one-row decode: RoPE factors at the position [2][256]
   unsigned *attn_ctr = nullptr;  // decode attention counters (attn_ctr_count), kept zero
-  // prefill: rows per chunk (0: no prefill workspace), attention rows per
-  // launch inside a chunk and their base positions on the device
+  // prefill: rows per chunk (0: no prefill workspace)
   int prefill_rows = 0;
-  int32_t *ppos = nullptr;
-  float *fq = nullptr, *fk = nullptr;  // prefill rows' q and k after RoPE
-  float *fpart = nullptr;              // flash attention's key-split partials
-  size_t fpart_floats = 0;
+  void *flash = nullptr;  // prefill attention's workspace
+  size_t flash_bytes = 0;
   int32_t *pos = nullptr, *tok = nullptr, *ids_hist = nullptr, *step = nullptr;
   int hist_cap = 1024;
   float *arg_val = nullptr;
@@ -228,14 +225,15 @@ static void prof_collect() {
 }
 
 // ---- per-layer enqueue --------------------------------------------------------
-// Prefill processes the prompt in chunks of up to kPrefillRows rows; their
-// projections run as GEMMs.  Flash attention takes a whole chunk per launch
-// (one block per 16 rows and kv head: long chunks fill the chip); the chunked
-// attention path runs kPrefillAttnRows rows per launch (its partial-result
-// buffer grows with the rows of a launch).  Workspace grows with the chunk:
-// about 170 KB per row at E4B shapes.
+// Prefill processes the prompt in chunks of up to kPrefillRows rows: their
+// projections run as GEMMs, flash attention takes a whole chunk per launch
+// (long chunks fill the chip).  Workspace grows with the chunk: about 170 KB
+// per row at E4B shapes.
 constexpr int kPrefillRows = 2048;
-constexpr int kPrefillAttnRows = 32;
+// Rows that the key-chunk count of a layer with a prefill allows for.  The
+// chunk kernels see at most 16 (kGemvMaxM) of them; the number bounds the
+// longest accepted cache (kAttnMaxChunks chunks: 8160 positions).
+constexpr int kChunkRows = 32;
 
 struct RunCfg {
   int B, T;                 // sequences, rows per sequence
@@ -244,8 +242,7 @@ struct RunCfg {
   float *hidden;            // optional [n_layers][B*T][D]
   int first_layer, n_layers;
   int seq0;                 // first sequence (caches / positions offset)
-  int plan_pos;             // first row's position as the host knows it (B = 1);
-                            // sizes the prefill attention's key split only
+  int plan_pos;             // first row's position as the host knows it (B = 1)
   int pos_bound;            // every row's position is below it (decode attention
                             // launches only the key chunks below it)
   float *tap_last;          // optional [n_layers][D]: each layer's last output row
@@ -461,11 +458,10 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
     } else if (attn_rows_ok(a)) {
       // two to four rows of one sequence: chunk partials per row, merged
       if (int rc2 = launch_attention_rows(a, st)) return rc2;
-    } else if (rc.B == 1 && rc.T > kGemvMaxM && m->fq && prefill_flash_ok(a)) {
-      // prefill rows: flash attention on fp32 MFMA
-      if (int rc2 = launch_attention_prefill(a, m->fq, m->fk, m->fpart, m->fpart_floats, st))
-        return rc2;
-    } else if (rc.T <= kPrefillAttnRows || rc.B != 1) {
+    } else if (rc.T > kGemvMaxM) {
+      // prefill rows of one sequence: flash attention
+      if (int rc2 = launch_attention_prefill(a, m->flash, m->flash_bytes, st)) return rc2;
+    } else {
       if (g_prof.on && rc.T == 1) {
         const int k = d.cache_kind == MS_CACHE_CIRCULAR ? 1 : 0;
         g_prof.last_attn[k] = a;
@@ -474,17 +470,6 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
         g_prof.attn_part[k] = false;
       }
       if (int rc2 = launch_attention(a, st)) return rc2;
-    } else {
-      // a prefill chunk: consecutive row groups, each attending to the cache
-      // the groups before it have written (base positions in m->ppos)
-      for (int s = 0, r0 = 0; r0 < rc.T; ++s, r0 += kPrefillAttnRows) {
-        AttnArgs b = a;
-        b.T = std::min(kPrefillAttnRows, rc.T - r0);
-        b.qkv = m->qkv + (size_t)r0 * ld;
-        b.out = m->aO + (size_t)r0 * d.q_dim;
-        b.pos = m->ppos + s;
-        if (int rc2 = launch_attention(b, st)) return rc2;
-      }
     }
   }
   // 3. x2 = x + attn . Wo (residual epilogue)
@@ -824,7 +809,7 @@ extern "C" int ms_model_create(const ms_model_desc *desc, const ms_layer_desc *l
   if (d.vocab > 0) m->prefill_rows = std::max(m->Mmax, std::min(kPrefillRows, d.max_pos));
   const int M = std::max(m->Mmax, m->prefill_rows);  // workspace rows
   const int attn_rows = m->prefill_rows > kGemvMaxM
-                            ? std::max(d.max_rows, kPrefillAttnRows) : d.max_rows;
+                            ? std::max(d.max_rows, kChunkRows) : d.max_rows;
   auto cleanup = [&](int rc) {
     ms_model_destroy(m);
     return rc;
@@ -894,19 +879,22 @@ extern "C" int ms_model_create(const ms_model_desc *desc, const ms_layer_desc *l
       (rc = dmalloc(m, (void **)&m->x2n, (size_t)M * D * 4)) ||
       (rc = dmalloc(m, (void **)&m->aO, (size_t)M * m->q_max * 4)) ||
       (rc = dmalloc(m, (void **)&m->aF, (size_t)M * F * 4)) ||
-      (rc = dmalloc(m, &m->quant, quant_rows_bytes(gemm_row_pad(M), m->quant_k))) ||
-      (rc = dmalloc(m, (void **)&m->ppos, (size_t)(M / kPrefillAttnRows + 2) * 4)))
-    return cleanup(rc);
-  if (m->prefill_rows > kGemvMaxM &&
-      ((rc = dmalloc(m, (void **)&m->fq, (size_t)m->prefill_rows * m->q_max * 4)) ||
-       (rc = dmalloc(m, (void **)&m->fk, (size_t)m->prefill_rows * m->kv_max * 4))))
+      (rc = dmalloc(m, &m->quant, quant_rows_bytes(gemm_row_pad(M), m->quant_k))))
     return cleanup(rc);
   if (m->prefill_rows > kGemvMaxM) {
-    // key-split partials of any flash launch
-    for (auto &Ly : m->L)
-      m->fpart_floats = std::max(m->fpart_floats, flash_part_floats_max(Ly.d.head_dim));
-    if (m->fpart_floats && (rc = dmalloc(m, (void **)&m->fpart, m->fpart_floats * 4)))
-      return cleanup(rc);
+    // the workspace of any prefill attention launch
+    for (auto &Ly : m->L) {
+      AttnArgs a{};
+      a.B = 1;
+      a.T = m->prefill_rows;
+      a.n_heads = Ly.d.n_heads;
+      a.n_kv = Ly.d.n_kv_heads;
+      a.hd = Ly.d.head_dim;
+      a.cache_kind = Ly.d.cache_kind;
+      a.cache_len = Ly.d.cache_len;
+      m->flash_bytes = std::max(m->flash_bytes, flash_bytes_max(a));
+    }
+    if ((rc = dmalloc(m, &m->flash, m->flash_bytes))) return cleanup(rc);
   }
   if ((rc = dmalloc(m, (void **)&m->qkv, (size_t)M * m->qkv_max * 4)) ||
       (rc = dmalloc(m, (void **)&m->attn_part, max_part * 4)) ||
@@ -1457,17 +1445,12 @@ extern "C" int ms_prefill(ms_model *m, int seq, const int32_t *h_tokens, int n_t
   }
   m->stats = ms_stream_stats{};
   int rcode = MS_OK;
-  std::vector<int32_t> sub;
   for (int c0 = 0; c0 < n_tokens && rcode == MS_OK; c0 += T) {
     const int t = std::min(T, n_tokens - c0);
     const int base = pos0 + c0;
     if ((rcode = check_positions(m, &base, 1, t, 0))) break;
     MS_HIP_TRY(hipMemcpyAsync(m->pos + seq, &base, 4, hipMemcpyHostToDevice, st));
-    // base position of each attention row group of the chunk
-    sub.clear();
-    for (int r0 = 0; r0 < t; r0 += kPrefillAttnRows) sub.push_back(base + r0);
-    MS_HIP_TRY(hipMemcpyAsync(m->ppos, sub.data(), sub.size() * 4, hipMemcpyHostToDevice, st));
-    MS_HIP_TRY(hipStreamSynchronize(st));  // `sub` is reused by the next chunk
+    MS_HIP_TRY(hipStreamSynchronize(st));  // `base` is a local
     if ((rcode = m->lm_f32 ? launch_embed_f32(m->lm_f32, D, m->d.vocab, dtok + c0, t, m->x_in, st)
                            : launch_embed(m->lm_w, D, m->d.vocab, m->lm_scale, dtok + c0, t,
                                           m->x_in, st)))

@@ -1,0 +1,121 @@
+"""Prefill attention (flash.hip) against a float64 statement of causal GQA:
+numbers of query heads per kv head that do not divide the 64-query tiles, every
+head size, rows and positions at the edges of the 32-key tiles, key splits, a
+window shorter than the rows, and the cache contents afterwards.
+
+Bound: q, k, v and p are held to 2^-24 of each value, products of the small
+parts are dropped (2^-24), sums are fp32.  A score's error is then below about
+3 * 2^-24 * sum |q k| scale, at |q|, |k| ~ 2 and hd <= 512 below 1e-5 absolute,
+and moves a probability by as much relatively; the outputs' relative RMSE is
+held to 2e-6 (an fp32 evaluation shows 1e-7 .. 5e-7)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# name, heads, kv heads, head dim, circular, cache_len, clamp, T, base
+CASES = [
+    ("g5-first-tile", 10, 2, 128, 0, 256, 0, 17, 0),
+    ("g5-tile-edge", 10, 2, 128, 0, 256, 0, 32, 0),
+    ("g5-one-past", 10, 2, 128, 0, 256, 0, 33, 31),
+    ("g5-long", 10, 2, 128, 0, 1100, 0, 1000, 64),
+    ("g1", 2, 2, 128, 0, 256, 0, 65, 3),
+    ("g3-circular", 6, 2, 256, 1, 96, 0, 130, 50),
+    ("g4-window", 8, 2, 256, 1, 512, 0, 700, 0),
+    ("g20", 20, 1, 128, 1, 64, 0, 45, 200),
+    ("hd64", 8, 2, 64, 0, 512, 0, 300, 7),
+    ("hd512-split", 8, 2, 512, 0, 1024, 1, 600, 0),
+    ("hd512-clamp", 8, 2, 512, 0, 128, 1, 40, 100),
+    ("hd512-past-cache", 8, 2, 512, 0, 128, 1, 20, 300),
+]
+
+
+def reference(q, k, v, G, lo, hi, key0):
+    """q [T][nh][hd], k and v [keys][nkv][hd] at positions key0 .."""
+    T, nh, hd = q.shape
+    out = np.empty_like(q)
+    for h in range(nh):
+        s = q[:, h] @ k[:, h // G].T / np.sqrt(hd)
+        p = key0 + np.arange(k.shape[0])
+        s[(p[None] < lo[:, None]) | (p[None] > hi[:, None])] = -np.inf
+        e = np.exp(s - s.max(1, keepdims=True))
+        out[:, h] = (e / e.sum(1, keepdims=True)) @ v[:, h // G]
+    return out
+
+
+@pytest.mark.parametrize("scale", [1.0, 1e-3, 300.0])
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_prefill_attention(gpu, case, scale):
+    ms = gpu
+    name, nh, nkv, hd, circ, clen, clamp, T, base = case
+    print(f"[flash] {name} T={T} base={base} scale={scale}", flush=True)
+    rng = np.random.default_rng(T * 7 + base)
+    qd, kvd, G = nh * hd, nkv * hd, nh // nkv
+    kc = (rng.standard_normal((clen, kvd)) * 2).astype(np.float32)
+    # values of very different size by position, and k and q whose product keeps
+    # its size: the tiles' exponents must not lose the small ones
+    vc = (rng.standard_normal((clen, kvd)) * scale).astype(np.float32)
+    q = (rng.standard_normal((T, qd)) * 2 / scale).astype(np.float32)
+    kc *= np.float32(scale)
+    kn = (rng.standard_normal((T, kvd)) * 2 * scale).astype(np.float32)
+    vn = (rng.standard_normal((T, kvd)) * scale * np.exp2(rng.integers(-3, 4, (T, 1)))).astype(
+        np.float32)
+    desc = ms.LayerDesc(q_dim=qd, kv_dim=kvd, head_dim=hd, n_heads=nh, n_kv_heads=nkv,
+                        rot_dim=hd, theta=1e4, cache_kind=circ, cache_len=clen,
+                        clamp_reads=clamp)
+    pos = base + np.arange(T)
+    lo = np.maximum(0, pos - clen + 1) if circ else np.zeros(T, int)
+    hi = np.minimum(pos, clen - 1) if clamp else pos
+    k0 = int(lo[0])
+    old = np.arange(k0, min(base, base if circ else clen))
+    slot = old % clen if circ else old
+    k = np.concatenate([kc[slot], kn]).astype(np.float64)
+    v = np.concatenate([vc[slot], vn]).astype(np.float64)
+    if not circ and base > clen:  # nothing of the rows is attended
+        k, v = k[:clen], v[:clen]
+    ref = reference(q.astype(np.float64).reshape(T, nh, hd), k.reshape(-1, nkv, hd),
+                    v.reshape(-1, nkv, hd), G, lo, hi, k0).reshape(T, qd)
+    dq, dk, dv = (ms.DeviceBuffer.from_array(a) for a in (q, kn, vn))
+    dkc, dvc = ms.DeviceBuffer.from_array(kc), ms.DeviceBuffer.from_array(vc)
+    dout = ms.DeviceBuffer(T * qd * 4)
+    ms.check(ms.lib().ms_attention(C.byref(desc), dq.ptr, dk.ptr, dv.ptr, dkc.ptr, dvc.ptr, T,
+                                   base, dout.ptr))
+    got = dout.download(np.float32, (T, qd)).astype(np.float64)
+    err = np.sqrt(np.mean((got - ref) ** 2) / np.mean(ref ** 2))
+    print(f"[flash]   rel rmse {err:.2e}", flush=True)
+    assert err < 2e-6
+    wk, wv = kc.copy(), vc.copy()
+    for r in range(T):
+        s = (base + r) % clen if circ else base + r
+        if s < clen:
+            wk[s], wv[s] = kn[r], vn[r]
+    assert np.array_equal(dkc.download(np.float32, kc.shape), wk)
+    assert np.array_equal(dvc.download(np.float32, vc.shape), wv)
+
+
+def test_prefill_attention_nan_row_stays_in_its_tile(gpu):
+    """A NaN in the last row's q reaches no other row; an all-zero k or v tile
+    gives the mean of v, or zero."""
+    ms = gpu
+    T, nh, nkv, hd = 70, 5, 1, 128
+    rng = np.random.default_rng(3)
+    q = rng.standard_normal((T, nh * hd)).astype(np.float32)
+    q[-1, 5] = np.nan
+    kn = np.zeros((T, hd), np.float32)
+    vn = rng.standard_normal((T, hd)).astype(np.float32)
+    vn[:64] = 0
+    desc = ms.LayerDesc(q_dim=nh * hd, kv_dim=hd, head_dim=hd, n_heads=nh, n_kv_heads=nkv,
+                        rot_dim=hd, theta=1e4, cache_kind=0, cache_len=128, clamp_reads=0)
+    dq, dk, dv = (ms.DeviceBuffer.from_array(a) for a in (q, kn, vn))
+    dkc, dvc = (ms.DeviceBuffer.from_array(np.zeros((128, hd), np.float32)) for _ in "kv")
+    dout = ms.DeviceBuffer(T * nh * hd * 4)
+    ms.check(ms.lib().ms_attention(C.byref(desc), dq.ptr, dk.ptr, dv.ptr, dkc.ptr, dvc.ptr, T, 0,
+                                   dout.ptr))
+    got = dout.download(np.float32, (T, nh, hd))
+    mean = np.cumsum(vn.astype(np.float64), 0) / np.arange(1, T + 1)[:, None]
+    assert np.array_equal(got[:64], np.zeros((64, nh, hd), np.float32))
+    assert np.abs(got[:-1] - mean[:-1, None]).max() < 1e-6
+    assert np.abs(got[-1, 1:] - mean[-1]).max() < 1e-6
+    assert np.isnan(got[-1, 0]).all()
