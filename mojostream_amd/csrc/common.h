@@ -34,6 +34,7 @@ struct Ctx {
   int n_cu = 0;
   void *scratch = nullptr;  // kernel-level entry points' temporary buffer
   size_t scratch_bytes = 0;
+  void *host_box = nullptr;  // 256 pinned bytes: results that a kernel hands to the host
 };
 Ctx &ctx();
 int require_init();

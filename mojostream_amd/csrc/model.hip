@@ -153,6 +153,7 @@ struct ms_model {
   int32_t *shist = nullptr;     // [max_seqs][kSampleMaxHistory]
   int32_t *shist_n = nullptr;   // [max_seqs]
   int32_t *samp_ids = nullptr;  // [max_seqs]
+  float *samp_work = nullptr;   // [max_seqs][kSampleWorkFloats]
   int32_t *samp_ctr = nullptr;  // LM head calls that drew since set_sampling / reset
   std::vector<int> h_hist_n;    // host mirror of shist_n (ids in each history)
   // taps (ms_model_set_taps): per-layer output rows and raw logits of every
@@ -576,6 +577,7 @@ static int enqueue_pick(ms_model *m, const RunCfg &rc, int M, ArgmaxFin f, hipSt
     f.draws = m->samp_ctr;
   }
   s.ids_out = m->samp_ids;
+  s.work = m->samp_work;
   if (int r2 = launch_sample(s, M, st)) return r2;
   f.ids_in = m->samp_ids;
   return launch_argmax_fin(f, st);
@@ -1118,6 +1120,8 @@ static int alloc_pick(ms_model *m) {
     if (int rc = dmalloc(m, (void **)&m->logits, S * m->d.vocab * 4)) return rc;
   if (!m->samp_ids)
     if (int rc = dmalloc(m, (void **)&m->samp_ids, S * 4)) return rc;
+  if (!m->samp_work)
+    if (int rc = dmalloc(m, (void **)&m->samp_work, S * kSampleWorkFloats * 4)) return rc;
   return MS_OK;
 }
 

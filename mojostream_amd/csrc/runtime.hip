@@ -75,6 +75,7 @@ extern "C" int ms_init(int device) {
   if (int rc = q4_noalloc_init(device)) return rc;
   MS_HIP_TRY(hipStreamCreateWithFlags(&g_ctx.stream, hipStreamNonBlocking));
   MS_HIP_TRY(hipStreamCreateWithFlags(&g_ctx.copy_stream, hipStreamNonBlocking));
+  MS_HIP_TRY(hipHostMalloc(&g_ctx.host_box, 256, hipHostMallocDefault));
   g_ctx.n_cu = prop.multiProcessorCount;
   g_ctx.device = device;
   return MS_OK;
@@ -84,6 +85,7 @@ extern "C" int ms_shutdown(void) {
   if (g_ctx.device < 0) return MS_OK;
   (void)hipStreamSynchronize(g_ctx.stream);
   if (g_ctx.scratch) (void)hipFree(g_ctx.scratch);
+  if (g_ctx.host_box) (void)hipHostFree(g_ctx.host_box);
   (void)hipStreamDestroy(g_ctx.stream);
   (void)hipStreamDestroy(g_ctx.copy_stream);
   g_ctx = Ctx{};

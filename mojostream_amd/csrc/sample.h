@@ -4,6 +4,8 @@
 
 namespace ms {
 
+constexpr int kSampleSlices = 1024;      // contiguous slices of a row
+constexpr size_t kSampleWorkFloats = 4 * kSampleSlices;  // workspace per row
 constexpr int kSampleMaxHistory = 8192;  // ids of a row's history the penalty sees
 
 struct SampleArgs {
@@ -13,7 +15,8 @@ struct SampleArgs {
   float penalty;          // > 1: repetition penalty over the history
   int32_t *hist;          // [rows][hist_ld] token history (prompt + generated)
   int hist_ld;
-  int32_t *hist_n;        // [rows] history length (device)
+  int32_t *hist_n;        // [rows] history length (device), or null:
+  int hist_len;           // the length
   int hist_cap;           // hist_append: capacity of a row's history
   int hist_append;        // append the sampled id to the history
   uint64_t seed;          // with step: base seed of draw_seed(seed, seq0 + row, *step);
@@ -21,6 +24,7 @@ struct SampleArgs {
   int seq0;               // sequence index of row 0 (with step)
   const int32_t *step;    // device draw counter or null
   int32_t *ids_out;       // [rows] or null
+  float *work;            // [rows][kSampleWorkFloats]
   int32_t *tok_state;     // [rows] or null: next input token
 };
 
