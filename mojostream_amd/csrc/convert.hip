@@ -10,11 +10,21 @@
 // some block is "tiny"; only then does the block structure matter, and only
 // then is it examined (k_tiny_blocks).
 //
-// k_absmax_part / k_absmax_fin   max |w| over the matrix and a non-finite flag.
-// k_q4_pack_t   64 (in) x 128 (out) tiles through LDS: coalesced reads along
-//               the HF rows, the tile transposed in LDS, 16 packed bytes per
-//               thread written along the (in, out) rows.  HBM-bound: the
-//               weight once (2 or 4 B per element) plus half a byte written.
+// k_absmax_part  max |w| and a non-finite flag, one pair per block.
+// k_q4_pack_t    every block reduces the pairs and forms the scale itself, so
+//                that no launch or host round trip stands between the passes; a
+//                weight that has to be refused or examined packs nothing and
+//                block 0 tells the host.  A thread quantizes 8 rows of 16 bytes
+//                in registers (eight loads in flight) and the codes are
+//                transposed in LDS as dwords of 8 codes; writes are 128 bytes of
+//                an (in, out) row.
+//
+// Bound by HBM: the weight twice (the second time partly from the last-level
+// cache) and half a byte per element written.  bf16 10240 x 2560: 11 + 17.5 us,
+// 39 us the call, against 11.7 + 3.4 + 23.6 us of kernels and a copy to the
+// host between them, 68 us the call.  The divisions of the former pack kernel
+// took most of its time; with the scale's reciprocal a quotient takes five
+// operations.
 #include "common.h"
 #include "devutil.h"
 
@@ -22,11 +32,14 @@
 
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 namespace ms {
 namespace {
 
-constexpr int kTk = 64, kTn = 128;
+constexpr int kTk = 64;        // in (k) values of a tile
+constexpr int kTn = 256;       // out (n) values of a tile of 16-bit weights; fp32: half
+constexpr int kRows = 8;       // n values per thread
 constexpr int kMaxParts = 1024;
 
 // dtype 0 fp32, 1 bf16, 2 fp16 (SafetensorsReader.load_f32, convert.py:100-110)
@@ -36,6 +49,11 @@ __device__ inline float load_w(const void *w, int dtype, size_t i) {
   if (dtype == 1) return __uint_as_float((uint32_t)h << 16);
   return __half2float(__ushort_as_half(h));
 }
+
+// 16-byte words at element alignment
+typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef u32x4 u32x4_a1 __attribute__((aligned(1)));
 
 // The 16-byte word v as 4 (fp32) or 8 (bf16, fp16) values.
 template <int DT>
@@ -67,15 +85,26 @@ __global__ __launch_bounds__(256) void k_absmax_part(const void *w, size_t n, si
   float m = 0.f;
   int bad = 0;
   const size_t g = (size_t)blockIdx.x * 256 + tid, stride = (size_t)gridDim.x * 256;
-  for (size_t v = g; v < nvec; v += stride) {
+  auto take = [&](const u32x4 d) {
     float x[PER];
-    unpack16<DT>(ldg_nt<u32x4>(static_cast<const uint8_t *>(w) + 16 * v), x);
+    unpack16<DT>(d, x);
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       bad |= !isfinite(x[i]);
       m = fmaxf(m, fabsf(x[i]));
     }
+  };
+  size_t v = g;
+  for (; v + 3 * stride < nvec; v += 4 * stride) {
+    // four loads in flight
+    u32x4 d[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      d[i] = ldg<u32x4>(static_cast<const uint8_t *>(w) + 16 * (v + i * stride));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) take(d[i]);
   }
+  for (; v < nvec; v += stride) take(ldg<u32x4>(static_cast<const uint8_t *>(w) + 16 * v));
   for (size_t i = nvec * PER + g; i < n; i += stride) {
     const float x = load_w(static_cast<const void *>(w), DT, i);
     bad |= !isfinite(x);
@@ -97,30 +126,6 @@ __global__ __launch_bounds__(256) void k_absmax_part(const void *w, size_t n, si
   }
 }
 
-__global__ __launch_bounds__(256) void k_absmax_fin(float *part, int nb) {
-  __shared__ float sm[256], sb[256];
-  const int tid = threadIdx.x;
-  float m = 0.f, b = 0.f;
-  for (int i = tid; i < nb; i += 256) {
-    m = fmaxf(m, part[2 * i]);
-    b = fmaxf(b, part[2 * i + 1]);
-  }
-  sm[tid] = m;
-  sb[tid] = b;
-  __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if (tid < s) {
-      sm[tid] = fmaxf(sm[tid], sm[tid + s]);
-      sb[tid] = fmaxf(sb[tid], sb[tid + s]);
-    }
-    __syncthreads();
-  }
-  if (tid == 0) {
-    part[0] = sm[0];
-    part[1] = sb[0];
-  }
-}
-
 // flag = 1 when a block of bs consecutive elements of the (in, out) matrix has
 // max |w| <= 1e-8 (convert.py:311-314).  Every writer stores the same value.
 __global__ __launch_bounds__(256) void k_tiny_blocks(const void *w, int dtype, int n_out, int n_in,
@@ -137,68 +142,117 @@ __global__ __launch_bounds__(256) void k_tiny_blocks(const void *w, int dtype, i
   if (!((double)m > 1e-8)) flag[0] = 1;
 }
 
-__device__ inline uint32_t q4_code(float x, float s) {
-  const int q = (int)rintf(__fdiv_rn(x, s));
-  return (uint32_t)(min(7, max(-8, q)) + 8);
+// clip(round_half_even(x / s), -8, 7) + 8, the quotient rounded to fp32 first as
+// the reference's is.  With r = 1 / s correctly rounded, q = x r is within two
+// units in the last place of the quotient; q + (x - q s) r is within one, and the
+// same step from there gives the correctly rounded quotient (Markstein, IBM J.
+// Res. Dev. 34, 1990; the residuals are exact, but for |x| far below s, whose
+// code is 8 whatever they are).  Adding 1.5 2^23 rounds half to even.
+__device__ inline uint32_t q4_code(float x, float s, float r) {
+  float q = x * r;
+  q = __builtin_fmaf(__builtin_fmaf(-q, s, x), r, q);
+  q = __builtin_fmaf(__builtin_fmaf(-q, s, x), r, q);
+  q = __builtin_amdgcn_fmed3f(q, -8.f, 7.f);
+  return __float_as_uint(q + (12582912.f + 8.f)) & 15u;
 }
 
-// VEC: rows of the weight read as 16-byte words (n_in a multiple of the word's
-// element count, base aligned); else element by element.
-template <int DT, bool VEC>
-__global__ __launch_bounds__(256) void k_q4_pack_t(const void *w, int n_out, int n_in, float s,
-                                                   uint8_t *out) {
+// s_given > 0: the scale; else it comes from the npart pairs of k_absmax_part,
+// and a non-finite weight or a scale below 1e-8 packs nothing.  Block 0 writes
+// (max |w|, flag) to host.  Rows
+// of odd lengths start anywhere: the 16-byte words read are element-aligned only,
+// and those written at any byte, which the memory unit takes.
+template <int DT>
+__global__ __launch_bounds__(256) void k_q4_pack_t(const void *w, int n_out, int n_in,
+                                                   const float *part, int npart, float s_given,
+                                                   float *host, uint8_t *out) {
   constexpr int PER = DT == 0 ? 4 : 8, ESZ = DT == 0 ? 4 : 2;
-  __shared__ float t[kTk][kTn + 1];
+  constexpr int CPR = kTk / PER;                   // threads along k
+  constexpr int TN = 256 / CPR * kRows;            // n values of the tile
+  constexpr int LD = TN / 8 + 1;                   // dwords per k row of the tile
+  typedef typename std::conditional<DT == 0, u32x4_a4, u32x4_a2>::type Word;
+  __shared__ uint32_t t[kTk * LD];
+  __shared__ float red[2][4];
   const int tid = threadIdx.x;
-  const int k0 = blockIdx.x * kTk, n0 = blockIdx.y * kTn;
-  if constexpr (VEC) {
-    constexpr int CPR = kTk / PER;  // words per tile row
+  const int k0 = blockIdx.x * kTk, n0 = blockIdx.y * TN;
+  const int c = (tid % CPR) * PER, r0 = tid / CPR * kRows;
+  u32x4 raw[kRows];
+  const bool whole = k0 + c + PER <= n_in;
+  auto load = [&]() {
 #pragma unroll
-    for (int e = tid; e < kTn * CPR; e += 256) {
-      const int r = e / CPR, c = (e % CPR) * PER;
-      const int n = n0 + r, k = k0 + c;
-      float x[PER];
-      if (n < n_out && k < n_in) {
-        const uint8_t *src = static_cast<const uint8_t *>(w) + ((size_t)n * n_in + k) * ESZ;
-        unpack16<DT>(ldg_nt<u32x4>(src), x);
-      } else {
-#pragma unroll
-        for (int i = 0; i < PER; ++i) x[i] = 0.f;
-      }
-#pragma unroll
-      for (int i = 0; i < PER; ++i) t[c + i][r] = x[i];
+    for (int i = 0; i < kRows; ++i) {
+      raw[i] = u32x4{0, 0, 0, 0};
+      if (whole && n0 + r0 + i < n_out)
+        raw[i] = *(const __attribute__((address_space(1))) Word *)(
+            static_cast<const uint8_t *>(w) + ((size_t)(n0 + r0 + i) * n_in + k0 + c) * ESZ);
     }
-  } else {
-    for (int e = tid; e < kTk * kTn; e += 256) {
-      const int r = e / kTk, c = e % kTk;  // r: out index in the tile, c: in index
-      const int n = n0 + r, k = k0 + c;
-      t[c][r] = (n < n_out && k < n_in) ? load_w(w, DT, (size_t)n * n_in + k) : 0.f;
+  };
+  load();
+  float s = s_given;
+  if (!(s > 0.f)) {
+    float m = 0.f, b = 0.f;
+    for (int i = tid; i < npart; i += 256) {
+      const float2 p = reinterpret_cast<const float2 *>(part)[i];
+      m = fmaxf(m, p.x);
+      b = fmaxf(b, p.y);
     }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      m = fmaxf(m, __shfl_xor(m, o, 64));
+      b = fmaxf(b, __shfl_xor(b, o, 64));
+    }
+    if ((tid & 63) == 0) {
+      red[0][tid >> 6] = m;
+      red[1][tid >> 6] = b;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      m = fmaxf(m, red[0][i]);
+      b = fmaxf(b, red[1][i]);
+    }
+    if (tid == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
+      host[0] = m;
+      host[1] = b;
+    }
+    const double gs = (double)m / 7.0;
+    if (b != 0.f || !(gs >= 1e-8)) return;
+    s = (float)gs;
   }
+  const float r = 1.0f / s;
+  uint32_t code[PER];
+#pragma unroll
+  for (int j = 0; j < PER; ++j) code[j] = 0;
+#pragma unroll
+  for (int i = 0; i < kRows; ++i) {
+    float x[PER];
+    unpack16<DT>(raw[i], x);
+    if (!whole) {
+      // the ragged end of a row, element by element
+      for (int j = 0; j < PER; ++j)
+        x[j] = n0 + r0 + i < n_out && k0 + c + j < n_in
+                   ? load_w(w, DT, (size_t)(n0 + r0 + i) * n_in + k0 + c + j)
+                   : 0.f;
+    }
+#pragma unroll
+    for (int j = 0; j < PER; ++j) code[j] |= q4_code(x[j], s, r) << (4 * i);
+  }
+#pragma unroll
+  for (int j = 0; j < PER; ++j) t[(c + j) * LD + r0 / 8] = code[j];
   __syncthreads();
-  const int c = tid >> 2, j0 = (tid & 3) * 16;  // 16 bytes = 32 out values of row k
-  const int k = k0 + c;
-  if (k >= n_in) return;
+  // 16-byte pieces of the rows
   const size_t half = (size_t)n_out / 2;
-  const size_t jb = (size_t)n0 / 2 + j0;
-  if (jb >= half) return;
-  uint32_t wd[4];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    uint32_t v = 0;
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int j = j0 + 4 * q + b;
-      const uint32_t lo = q4_code(t[c][2 * j], s), hi = q4_code(t[c][2 * j + 1], s);
-      v |= (lo | (hi << 4)) << (8 * b);
+  for (int e = tid; e < kTk * TN / 32; e += 256) {
+    const int kk = e / (TN / 32), p = e % (TN / 32);
+    const size_t jb = (size_t)n0 / 2 + 16 * p;
+    if (k0 + kk >= n_in || jb >= half) continue;
+    const uint32_t *q = t + kk * LD + 4 * p;
+    uint8_t *dst = out + (size_t)(k0 + kk) * half + jb;
+    if (jb + 16 <= half) {
+      *reinterpret_cast<u32x4_a1 *>(dst) = u32x4{q[0], q[1], q[2], q[3]};
+    } else {
+      for (int j = 0; j < 16 && jb + j < half; ++j) dst[j] = (uint8_t)(q[j / 4] >> (8 * (j % 4)));
     }
-    wd[q] = v;
-  }
-  uint8_t *dst = out + (size_t)k * half + jb;
-  if (jb + 16 <= half && (half & 15) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-    *reinterpret_cast<uint4 *>(dst) = uint4{wd[0], wd[1], wd[2], wd[3]};
-  } else {
-    for (int j = 0; j < 16 && jb + j < half; ++j) dst[j] = (uint8_t)(wd[j / 4] >> (8 * (j % 4)));
   }
 }
 
@@ -216,7 +270,7 @@ extern "C" int ms_q4_quantize(uint8_t *d_packed, float *h_scale, const void *d_w
   MS_CHECK_ARG(n_out >= 2 && n_out % 2 == 0 && n_in >= 1,
                "q4_quantize: out dimension must be even (two values per byte, convert.py:304)");
   MS_CHECK_ARG(block_size >= 1, "q4_quantize: block_size must be positive");
-  MS_CHECK_ARG((long)n_in <= 65535L * kTk && n_out / kTn < 65535, "q4_quantize: matrix too large");
+  MS_CHECK_ARG((long)n_in <= 65535L * kTk && n_out / 128 < 65535, "q4_quantize: matrix too large");
   hipStream_t st = ctx().stream;
   const size_t n = (size_t)n_out * n_in;
   void *buf = nullptr;
@@ -233,20 +287,34 @@ extern "C" int ms_q4_quantize(uint8_t *d_packed, float *h_scale, const void *d_w
     hipLaunchKernelGGL(k_absmax_part<1>, dim3(nb), dim3(256), 0, st, d_w, n, nvec, part);
   else
     hipLaunchKernelGGL(k_absmax_part<2>, dim3(nb), dim3(256), 0, st, d_w, n, nvec, part);
-  hipLaunchKernelGGL(k_absmax_fin, dim3(1), dim3(256), 0, st, part, nb);
+  float *box = static_cast<float *>(ctx().host_box);
+  auto pack = [&](float s) {
+    const int tn = dtype == 0 ? kTn / 2 : kTn;
+    const dim3 grid(cdiv((long)n_in, kTk), cdiv((long)n_out, tn));
+    if (dtype == 0)
+      hipLaunchKernelGGL(k_q4_pack_t<0>, grid, dim3(256), 0, st, d_w, n_out, n_in, part, nb, s,
+                         box, d_packed);
+    else if (dtype == 1)
+      hipLaunchKernelGGL(k_q4_pack_t<1>, grid, dim3(256), 0, st, d_w, n_out, n_in, part, nb, s,
+                         box, d_packed);
+    else
+      hipLaunchKernelGGL(k_q4_pack_t<2>, grid, dim3(256), 0, st, d_w, n_out, n_in, part, nb, s,
+                         box, d_packed);
+  };
+  pack(0.f);
   MS_HIP_TRY(hipGetLastError());
-  float fin[2];
-  MS_HIP_TRY(hipMemcpyAsync(fin, part, 8, hipMemcpyDeviceToHost, st));
   MS_HIP_TRY(hipStreamSynchronize(st));
-  MS_CHECK_ARG(fin[1] == 0.f, "q4_quantize: the weight holds NaN or infinity");
+  const float gmax = reinterpret_cast<volatile float *>(box)[0];
+  MS_CHECK_ARG(reinterpret_cast<volatile float *>(box)[1] == 0.f,
+               "q4_quantize: the weight holds NaN or infinity");
   // max over the block scales (convert.py:310-316), in double as Python does
-  const double g = fin[0];
-  double gs;
-  if (!(g > 1e-8)) {
-    gs = 1e-8;  // every block is tiny
-  } else {
-    gs = g / 7.0;
-    if (gs < 1e-8) {
+  const double g = gmax;
+  double gs = g / 7.0;
+  if (!(gs >= 1e-8)) {
+    // nothing is packed yet
+    if (!(g > 1e-8)) {
+      gs = 1e-8;  // every block is tiny
+    } else {
       const size_t nblocks = (n + block_size - 1) / block_size;
       int tiny = 0;
       MS_HIP_TRY(hipMemcpyAsync(flag, &tiny, 4, hipMemcpyHostToDevice, st));
@@ -257,22 +325,10 @@ extern "C" int ms_q4_quantize(uint8_t *d_packed, float *h_scale, const void *d_w
       MS_HIP_TRY(hipStreamSynchronize(st));
       if (tiny) gs = 1e-8;
     }
+    pack((float)gs);
+    MS_HIP_TRY(hipGetLastError());
+    MS_HIP_TRY(hipStreamSynchronize(st));
   }
-  const float s = (float)gs;
-  const dim3 grid(cdiv((long)n_in, kTk), cdiv((long)n_out, kTn));
-  const bool vec = aligned && n_in % per == 0;
-#define MS_PACK(DT, V) \
-  hipLaunchKernelGGL((k_q4_pack_t<DT, V>), grid, dim3(256), 0, st, d_w, n_out, n_in, s, d_packed)
-  if (dtype == 0) {
-    if (vec) MS_PACK(0, true); else MS_PACK(0, false);
-  } else if (dtype == 1) {
-    if (vec) MS_PACK(1, true); else MS_PACK(1, false);
-  } else {
-    if (vec) MS_PACK(2, true); else MS_PACK(2, false);
-  }
-#undef MS_PACK
-  MS_HIP_TRY(hipGetLastError());
-  MS_HIP_TRY(hipStreamSynchronize(st));
-  *h_scale = s;
+  *h_scale = (float)gs;
   return MS_OK;
 }

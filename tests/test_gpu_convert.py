@@ -63,6 +63,35 @@ def test_q4_quantize_vs_oracle(gpu, oracle, dt, shape):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("dt", ["F32", "BF16", "F16"])
+@pytest.mark.parametrize("shape", [(254, 63), (256, 64), (258, 65), (514, 129), (2, 4097),
+                                   (4098, 3), (126, 71), (130, 8)])
+def test_q4_quantize_tile_edges(gpu, oracle, dt, shape):
+    """Tiles of 64 in values by 256 (fp32: 128) out values, 16-byte words that
+    start at any element, and quotients at and next to ties: a maximum of seven
+    times a power of two puts the scale on the grid."""
+    ms = gpu
+    n_out, n_in = shape
+    say(f"q4_quantize edges {dt} n_out={n_out} n_in={n_in}")
+    rng = np.random.default_rng(n_out * 11 + n_in)
+    w = (rng.integers(-14, 15, (n_out, n_in)) / 2.0).astype(np.float32)
+    w += rng.integers(-2, 3, w.shape).astype(np.float32) * np.float32(2.0 ** -9)
+    w = np.clip(w, -7.0, 7.0) * np.float32(2.0 ** -6)
+    w[0, 0] = 7.0 * 2.0 ** -6
+    if dt == "BF16":
+        raw = to_bf16_bits(w)
+        w = from_bf16_bits(raw)
+    elif dt == "F16":
+        raw = w.astype(np.float16)
+        w = raw.astype(np.float32)
+    else:
+        raw = w
+    got, s = device_quantize(ms, raw, ms.Q4_DTYPES[dt], n_out, n_in)
+    want, s_want = oracle.q4_quantize(w)
+    assert s == s_want == np.float32(2.0 ** -6)
+    assert np.array_equal(got, want)
+
+
 def test_q4_quantize_grid_ties_and_tiny_blocks(gpu, oracle):
     ms = gpu
     say("q4_quantize: exact grid with ties, tiny-block rule, all zeros")
