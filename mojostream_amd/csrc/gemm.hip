@@ -15,24 +15,35 @@
 // with xsum = sum_k X_k from the quantization.  Each limb's dot product is
 // exact in int32; the three limbs of an output combine exactly
 // (limb_combine3), minus 8 * xsum, and are scaled by 2^-s and the tensor
-// scale.  launch_gemm picks the 32-row kernel (k_gemm) or the big tile
-// (k_gemm_big, described further down) per launch.
+// scale.
 //
-// k_gemm tiling: a block computes kBM = 32 activation rows (96 limb rows, 6 MFMA A
-// tiles) by 4 kWB panels (8 panels, 128 columns).  Wave (wa, wb) owns rows
-// 16wa..16wa+15 (one A tile per limb) and panels 4wb..4wb+3: 12 accumulators
-// and 24 MFMAs per 128-row step of K.  Both operands of a step (A 96 limb rows
-// x 128 bytes, B one 1 KiB super-tile of each panel) go from global memory
-// straight into LDS (global_load_lds: each wave instruction fills 1 KiB), in
-// a ring of three steps; loads run two steps ahead of the MFMAs, which a
-// step's MFMA time alone does not cover.  A limb rows are stored without
-// padding, chunk c of row r at chunk position c ^ a_swz(r), so the rows one
-// fragment read touches fall in different bank groups.
+// Tiling.  A block of four waves computes 32 RT activation rows (RT A tiles per
+// limb and wave) by 2 PW panels; wave (wr, wc) owns RT 16-row tiles of each limb
+// and PW panels: 3 RT PW accumulators and 6 RT PW MFMAs per 128-value step of K.
+// Both operands of a step (A 12 RT KiB, B one 1 KiB super-tile per panel) go from
+// global memory straight into LDS in a ring of two steps (three for the smallest
+// tile), two blocks per CU (2 x 80 KiB for RT = 2, PW = 8), so that one block's
+// barriers, start and epilogue overlap the other's MFMAs.  A limb rows are stored
+// without padding, chunk c of row r at chunk position c ^ a_swz(r), so the rows
+// one fragment read touches fall in different bank groups.
 //
-// EPI_SWIGLU: the first half of the wave columns computes gate panels, the
-// second half the up panels of the same columns; the gate values pass through
-// LDS and the up waves write up * gate * sigmoid(gate) (swiglu_inplace,
-// kernels.mojo:519-532).
+// What bounds it: at 2048 rows the operand traffic and the instructions between
+// the MFMAs.  A loop of the same MFMAs, LDS reads, unpacking and operand loads
+// runs at 3.14 POP/s on this card (3.76 without the operand loads, 4.33 MFMAs
+// alone; the nominal 5.0 is not reached).  Measured (E4B, 2048 rows; the one-row-
+// tile kernel with compiler scheduling before it): Gate|Up 240 us, 2.68 POP/s
+// (266 us); Down 135 (139), sliding Q|K|V 43.8 (49), full Q|K|V 79 (87); 14B
+// class, 1000 rows: Gate|Up 335 (404), Down 181 (193).
+//
+// Short prompts leave most CUs idle where the matrix is narrow (O, Down: 20
+// column tiles): gemm_ksplit splits K over blocks, whose exact int64 sums
+// k_gemm_kcombine adds: the same integer, so the result does not depend on the
+// split.  Down at 77 rows: 43 -> 20 us with its combine; E4B prefill of 77 tokens
+// 5.4 -> 4.25 ms.
+//
+// EPI_SWIGLU: wave column wc holds the gate panels of PW / 2 column groups (slots
+// j < PW / 2) and the up panels of the same groups, so each output's gate and up
+// values meet in one lane (swiglu_inplace, kernels.mojo:519-532).
 #include <algorithm>
 
 #include "devutil.h"
@@ -41,16 +52,7 @@
 namespace ms {
 namespace {
 
-constexpr int kBM = 32;                  // activation rows per block
-constexpr int kWB = 2;                   // wave columns: 4 panels each
-constexpr int kNT = 128 * kWB;           // threads (2 wave rows x kWB wave columns)
-constexpr int kLimbs = 3;                // limb planes of the A operand
-constexpr int kAstage = kLimbs * kBM * 128;  // one K step of A: 96 limb rows x 128 bytes
-constexpr int kBstage = 8 * 1024;        // one super-tile of each of the 8 panels
-constexpr int kStage = kAstage + kBstage;
-constexpr int kStages = 3;               // K steps resident in LDS
-constexpr int kGemmLds = kStages * kStage;  // 60 KiB
-constexpr int kLoads = 5;                // direct loads per thread per K step
+constexpr int kLimbs = 3;     // limb planes of the A operand
 
 // LDS position of 16-byte chunk c of A limb row r: c ^ a_swz(r).  The rows
 // one A fragment read touches are r0 + 0..15; a 16-byte read goes in phases
@@ -75,7 +77,6 @@ __device__ inline void seg_panel(int pi, int K, const uint8_t *w0, const uint8_t
   *sc = si == 0 ? s0 : (si == 1 ? s1 : s2);
   *col = (si == 0 ? c0 : (si == 1 ? c1 : c2)) + loc * 16;
 }
-typedef const __attribute__((address_space(1))) void gbl_void;
 
 // Exact limb combine of one output, minus the zero-point term z: each limb's
 // int32 dot product is below 2^25 in magnitude (K <= 16384, |limb| <= 128,
@@ -85,298 +86,27 @@ __device__ inline double limb_combine3(int d0, int d1, int d2, double z) {
   return __builtin_fma((double)d2, 65536.0, __builtin_fma((double)d1, 256.0, (double)d0)) - z;
 }
 
-template <int EPI>
-__global__ __launch_bounds__(kNT) void k_gemm(GemmArgs g) {
-  extern __shared__ __align__(16) uint8_t lds[];
-  const int M = launder(g.M), K = launder(g.K);
-  const int8_t *limbs = launder(g.a.limbs);
-  const int32_t *shift = launder(g.a.shift);
-  const int64_t *xsum = launder(g.a.xsum);
-  const uint8_t *sw0 = launder(g.seg[0].w), *sw1 = launder(g.seg[1].w),
-                *sw2 = launder(g.seg[2].w);
-  const float ss0 = launder(g.seg[0].scale), ss1 = launder(g.seg[1].scale),
-              ss2 = launder(g.seg[2].scale);
-  const int nseg = launder(g.nseg);
-  const int sn0 = launder(g.seg[0].n_cols) >> 4;
-  const int sn1 = nseg > 1 ? launder(g.seg[1].n_cols) >> 4 : 0;
-  const int sn2 = nseg > 2 ? launder(g.seg[2].n_cols) >> 4 : 0;
-  const int sc0 = launder(g.seg[0].out_col0), sc1 = launder(g.seg[1].out_col0),
-            sc2 = launder(g.seg[2].out_col0);
-  float *out = launder(g.out);
-  const int ldo = launder(g.ldo);
-  const float *resid = EPI == EPI_RESID ? launder(g.resid) : nullptr;
-  float *out2 = EPI == EPI_RESID ? launder(g.out2) : nullptr;
-  float *sw_out = EPI == EPI_SWIGLU ? launder(g.sw_out) : nullptr;
-  const int ldo_sw = EPI == EPI_SWIGLU ? launder(g.ldo_sw) : 0;
+constexpr int kGRows = 32;    // activation rows per row tile of a wave pair
+constexpr int kGNT = 256;     // threads per block
+constexpr int gemm_stage(int rt, int pw) { return kLimbs * kGRows * rt * 128 + 2048 * pw; }
+// K steps in LDS: the smallest tile runs where few blocks share a CU and keeps
+// one step more in flight
+constexpr int gemm_stages(int rt, int pw) { return rt * pw <= 4 ? 3 : 2; }
+constexpr int gemm_lds(int rt, int pw) { return gemm_stages(rt, pw) * gemm_stage(rt, pw); }
+// Epilogue of a K part (GemmArgs::ksplit): its exact sums, for k_gemm_kcombine
+constexpr int EPI_PART = 100;
 
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int lane = tid & 63;
-  const int wa = wave & 1, wb = wave >> 1;
-  // EPI_SWIGLU: wave columns [0, kWB/2) hold gate panels, the rest the up
-  // panels of the same columns
-  const int half = wb / (kWB / 2), sub = wb % (kWB / 2);
-  const int r0 = blockIdx.y * kBM;
-  const int KG = K >> 7;
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
-  // panel slot sl of the block's 8 -> weights, scale, first column, valid
-  // (block-uniform selects).  EPI_SWIGLU: slots 0-3 gate, 4-7 up panels of
-  // the same 4 column groups.
-  auto slot = [&](int sl, const uint8_t **w, float *sc, int *cl, bool *ok) {
-    if constexpr (EPI == EPI_SWIGLU) {
-      const int hf = sl >> 2, cp = blockIdx.x * 4 + (sl & 3);
-      *ok = cp < sn0;
-      *w = (hf == 0 ? sw0 : sw1) + (size_t)(*ok ? cp : 0) * K * 8;
-      *sc = hf == 0 ? ss0 : ss1;
-      *cl = cp * 16;
-    } else {
-      seg_panel(blockIdx.x * 8 + sl, K, sw0, sw1, sw2, ss0, ss1, ss2, sn0, sn1, sn2, sc0, sc1,
-                sc2, w, sc, cl, ok);
-    }
-  };
-  // the panels this wave computes: slots 4 wb .. 4 wb + 3
-  float wsc[4];
-  int col[4];
-  bool pv[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const uint8_t *w;
-    slot(4 * wb + j, &w, &wsc[j], &col[j], &pv[j]);
-  }
-  // the panels this wave loads: slots 2 wave, 2 wave + 1 (an invalid slot
-  // loads a valid panel, so every wave issues the same number of loads)
-  const uint8_t *lw[2];
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    float sc;
-    int cl;
-    bool ok;
-    slot(2 * wave + j, &lw[j], &sc, &cl, &ok);
-  }
-
-  // A: a stage holds limb rows 32l + m (limb l of block row m); this wave
-  // fills LDS blocks 3 wave + i (stage rows 8q .. 8q + 7); lane l writes row
-  // 8q + l / 8 at chunk position l % 8, which holds chunk (l % 8) ^
-  // a_swz(row) of the row, so the rows one fragment read touches fall in
-  // different bank groups
-  const int pr = launder(g.a.plane_rows);
-  const int8_t *asrc[kLimbs];
-#pragma unroll
-  for (int i = 0; i < kLimbs; ++i) {
-    const int row = 8 * (kLimbs * wave + i) + (lane >> 3);
-    const int c = (lane & 7) ^ a_swz(row);
-    asrc[i] = limbs + ((size_t)(row >> 5) * pr + r0 + (row & 31)) * K + c * 16;
-  }
-  // K step G into stage stg: global memory straight into LDS
-  auto issue = [&](int G, int stg) {
-    uint8_t *sa = lds + stg * kStage;
-#pragma unroll
-    for (int i = 0; i < kLimbs; ++i)
-      __builtin_amdgcn_global_load_lds((gbl_void *)(asrc[i] + (size_t)G * 128),
-                                       (lds_void *)(sa + (kLimbs * wave + i) * 1024), 16, 0, 0);
-#pragma unroll
-    for (int j = 0; j < 2; ++j)
-      __builtin_amdgcn_global_load_lds((gbl_void *)(lw[j] + (size_t)G * 1024 + lane * 16),
-                                       (lds_void *)(sa + kAstage + (2 * wave + j) * 1024), 16,
-                                       0, 0);
-  };
-
-  // acc[l][j]: limb l of block rows 16 wa .. 16 wa + 15, panel 4 wb + j
-  v4i acc[kLimbs][4];
-#pragma unroll
-  for (int a = 0; a < kLimbs; ++a)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[a][j] = v4i{0, 0, 0, 0};
-
-  const int li = lane & 15, lg = lane >> 4;
-  const int swz = a_swz(li);  // a_swz(row) for every row this lane reads
-  auto compute = [&](int stg) {
-    const uint8_t *sa = lds + stg * kStage;
-    u32x4 braw[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      braw[j] = *reinterpret_cast<const u32x4 *>(sa + kAstage + (4 * wb + j) * 1024 + lane * 16);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      v4i bf[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t d0 = braw[j][2 * h], d1 = braw[j][2 * h + 1];
-        bf[j] = v4i{(int)(d0 & 0x0F0F0F0Fu), (int)((d0 >> 4) & 0x0F0F0F0Fu),
-                    (int)(d1 & 0x0F0F0F0Fu), (int)((d1 >> 4) & 0x0F0F0F0Fu)};
-      }
-      const int pos = (2 * lg + h) ^ swz;
-#pragma unroll
-      for (int a = 0; a < kLimbs; ++a) {
-        const v4i af = *reinterpret_cast<const v4i *>(sa + (32 * a + 16 * wa + li) * 128 +
-                                                      pos * 16);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[a][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, bf[j], acc[a][j], 0, 0, 0);
-      }
-    }
-  };
-
-  // the epilogue's row shifts and sums, loaded before the K loop: lane
-  // j + 16 rr holds rows 16 wa + 4 rr + i of column j (rows past M: shift
-  // 0, sum 0; their outputs are not stored)
-  int32_t rsh[4];
-  double rz[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = r0 + 16 * wa + 4 * (lane >> 4) + i;
-    rsh[i] = row < M ? ldg<int32_t>(shift + row) : 0;
-    rz[i] = row < M ? (double)(8 * ldg<long long>(xsum + row)) : 0.0;
-  }
-
-  // K steps of this block: all of them, or part blockIdx.z of ksplit
-  const int ks = launder(g.ksplit) > 1 ? launder(g.ksplit) : 1;
-  const int G0 = (int)((long)KG * blockIdx.z / ks), NG = (int)((long)KG * (blockIdx.z + 1) / ks) - G0;
-
-  // Ring of kStages K steps: step i + 2 is issued into the stage step i - 1
-  // used, once every wave has passed the barrier after computing it.  The
-  // barrier is a bare s_barrier: this wave's own loads of step i are waited
-  // for explicitly, and those of step i + 1 stay in flight (a __syncthreads
-  // would wait for them too).
-  issue(G0, 0);
-  if (NG > 1) issue(G0 + 1, 1);
-  for (int i = 0; i < NG; ++i) {
-    if (i + 1 < NG)
-      __builtin_amdgcn_s_waitcnt(0x0F70 | kLoads);  // vmcnt(6)
-    else
-      __builtin_amdgcn_s_waitcnt(0x0F70);           // vmcnt(0)
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (i + 2 < NG) issue(G0 + i + 2, (i + 2) % kStages);
-    compute(i % kStages);
-  }
-
-  // ---- epilogue: lane (column jc, row rr of each A tile)
-  const int jc = lane & 15, rr = lane >> 4;
-  if constexpr (EPI == EPI_STORE || EPI == EPI_ACCUMULATE) {
-    if (ks > 1) {
-      // this part's exact sums d0 + 2^8 d1 + 2^16 d2 (k_gemm_kcombine)
-      int64_t *kp = launder(g.kpart) + (size_t)blockIdx.z * M * ldo;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = r0 + 16 * wa + 4 * rr + i;
-        if (row >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (!pv[j]) continue;
-          kp[(size_t)row * ldo + col[j] + jc] = (int64_t)acc[0][j][i] +
-                                                ((int64_t)acc[1][j][i] << 8) +
-                                                ((int64_t)acc[2][j][i] << 16);
-        }
-      }
-      return;
-    }
-  }
-  float v[4][4];  // [row i][panel j]
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float sc = ldexpf(1.0f, -rsh[i]);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      v[i][j] = (float)(limb_combine3(acc[0][j][i], acc[1][j][i], acc[2][j][i], rz[i]) *
-                        (double)sc * (double)wsc[j]);
-  }
-  if constexpr (EPI == EPI_SWIGLU) {
-    // gate values of wave (wa, sub) -> LDS -> up wave (wa, sub)
-    __syncthreads();  // every wave is done reading the operand stages
-    float *xg = reinterpret_cast<float *>(lds);
-    const int xo = (wa * (kWB / 2) + sub) * 16;
-    if (half == 0) {
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) xg[(xo + a * 4 + j) * 64 + lane] = v[a][j];
-    }
-    __syncthreads();
-    if (half == 1) {
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const int row = r0 + 16 * wa + 4 * rr + a;
-        if (row >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (!pv[j]) continue;
-          const float gt = xg[(xo + a * 4 + j) * 64 + lane], up = v[a][j];
-          sw_out[(size_t)row * ldo_sw + col[j] + jc] = up * gt * (1.0f / (1.0f + expf(-gt)));
-        }
-      }
-    }
-  } else {
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int row = r0 + 16 * wa + 4 * rr + a;
-      if (row >= M) continue;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (!pv[j]) continue;
-        const size_t oi = (size_t)row * ldo + col[j] + jc;
-        if constexpr (EPI == EPI_STORE) {
-          out[oi] = v[a][j];
-        } else if constexpr (EPI == EPI_ACCUMULATE) {
-          out[oi] += v[a][j];
-        } else {
-          const float x = resid[oi] + v[a][j];
-          out[oi] = x;
-          if (out2) out2[oi] = x;
-        }
-      }
-    }
-  }
-}
-
-// ------------------------------------------------------------------------------
-// Big-tile variant for GEMMs with many blocks.  A block computes kGBM = 32
-// activation rows (96 limb rows) by kGPan = 16 panel slots (SwiGLU: the gate
-// and the up panels of 8 column groups).  Four waves; wave (wr, wc) owns rows
-// 16wr..16wr+15 (one A tile per limb) and 8 panel slots: 24 accumulators.
-// Both operands of a K step (A 12 KiB, B 16 KiB) go from global memory
-// straight into LDS (global_load_lds_dwordx4: each wave instruction fills
-// 1 KiB, lane l the 16 bytes at l * 16), in a ring of two steps: 56 KiB, so
-// two blocks share a CU and one block's barriers, pipeline start and epilogue
-// overlap the other's MFMAs (with one 8-wave block per CU, the per-step
-// barrier and the epilogue left the MFMA units idle for a third of the time).
-// A limb rows are stored without padding, the 16-byte chunk c of row r at
-// chunk position c ^ a_swz(r): the rows one A fragment read touches then fall
-// in different bank groups.
-//
-// EPI_SWIGLU: wave column wc holds the gate panels of column groups
-// CGW wc .. CGW wc + CGW - 1 (slots j < CGW, CGW = PS / 4) and the up panels
-// of the same groups (j >= CGW), so each output's gate and up values meet in
-// one lane.
-//
-// PS = 16 panel slots per block, 20 (wave tile 3 A tiles x 10 panels) or 10
-// (3 x 5) for launches whose 16-slot tiles leave a last round of blocks
-// mostly empty: O and Down at 2048 rows (N = 160 panels) make 512
-// twenty-slot tiles, one full round at two blocks per CU, against 640
-// sixteen-slot ones (1.25 rounds).  The 20-slot tile also reads each A step
-// for 20 panels instead of 16 or 10.  For SwiGLU a block of PS slots holds
-// the gate and up panels of PS / 2 column groups, PS / 4 per wave column.
-// ------------------------------------------------------------------------------
-constexpr int kGBM = 32;                     // activation rows per block
-constexpr int kGPan = 16;                    // panel slots per block (wide tile)
-constexpr int kGPanNarrow = 10;              // panel slots per block (narrow tile)
-constexpr int kGPanWide = 20;                // panel slots per block (20-slot tile)
-constexpr int kGStageA = kLimbs * kGBM * 128;  // 96 limb rows x 128 bytes
-constexpr int kGStages = 2;
-constexpr int kGNT = 256;                    // threads per block
-// one super-tile per panel slot after the A step; two stages
-constexpr int gemm_big_stage(int ps) { return kGStageA + ps * 1024; }
-constexpr int gemm_big_lds(int ps) { return kGStages * gemm_big_stage(ps); }
-
-template <int EPI, int PS>
-__global__ __launch_bounds__(kGNT, 2) void k_gemm_big(GemmArgs g) {
-  static_assert(PS == kGPan || PS == kGPanWide || (PS == kGPanNarrow && EPI != EPI_SWIGLU),
-                "panel slots");
-  constexpr int PW = PS / 2;                 // panel slots per wave
+template <int EPI, int RT, int PW>
+__global__ __launch_bounds__(kGNT, 2) void k_gemm(GemmArgs g) {
+  constexpr int PS = 2 * PW;                 // panel slots per block
+  constexpr int BM = kGRows * RT;            // activation rows per block
   constexpr int CG = PS / 2;                 // SwiGLU: column groups per block
   constexpr int CGW = CG / 2;                // SwiGLU: column groups per wave column
-  constexpr int kGStage = gemm_big_stage(PS);
+  constexpr int kA = kLimbs * BM * 128;      // A bytes of a stage
+  constexpr int kStage = gemm_stage(RT, PW), kStages = gemm_stages(RT, PW);
+  static_assert(EPI != EPI_SWIGLU || PW % 2 == 0, "gate and up panels of a wave");
   extern __shared__ __align__(16) uint8_t lds[];
   const int M = launder(g.M), K = launder(g.K);
   const int8_t *limbs = launder(g.a.limbs);
@@ -403,13 +133,13 @@ __global__ __launch_bounds__(kGNT, 2) void k_gemm_big(GemmArgs g) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lane = tid & 63;
   const int wr = wave & 1, wc = wave >> 1;
-  const int r0 = blockIdx.y * kGBM;
+  const int r0 = blockIdx.y * BM;
   const int KG = K >> 7;
 
   // panel slot -> weights, scale, first column, valid (block-uniform selects)
   auto slot = [=](int sl, const uint8_t **w, float *sc, int *col, bool *ok) {
     if constexpr (EPI == EPI_SWIGLU) {
-      const int half = sl / CG, cp = blockIdx.x * CG + sl % CG;
+      const int half = sl >= CG ? 1 : 0, cp = blockIdx.x * CG + sl - half * CG;
       *ok = cp < sn0;
       *w = (half == 0 ? sw0 : sw1) + (size_t)(*ok ? cp : 0) * K * 8;
       *sc = half == 0 ? ss0 : ss1;
@@ -425,101 +155,167 @@ __global__ __launch_bounds__(kGNT, 2) void k_gemm_big(GemmArgs g) {
     else return PW * wc + j;
   };
   // this wave loads panel slots wave, wave + 4, .. (an invalid slot loads a
-  // valid panel)
+  // valid panel, one past the last slot its first one)
   constexpr int kBL = (PS + 3) / 4;  // B loads per wave per step (the most)
-  const uint8_t *lw[kBL];
+  __amdgpu_buffer_rsrc_t bsrc[kBL];
 #pragma unroll
   for (int j = 0; j < kBL; ++j) {
+    const uint8_t *w;
     float sc;
     int col;
     bool ok;
-    slot(wave + 4 * j < PS ? wave + 4 * j : wave, &lw[j], &sc, &col, &ok);
+    slot(wave + 4 * j < PS ? wave + 4 * j : wave, &w, &sc, &col, &ok);
+    bsrc[j] = buffer_of(launder(w), K * 8);
   }
-  // A: a stage holds limb rows 32l + m (limb l of block row m); this wave
-  // fills LDS blocks 3 wave + i (stage rows 8q .. 8q + 7); lane l writes row
-  // 8q + l / 8 at chunk position l % 8, which holds chunk (l % 8) ^
-  // a_swz(row) of the row
+  // A: a stage holds limb rows BM l + m (limb l of block row m); this wave
+  // fills rows 8 (RT wave + u) .. + 7 of every limb; lane l writes row
+  // + l / 8 at chunk position l % 8, which holds chunk (l % 8) ^ a_swz(row) of
+  // the row.  Rows past the planes read zeros.
   const int pr = launder(g.a.plane_rows);
-  const int8_t *asrc[kLimbs];
+  __amdgpu_buffer_rsrc_t asrc[kLimbs];
 #pragma unroll
-  for (int i = 0; i < kLimbs; ++i) {
-    const int row = 8 * (kLimbs * wave + i) + (lane >> 3);
-    const int c = (lane & 7) ^ a_swz(row);
-    asrc[i] = limbs + ((size_t)(row >> 5) * pr + r0 + (row & 31)) * K + c * 16;
+  for (int l = 0; l < kLimbs; ++l)
+    asrc[l] = buffer_of(launder(limbs + ((size_t)l * pr + r0) * K), min(pr - r0, BM) * K);
+  int aoff[RT];
+#pragma unroll
+  for (int u = 0; u < RT; ++u) {
+    const int row = 8 * (RT * wave + u) + (lane >> 3);
+    aoff[u] = row * K + ((lane & 7) ^ a_swz(row)) * 16;
   }
   auto issue = [&](int G, int stg) {
-    uint8_t *sa = lds + stg * kGStage;
+    uint8_t *sa = lds + stg * kStage;
 #pragma unroll
-    for (int i = 0; i < kLimbs; ++i)
-      __builtin_amdgcn_global_load_lds((gbl_void *)(asrc[i] + (size_t)G * 128),
-                                       (lds_void *)(sa + (kLimbs * wave + i) * 1024), 16, 0, 0);
+    for (int l = 0; l < kLimbs; ++l)
+#pragma unroll
+      for (int u = 0; u < RT; ++u)
+        load_lds16(asrc[l], sa + (BM * l + 8 * (RT * wave + u)) * 128, aoff[u], G * 128);
 #pragma unroll
     for (int j = 0; j < kBL; ++j)
-      if (wave + 4 * j < PS)
-        __builtin_amdgcn_global_load_lds((gbl_void *)(lw[j] + (size_t)G * 1024 + lane * 16),
-                                         (lds_void *)(sa + kGStageA + (wave + 4 * j) * 1024), 16,
-                                         0, 0);
+      if (4 * j + 3 < PS || wave + 4 * j < PS)
+        load_lds16(bsrc[j], sa + kA + (wave + 4 * j) * 1024, lane * 16, G * 1024);
   };
 
-  // acc[l][j]: limb l of block rows 16 wr .. 16 wr + 15, panel slot wslot(j)
-  v4i acc[kLimbs][PW];
+  // acc[l][u][j]: limb l of block rows 16 (RT wr + u) .. + 15, panel slot wslot(j)
+  v4i acc[kLimbs][RT][PW];
 #pragma unroll
   for (int a = 0; a < kLimbs; ++a)
 #pragma unroll
-    for (int j = 0; j < PW; ++j) acc[a][j] = v4i{0, 0, 0, 0};
+    for (int u = 0; u < RT; ++u)
+#pragma unroll
+      for (int j = 0; j < PW; ++j) acc[a][u][j] = v4i{0, 0, 0, 0};
 
   const int li = lane & 15, lg = lane >> 4;
   const int swz = a_swz(li);  // a_swz(row) for every row this lane reads
+  const int apos[2] = {(16 * RT * wr + li) * 128 + ((2 * lg) ^ swz) * 16,
+                       (16 * RT * wr + li) * 128 + ((2 * lg + 1) ^ swz) * 16};
+  // One K step: two halves of 64 values.  The order is written out and held by
+  // scheduling barriers: the next A fragment is read before the MFMAs of each,
+  // and the second half's weights are unpacked between MFMAs.  (Left to itself
+  // the compiler reads each fragment right before its MFMAs and waits for it.)
   auto compute = [&](int stg) {
-    const uint8_t *sa = lds + stg * kGStage;
-    const uint8_t *sb = sa + kGStageA + lane * 16;
-    u32x4 braw[PW];
+    const uint8_t *sa = lds + stg * kStage;
+    const uint8_t *sb = sa + kA + lane * 16;
+    constexpr int NA = kLimbs * RT;  // A fragments per half step
+    v4i af[2];
+    auto aread = [&](int h, int t) {
+      return *reinterpret_cast<const v4i *>(sa + (BM * (t / RT) + 16 * (t % RT)) * 128 + apos[h]);
+    };
+    if constexpr (RT * PW <= 12) {
+      v4i bf[2][PW];
+      u32x4 raw[PW];
+      auto unpack = [&](int h, int j) {
+        const uint32_t d0 = raw[j][2 * h], d1 = raw[j][2 * h + 1];
+        bf[h][j] = v4i{(int)(d0 & 0x0F0F0F0Fu), (int)((d0 >> 4) & 0x0F0F0F0Fu),
+                       (int)(d1 & 0x0F0F0F0Fu), (int)((d1 >> 4) & 0x0F0F0F0Fu)};
+      };
 #pragma unroll
-    for (int j = 0; j < PW; ++j) braw[j] = *reinterpret_cast<const u32x4 *>(sb + wslot(j) * 1024);
+      for (int j = 0; j < PW; ++j)
+        raw[j] = *reinterpret_cast<const u32x4 *>(sb + wslot(j) * 1024);
+      af[0] = aread(0, 0);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      v4i bf[PW];
+      for (int j = 0; j < PW; ++j) unpack(0, j);
 #pragma unroll
-      for (int j = 0; j < PW; ++j) {
-        const uint32_t d0 = braw[j][2 * h], d1 = braw[j][2 * h + 1];
-        bf[j] = v4i{(int)(d0 & 0x0F0F0F0Fu), (int)((d0 >> 4) & 0x0F0F0F0Fu),
-                    (int)(d1 & 0x0F0F0F0Fu), (int)((d1 >> 4) & 0x0F0F0F0Fu)};
+      for (int q = 0; q < 2 * NA; ++q) {
+        const int h = q / NA, t = q % NA;
+        __builtin_amdgcn_sched_barrier(0);
+        if (q + 1 < 2 * NA) af[(q + 1) & 1] = aread((q + 1) / NA, (q + 1) % NA);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < PW; ++j) {
+          acc[t / RT][t % RT][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+              af[q & 1], bf[h][j], acc[t / RT][t % RT][j], 0, 0, 0);
+          // (the second half's words between the first half's MFMAs)
+          if (h == 0 && (q * PW + j) % NA == 0) unpack(1, (q * PW + j) / NA);
+        }
       }
-      const int pos = (2 * lg + h) ^ swz;
-#pragma unroll
-      for (int a = 0; a < kLimbs; ++a) {
-        const v4i af = *reinterpret_cast<const v4i *>(sa + (32 * a + 16 * wr + li) * 128 +
-                                                      pos * 16);
+    } else {
+      // 192 accumulators: one half's weights at a time
+      v4i bf[PW];
+      u32x2 raw[PW];
+      auto braw = [&](int h) {
+        asm volatile("" ::: "memory");  // (or the halves' reads become one)
 #pragma unroll
         for (int j = 0; j < PW; ++j)
-          acc[a][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, bf[j], acc[a][j], 0, 0, 0);
+          raw[j] = *reinterpret_cast<const u32x2 *>(sb + wslot(j) * 1024 + 8 * h);
+      };
+      auto unpack = [&](int j) {
+        bf[j] = v4i{(int)(raw[j].x & 0x0F0F0F0Fu), (int)((raw[j].x >> 4) & 0x0F0F0F0Fu),
+                    (int)(raw[j].y & 0x0F0F0F0Fu), (int)((raw[j].y >> 4) & 0x0F0F0F0Fu)};
+      };
+      braw(0);
+      af[0] = aread(0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < PW; ++j) unpack(j);
+#pragma unroll
+      for (int q = 0; q < 2 * NA; ++q) {
+        const int t = q % NA;
+        __builtin_amdgcn_sched_barrier(0);
+        if (q == NA - 2) braw(1);
+        if (q + 1 < 2 * NA) af[(q + 1) & 1] = aread((q + 1) / NA, (q + 1) % NA);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < PW; ++j) {
+          acc[t / RT][t % RT][j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+              af[q & 1], bf[j], acc[t / RT][t % RT][j], 0, 0, 0);
+          if (q == NA - 1) {
+            if (j > 0) unpack(j - 1);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        if (q == NA - 1) unpack(PW - 1);
       }
     }
   };
 
-  // Ring of two K steps: step G + 1 is issued into the stage step G - 1 used,
-  // once every wave has passed the barrier after computing it.  The barrier
-  // is a bare s_barrier after this wave's own loads of step G have landed.
-  issue(0, 0);
-  for (int G = 0; G < KG; ++G) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  // K steps of this block: all of them, or part blockIdx.z of ksplit
+  const int ks = EPI == EPI_PART ? launder(g.ksplit) : 1;
+  const int G0 = (int)((long)KG * blockIdx.z / ks);
+  const int NG = (int)((long)KG * (blockIdx.z + 1) / ks) - G0;
+  // Ring of kStages K steps: step i + kStages - 1 is issued into the stage that
+  // step i - 1 used, once every wave has passed the barrier after computing it.
+  // The barrier is a bare s_barrier after this wave's own loads of step i have
+  // landed (a __syncthreads would wait for the later steps' too).
+  constexpr int kLoads = kLimbs * RT + kBL;  // a wave's loads per step
+  static_assert(kStages == 2 || PS % 4 == 0, "a ring of three counts every wave's loads");
+  issue(G0, 0);
+  if (kStages == 3 && NG > 1) issue(G0 + 1, 1);
+  for (int i = 0; i < NG; ++i) {
+    if (kStages == 3 && i + 1 < NG)
+      __builtin_amdgcn_s_waitcnt(0x0070 | kLoads);  // vmcnt(kLoads) lgkmcnt(0)
+    else
+      __builtin_amdgcn_s_waitcnt(0x0070);            // vmcnt(0) lgkmcnt(0)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (G + 1 < KG) issue(G + 1, (G + 1) & 1);
-    compute(G & 1);
+    const int n = i + kStages - 1;
+    if (n < NG) issue(G0 + n, n % kStages);
+    compute(i % kStages);
   }
 
   // ---- epilogue: lane (column jc, row rr of each A tile)
   const int jc = lane & 15, rr = lane >> 4;
-  // lane j + 16 rr holds rows 16 wr + 4 rr + i of column j
-  double rsc[4], rz[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = r0 + 16 * wr + 4 * (lane >> 4) + i;
-    rsc[i] = row < M ? (double)ldexpf(1.0f, -ldg<int32_t>(shift + row)) : 0.0;
-    rz[i] = row < M ? (double)(8 * ldg<long long>(xsum + row)) : 0.0;
-  }
   float wsc[PW];
   int col[PW];
   bool pv[PW];
@@ -528,115 +324,119 @@ __global__ __launch_bounds__(kGNT, 2) void k_gemm_big(GemmArgs g) {
     const uint8_t *w;
     slot(wslot(j), &w, &wsc[j], &col[j], &pv[j]);
   }
-  auto value = [&](int i, int j) {
-    return (float)(limb_combine3(acc[0][j][i], acc[1][j][i], acc[2][j][i], rz[i]) * rsc[i] *
-                   (double)wsc[j]);
-  };
-  if constexpr (EPI == EPI_SWIGLU) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int row = r0 + 16 * wr + 4 * rr + a;
+  for (int u = 0; u < RT; ++u)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // lane j + 16 rr holds rows 16 (RT wr + u) + 4 rr + i of column j
+      const int row = r0 + 16 * (RT * wr + u) + 4 * rr + i;
       if (row >= M) continue;
+      if constexpr (EPI == EPI_PART) {
+        // exact sums d0 + 2^8 d1 + 2^16 d2
+        int64_t *kp = launder(g.kpart) + ((size_t)blockIdx.z * M + row) * ldo;
 #pragma unroll
-      for (int j = 0; j < CGW; ++j) {
-        if (!pv[j]) continue;
-        const float gt = value(a, j), up = value(a, j + CGW);
-        sw_out[(size_t)row * ldo_sw + col[j] + jc] = up * gt * (1.0f / (1.0f + expf(-gt)));
+        for (int j = 0; j < PW; ++j)
+          if (pv[j])
+            kp[col[j] + jc] = (int64_t)acc[0][u][j][i] + ((int64_t)acc[1][u][j][i] << 8) +
+                              ((int64_t)acc[2][u][j][i] << 16);
+        continue;
       }
-    }
-  } else {
+      const double rsc = (double)ldexpf(1.0f, -ldg<int32_t>(shift + row));
+      const double rz = (double)(8 * ldg<long long>(xsum + row));
+      auto value = [&](int j) {
+        return (float)(limb_combine3(acc[0][u][j][i], acc[1][u][j][i], acc[2][u][j][i], rz) *
+                       rsc * (double)wsc[j]);
+      };
+      if constexpr (EPI == EPI_SWIGLU) {
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int row = r0 + 16 * wr + 4 * rr + a;
-      if (row >= M) continue;
+        for (int j = 0; j < CGW; ++j) {
+          if (!pv[j]) continue;
+          const float gt = value(j), up = value(j + CGW);
+          sw_out[(size_t)row * ldo_sw + col[j] + jc] = up * gt * (1.0f / (1.0f + expf(-gt)));
+        }
+      } else {
 #pragma unroll
-      for (int j = 0; j < PW; ++j) {
-        if (!pv[j]) continue;
-        const size_t oi = (size_t)row * ldo + col[j] + jc;
-        const float x = value(a, j);
-        if constexpr (EPI == EPI_STORE) {
-          out[oi] = x;
-        } else if constexpr (EPI == EPI_ACCUMULATE) {
-          out[oi] += x;
-        } else {
-          const float y = resid[oi] + x;
-          out[oi] = y;
-          if (out2) out2[oi] = y;
+        for (int j = 0; j < PW; ++j) {
+          if (!pv[j]) continue;
+          const size_t oi = (size_t)row * ldo + col[j] + jc;
+          const float x = value(j);
+          if constexpr (EPI == EPI_STORE) {
+            out[oi] = x;
+          } else if constexpr (EPI == EPI_ACCUMULATE) {
+            out[oi] += x;
+          } else {
+            const float y = resid[oi] + x;
+            out[oi] = y;
+            if (out2) out2[oi] = y;
+          }
         }
       }
     }
-  }
 }
 
 }  // namespace
 
-// Rows of the quantized operand a GEMM reads: the big tile's row block.
-int gemm_row_pad(int M) { return (M + kGBM - 1) / kGBM * kGBM; }
+// Rows of the quantized operand a GEMM reads: rows of whole tiles of 32.
+int gemm_row_pad(int M) { return (M + kGRows - 1) / kGRows * kGRows; }
 
 namespace {
 
-// The kernel for a GEMM, from a model of its time in wide-tile K steps: a
-// launch of B blocks runs ceil(B / slots) rounds (two blocks per CU); a K step
-// of the 10-slot tile costs 0.85 of a 16-slot one (5/8 of the MFMAs, but more
-// LDS reads and barriers per MFMA), and the 32-row, 8-panel kernel's 0.8: the
-// factors that reproduce the measured choices (at 2048 rows O and Down run
-// 146 us with 16 slots, 126 us with 10; at 512 rows the 32-row kernel's 49 us
-// beat the 10-slot tile's 52).  (A split of K over several blocks, their
-// exact partials meeting through a counter or in a second launch, was
-// slower: see the notes on the measured variants.)
-constexpr double kNarrowStepCost = 0.85;
-// the 20-slot tile's K step: 1.25 times the MFMAs of a 16-slot one, less the
-// A reads it saves (each A step serves 20 panels).  At 2048 rows O and Down
-// make 512 twenty-slot tiles, one round (TTFT at 2048 tokens 32.9 -> 32.4
-// ms), and Gate|Up 4096 tiles, 8 rounds against 10 (31.9 -> 31.4 ms; 512
-// tokens 10.5 -> 10.3 ms)
-constexpr double kWideStepCost = 1.2;
-constexpr double kSmallStepCost = 0.8;
+// The tiles, and the time of one K step in a full round of blocks (two per CU),
+// microseconds, from launches of 32 to 2048 rows on the E4B and 14B matrices.
+struct Tile {
+  int rt, pw;
+  double step;
+};
+constexpr Tile kTiles[] = {{2, 8, 2.40}, {2, 6, 1.96}, {2, 5, 1.65},
+                           {1, 8, 1.35}, {1, 5, 0.88}, {1, 4, 0.80}};
+constexpr int kPartTile = 5;  // the tile of a K part
 
-// 0: the 32-row kernel; else the big tile's panel slots (16, 20 or 10)
-int gemm_pick(const GemmArgs &g, int np) {
-  const bool swiglu = g.epi == EPI_SWIGLU;
-  const long slots = 2L * (ctx().n_cu > 0 ? ctx().n_cu : 256);
-  auto rounds = [&](long blocks) { return (double)((blocks + slots - 1) / slots); };
-  const long rows = gemm_row_pad(g.M) / kGBM;
-  const long wide = (long)(swiglu ? (np / 2 + 7) / 8 : (np + kGPan - 1) / kGPan) * rows;
-  const long narrow = (long)((np + kGPanNarrow - 1) / kGPanNarrow) * rows;
-  const long small = (long)(swiglu ? (np / 2 + 2 * kWB - 1) / (2 * kWB)
-                                   : (np + 4 * kWB - 1) / (4 * kWB)) *
-                     ((g.M + kBM - 1) / kBM);
-  const long wide20 =
-      (long)(swiglu ? (np / 2 + kGPanWide / 2 - 1) / (kGPanWide / 2)
-                    : (np + kGPanWide - 1) / kGPanWide) * rows;
-  int pick = kGPan;
-  double cost = rounds(wide);
-  if (rounds(wide20) * kWideStepCost < cost) {
-    pick = kGPanWide;
-    cost = rounds(wide20) * kWideStepCost;
-  }
-  if (!swiglu && rounds(narrow) * kNarrowStepCost < cost) {
-    pick = kGPanNarrow;
-    cost = rounds(narrow) * kNarrowStepCost;
-  }
-  if (rounds(small) * kSmallStepCost < cost) pick = 0;
-  return pick;
+long gemm_slots() { return 2L * (ctx().n_cu > 0 ? ctx().n_cu : 256); }
+
+dim3 tile_grid(const Tile &t, int M, int np, bool swiglu) {
+  const int cols = swiglu ? (np / 2 + t.pw - 1) / t.pw : (np + 2 * t.pw - 1) / (2 * t.pw);
+  return dim3(cols, (M + kGRows * t.rt - 1) / (kGRows * t.rt));
 }
 
-template <int PS>
-void launch_big(const GemmArgs &g, int np, hipStream_t st) {
-  const int gxb = g.epi == EPI_SWIGLU ? (np / 2 + PS / 2 - 1) / (PS / 2) : (np + PS - 1) / PS;
-  const dim3 grid(gxb, gemm_row_pad(g.M) / kGBM);
-  const size_t lds = gemm_big_lds(PS);
+// Time of a K step of `blocks` blocks: the full rounds, and for what is left 0.58
+// of a round with at most one block per CU (a lone block's waves wait for their
+// own chain), nearly a whole one above.  Down at 1024, 1536 and 2048 rows (256, 384
+// and 512 blocks of the 2 x 5 tile) 88, 128, 149 us; 640 blocks of the 1 x 8 tile
+// 1.6 rounds, 640 to 960 of the 1 x 4 tile 1.55 to 2.0.
+double step_time(const Tile &t, long blocks) {
+  const long slots = gemm_slots(), part = blocks % slots;
+  return ((double)(blocks / slots) + (part == 0 ? 0.0 : 2 * part <= slots ? 0.58 : 0.96)) *
+         t.step;
+}
+
+// The tile with the least time by that rule.
+const Tile &gemm_pick(int M, int np, bool swiglu, double *step) {
+  const Tile *pick = nullptr;
+  for (const Tile &t : kTiles) {
+    if (swiglu && t.pw % 2) continue;
+    const dim3 g = tile_grid(t, M, np, swiglu);
+    const double s = step_time(t, (long)g.x * g.y);
+    if (!pick || s < *step) {
+      pick = &t;
+      *step = s;
+    }
+  }
+  return *pick;
+}
+
+template <int RT, int PW>
+void launch_tile(const GemmArgs &g, dim3 grid, hipStream_t st) {
+  const size_t lds = gemm_lds(RT, PW);
+#define MS_GEMM(E) hipLaunchKernelGGL((k_gemm<E, RT, PW>), grid, dim3(kGNT), lds, st, g)
   switch (g.epi) {
-    case EPI_STORE: hipLaunchKernelGGL((k_gemm_big<EPI_STORE, PS>), grid, dim3(kGNT), lds, st, g); break;
-    case EPI_ACCUMULATE:
-      hipLaunchKernelGGL((k_gemm_big<EPI_ACCUMULATE, PS>), grid, dim3(kGNT), lds, st, g);
-      break;
-    case EPI_RESID: hipLaunchKernelGGL((k_gemm_big<EPI_RESID, PS>), grid, dim3(kGNT), lds, st, g); break;
+    case EPI_STORE: MS_GEMM(EPI_STORE); break;
+    case EPI_ACCUMULATE: MS_GEMM(EPI_ACCUMULATE); break;
+    case EPI_RESID: MS_GEMM(EPI_RESID); break;
     default:
-      if constexpr (PS == kGPan || PS == kGPanWide)
-        hipLaunchKernelGGL((k_gemm_big<EPI_SWIGLU, PS>), grid, dim3(kGNT), lds, st, g);
+      if constexpr (PW % 2 == 0) MS_GEMM(EPI_SWIGLU);
       break;
   }
+#undef MS_GEMM
 }
 
 }  // namespace
@@ -655,24 +455,47 @@ __global__ __launch_bounds__(256) void k_gemm_kcombine(GemmArgs g) {
   const float sc = ldexpf(1.0f, -ldg<int32_t>(g.a.shift + row));
   const float v = (float)(((double)t - z8) * (double)sc * (double)g.seg[0].scale);
   float *o = g.out + (size_t)row * N + c;
-  if constexpr (EPI == EPI_STORE) *o = v;
-  else *o += v;
+  if constexpr (EPI == EPI_STORE) {
+    *o = v;
+  } else if constexpr (EPI == EPI_ACCUMULATE) {
+    *o += v;
+  } else {
+    const float x = g.resid[(size_t)row * N + c] + v;
+    *o = x;
+    if (g.out2) g.out2[(size_t)row * N + c] = x;
+  }
 }
 
+size_t gemm_part_bytes() {
+  // at most two part blocks per CU, each with the int64 sums of one tile
+  const Tile &t = kTiles[kPartTile];
+  return (size_t)gemm_slots() * kGRows * t.rt * 32 * t.pw * 8;
+}
+
+// The number of parts with the least time: a part's K steps, about 2 us for the
+// combine's launch, and the partial sums written and read back at 6 TB/s.  Down
+// (K = 10240) at 32, 64, 128, 256 rows: 43.2, 44.2, 45.5, 47.1 us in one part;
+// 19.5, 21.5, 27.9, 36.1 split in 8, 6, 3 and 3.  O (K = 2048) gains up to 32 rows
+// only (14.4 -> 13.3 us; at 128 rows the split would cost 1.5 us).
 int gemm_ksplit(int M, int K, int N) {
   if (M <= kGemvMaxM || K % 128 != 0 || N % 16 != 0) return 1;
-  GemmArgs g{};
-  g.epi = EPI_STORE;
-  g.M = M;
-  g.K = K;
-  g.nseg = 1;
-  const int np = N / 16;
-  if (gemm_pick(g, np) != 0) return 1;
-  const long blocks = (long)((np + 4 * kWB - 1) / (4 * kWB)) * ((M + kBM - 1) / kBM);
-  const long cus = ctx().n_cu > 0 ? ctx().n_cu : 256;
-  long ks = cus / blocks;
-  ks = std::min<long>(ks, std::min(8, K / 128 / 8));  // at least 8 K steps a part
-  return ks > 1 ? (int)ks : 1;
+  const Tile &t = kTiles[kPartTile];
+  const dim3 g = tile_grid(t, M, N / 16, false);
+  const long blocks = (long)g.x * g.y;
+  const int steps = K / 128;
+  double best = 0;
+  gemm_pick(M, N / 16, false, &best);
+  best *= steps;
+  int ks = 1;
+  for (int k = 2; k <= 8 && 4 * k <= steps && blocks * k <= gemm_slots(); ++k) {
+    const double us = (steps + k - 1) / k * step_time(t, blocks * k) + 2.0 +
+                      16e-6 * k * (double)M * N / 6.0;
+    if (us < best) {
+      best = us;
+      ks = k;
+    }
+  }
+  return ks;
 }
 
 int launch_gemm(const GemmArgs &g, hipStream_t st) {
@@ -696,41 +519,32 @@ int launch_gemm(const GemmArgs &g, hipStream_t st) {
   for (int i = 0; i < g.nseg; ++i) np += g.seg[i].n_cols / 16;
   const bool swiglu = g.epi == EPI_SWIGLU;
   if (g.ksplit > 1) {
-    MS_CHECK_ARG((g.epi == EPI_STORE || g.epi == EPI_ACCUMULATE) && g.nseg == 1 && g.kpart &&
-                     g.ldo == g.seg[0].n_cols && g.ksplit <= g.K / 128,
-                 "GEMM: K split needs one segment, store or accumulate, ldo = N");
-    const dim3 grid((np + 4 * kWB - 1) / (4 * kWB), (g.M + kBM - 1) / kBM, g.ksplit);
+    MS_CHECK_ARG(!swiglu && g.nseg == 1 && g.kpart && g.ldo == g.seg[0].n_cols &&
+                     g.ksplit <= g.K / 128,
+                 "GEMM: K split needs one segment, a plain epilogue, ldo = N");
+    dim3 grid = tile_grid(kTiles[kPartTile], g.M, np, false);
+    grid.z = g.ksplit;
     const dim3 cgrid((g.ldo + 255) / 256, g.M);
-    if (g.epi == EPI_STORE) {
-      hipLaunchKernelGGL(k_gemm<EPI_STORE>, grid, dim3(kNT), kGemmLds, st, g);
+    hipLaunchKernelGGL((k_gemm<EPI_PART, 1, 4>), grid, dim3(kGNT), gemm_lds(1, 4), st, g);
+    if (g.epi == EPI_STORE)
       hipLaunchKernelGGL(k_gemm_kcombine<EPI_STORE>, cgrid, dim3(256), 0, st, g);
-    } else {
-      hipLaunchKernelGGL(k_gemm<EPI_ACCUMULATE>, grid, dim3(kNT), kGemmLds, st, g);
+    else if (g.epi == EPI_ACCUMULATE)
       hipLaunchKernelGGL(k_gemm_kcombine<EPI_ACCUMULATE>, cgrid, dim3(256), 0, st, g);
-    }
+    else
+      hipLaunchKernelGGL(k_gemm_kcombine<EPI_RESID>, cgrid, dim3(256), 0, st, g);
     MS_HIP_TRY(hipGetLastError());
     return MS_OK;
   }
-  const int pick = gemm_pick(g, np);
-  if (pick == kGPan) {
-    launch_big<kGPan>(g, np, st);
-  } else if (pick == kGPanWide) {
-    launch_big<kGPanWide>(g, np, st);
-  } else if (pick == kGPanNarrow) {
-    launch_big<kGPanNarrow>(g, np, st);
-  } else {
-    const dim3 blk(kNT);
-    const int gy = (g.M + kBM - 1) / kBM;
-    const dim3 grid(swiglu ? (np / 2 + 2 * kWB - 1) / (2 * kWB) : (np + 4 * kWB - 1) / (4 * kWB),
-                    gy);
-#define MS_GS(E) hipLaunchKernelGGL(k_gemm<E>, grid, blk, kGemmLds, st, g)
-    switch (g.epi) {
-      case EPI_STORE: MS_GS(EPI_STORE); break;
-      case EPI_ACCUMULATE: MS_GS(EPI_ACCUMULATE); break;
-      case EPI_RESID: MS_GS(EPI_RESID); break;
-      default: MS_GS(EPI_SWIGLU); break;
-    }
-#undef MS_GS
+  double step = 0;
+  const Tile &t = gemm_pick(g.M, np, swiglu, &step);
+  const dim3 grid = tile_grid(t, g.M, np, swiglu);
+  switch (t.rt * 100 + t.pw) {
+    case 208: launch_tile<2, 8>(g, grid, st); break;
+    case 206: launch_tile<2, 6>(g, grid, st); break;
+    case 205: launch_tile<2, 5>(g, grid, st); break;
+    case 108: launch_tile<1, 8>(g, grid, st); break;
+    case 105: launch_tile<1, 5>(g, grid, st); break;
+    default: launch_tile<1, 4>(g, grid, st); break;
   }
   MS_HIP_TRY(hipGetLastError());
   return MS_OK;

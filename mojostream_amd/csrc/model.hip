@@ -112,6 +112,7 @@ struct ms_model {
   // quantized activation rows for projections whose rows do not fit in LDS
   void *quant = nullptr;
   int quant_k = 0;
+  int64_t *kpart = nullptr;  // sums of the K parts of a short prompt's O and Down
   float *qkv = nullptr, *attn_part = nullptr;
   float *rope_cur = nullptr;  // one-row decode: RoPE factors at the position [2][256]
   unsigned *attn_ctr = nullptr;  // decode attention counters (attn_ctr_count), kept zero
@@ -289,6 +290,10 @@ static int launch_proj(ms_model *m, GemvArgs a, const RowSrc &r, int waves, hipS
     g.out2 = a.out2;
     g.sw_out = a.sw_out;
     g.ldo_sw = a.ldo_sw;
+    if (a.epi == EPI_RESID && a.nseg == 1 && a.ldo == a.seg[0].n_cols) {
+      g.ksplit = gemm_ksplit(a.M, a.K, a.ldo);
+      g.kpart = m->kpart;
+    }
     if (int rc = launch_quant_rows3(r, a.M, a.K, g.a, st)) return rc;
     return launch_gemm(g, st);
   }
@@ -884,6 +889,7 @@ extern "C" int ms_model_create(const ms_model_desc *desc, const ms_layer_desc *l
       (rc = dmalloc(m, &m->quant, quant_rows_bytes(gemm_row_pad(M), m->quant_k))))
     return cleanup(rc);
   if (m->prefill_rows > kGemvMaxM) {
+    if ((rc = dmalloc(m, (void **)&m->kpart, gemm_part_bytes()))) return cleanup(rc);
     // the workspace of any prefill attention launch
     for (auto &Ly : m->L) {
       AttnArgs a{};

@@ -141,7 +141,8 @@ struct GemmArgs {
   float *out2;         // EPI_RESID: optional copy
   float *sw_out;       // EPI_SWIGLU: [M][ldo_sw]
   int ldo_sw;
-  // K split over ksplit block groups (> 1: one segment, store or accumulate):
+  // K split over ksplit block groups (> 1: one segment, store, accumulate or
+  // residual):
   // each group stores its exact partial sums, int64 [ksplit][M][N], and a
   // combine kernel adds them and scales (the same value as without the split)
   int ksplit;
@@ -180,6 +181,8 @@ int launch_gemm(const GemmArgs &g, hipStream_t st);
 // K parts for C = A deq(W) with M rows, one segment: > 1 where the 32-row
 // GEMM would leave most CUs idle (a few row and column tiles, long K)
 int gemm_ksplit(int M, int K, int N);
+// Bytes of the partial sums of any such split.
+size_t gemm_part_bytes();
 // Rows a GEMM reads from its quantized operand (M rounded up to the row tile).
 int gemm_row_pad(int M);
 
