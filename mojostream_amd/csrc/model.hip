@@ -308,7 +308,8 @@ static int launch_proj(ms_model *m, GemvArgs a, const RowSrc &r, int waves, hipS
     if (gemv_lds_need(a) <= kLdsLimit) return launch_gemv_rec(a, st);
     a.waves = waves;
   }
-  if (a.K <= 8 * 2 * 64 * waves && gemv_lds_need(a) <= kLdsLimit) return launch_gemv_rec(a, st);
+  if (a.M <= 4 && a.K <= 8 * 2 * 64 * waves && gemv_lds_need(a) <= kLdsLimit)
+    return launch_gemv_rec(a, st);
   a.asrc = AS_QUANT;
   a.rows = RowSrc{};
   a.q = quant_rows_view(m->quant, a.M, a.K);

@@ -79,7 +79,8 @@ struct RowSrc {
 
 // Quantized rows in global memory: limb l of row m at
 // limbs[(4m + l) * K + limb position of k] (MFMA fragment order per 128-row
-// super-tile), shift[m] = s.  The GEMM's operand (launch_quant_rows3) has
+// super-tile), shift[m] = s; more than four rows: whole MFMA fragments (frag_pos
+// in q4.hip).  The GEMM's operand (launch_quant_rows3) has
 // three limbs in planes: limb l of row m at limbs[(l * plane_rows + m) * K +
 // limb position of k].
 struct QuantRows {

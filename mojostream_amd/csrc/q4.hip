@@ -285,14 +285,24 @@ __device__ inline void block_sum_max(float &ss, float &mx, float *sh, bool fresh
   mx = u;
 }
 
+// Limb l of the 8-value group q of row m for k_gemv_rows: whole A fragments, one
+// KiB per row group of four rows, super-tile and MFMA half, lane l's 16 bytes at
+// 16 l, so that a wave's load of a fragment is one contiguous KiB (from limb rows
+// it touches 16 rows, 64 separate pieces).
+__device__ inline size_t frag_pos(int K, int m, int l, int q) {
+  const int t = q & 3;
+  return ((((size_t)(m >> 2) * (K >> 7) + (q >> 4)) * 2 + (t >> 1)) * 64 + 4 * (m & 3) + l +
+          16 * ((q >> 2) & 3)) * 16 + 8 * (t & 1);
+}
+
 // Transform (x * pre_scale, rmsnorm, gamma: rmsnorm_inplace kernels.mojo:474-489,
 // ple_scale_inplace :506-516, rmsnorm_weighted_inplace :598-613), optional
 // fp32 stores by `writer`, quantization and limb stores: limb l of row m goes
 // to dst + (4m + l) * ld_dst + limb position (LIMBS 3: dst + (l * planes + m)
-// * ld_dst).  Returns the row shift s.
+// * ld_dst; FRAG: frag_pos, for k_gemv_rows).  Returns the row shift s.
 // XS: also the row's sum of X, exact (integer partial sums below 2^53 add
 // exactly in double), into *xsum_out for every thread.
-template <int NT, int NG, bool GAM, bool XS = false, int LIMBS = 4>
+template <int NT, int NG, bool GAM, bool XS = false, int LIMBS = 4, bool FRAG = false>
 __device__ inline void row_finish(const RowSrc &r, int K, int m, bool writer,
                                   RowRegs<NT, NG, GAM> &R, int8_t *dst, size_t ld_dst,
                                   float *sh, int *s_out, double *xsum_out = nullptr,
@@ -361,7 +371,8 @@ __device__ inline void row_finish(const RowSrc &r, int K, int m, bool writer,
 #pragma unroll
     for (int l = 0; l < LIMBS; ++l) {
       const size_t row = LIMBS == 4 ? (size_t)(4 * m + l) : (size_t)l * planes + m;
-      *reinterpret_cast<uint2 *>(dst + row * ld_dst + pos) = uint2{lo[l], hi[l]};
+      *reinterpret_cast<uint2 *>(dst + (FRAG ? frag_pos(K, m, l, q) : row * ld_dst + pos)) =
+          uint2{lo[l], hi[l]};
     }
   }
   *s_out = s;
@@ -381,8 +392,8 @@ __device__ inline void row_finish(const RowSrc &r, int K, int m, bool writer,
 }
 
 // One row per block of NT threads, NG groups of 8 values per thread
-// (K <= 8 NG NT).  LIMBS 3: the GEMM's planes.
-template <bool GAM, int NT, int LIMBS = 4, int NG = 2>
+// (K <= 8 NG NT).  LIMBS 3: the GEMM's planes; FRAG: k_gemv_rows' fragments.
+template <bool GAM, int NT, int LIMBS = 4, int NG = 2, bool FRAG = false>
 __global__ __launch_bounds__(NT) void k_quant_rows(RowSrc r, int K, QuantRows q) {
   __shared__ __align__(8) float sh[32];  // also 16 doubles (row sum)
   RowRegs<NT, NG, GAM> R;
@@ -390,7 +401,7 @@ __global__ __launch_bounds__(NT) void k_quant_rows(RowSrc r, int K, QuantRows q)
   row_load<NT, NG, GAM>(r, K, m, R);
   int s;
   double xs;
-  row_finish<NT, NG, GAM, true, LIMBS>(r, K, m, true, R, q.limbs, K, sh, &s, &xs, true,
+  row_finish<NT, NG, GAM, true, LIMBS, FRAG>(r, K, m, true, R, q.limbs, K, sh, &s, &xs, true,
                                        q.plane_rows);
   if (threadIdx.x == 0) {
     q.shift[m] = s;
@@ -398,11 +409,16 @@ __global__ __launch_bounds__(NT) void k_quant_rows(RowSrc r, int K, QuantRows q)
   }
 }
 
+// (whole row groups of four: the fragments of k_gemv_rows)
+static int quant_rows_pad(int M) { return (M + 3) & ~3; }
+
 size_t quant_rows_bytes(int M, int K) {
+  M = quant_rows_pad(M);
   return (size_t)4 * M * K + 64 + (size_t)M * 4 + 64 + (size_t)M * 8;
 }
 
 QuantRows quant_rows_view(void *buf, int M, int K) {
+  M = quant_rows_pad(M);
   QuantRows q{};
   uint8_t *b = static_cast<uint8_t *>(buf);
   q.limbs = reinterpret_cast<int8_t *>(b);
@@ -449,13 +465,14 @@ int launch_quant_rows(const RowSrc &r, int M, int K, const QuantRows &q, hipStre
   MS_CHECK_ARG(M >= 1 && K >= 8 && K % 8 == 0 && K <= kQuantMaxK,
                "quant: row length must be a multiple of 8 in [8, 16384]");
   MS_CHECK_ARG(r.x && r.ld >= K && q.limbs && q.shift && q.xsum, "quant: missing buffers");
-  // many rows of up to 4096 values on 256 threads: more rows per CU, shorter
-  // reductions (a few decode rows keep the 1024 threads per row)
-  if (K <= 16 * 256 && M >= 64) {
+  MS_CHECK_ARG(M <= kGemvMaxM, "quant: four limbs for at most 16 rows");
+  if (M > 4) {
     if (r.gamma)
-      hipLaunchKernelGGL((k_quant_rows<true, 256>), dim3(M), dim3(256), 0, st, r, K, q);
+      hipLaunchKernelGGL((k_quant_rows<true, 1024, 4, 2, true>), dim3(M), dim3(1024), 0, st, r,
+                         K, q);
     else
-      hipLaunchKernelGGL((k_quant_rows<false, 256>), dim3(M), dim3(256), 0, st, r, K, q);
+      hipLaunchKernelGGL((k_quant_rows<false, 1024, 4, 2, true>), dim3(M), dim3(1024), 0, st, r,
+                         K, q);
   } else if (r.gamma) {
     hipLaunchKernelGGL((k_quant_rows<true, 1024>), dim3(M), dim3(1024), 0, st, r, K, q);
   } else {
@@ -1547,9 +1564,260 @@ int launch_argmax_fin(const ArgmaxFin &f, hipStream_t st) {
   return MS_OK;
 }
 
+// ------------------------------------------------------------------------------
+// GEMV of 5 to 16 rows, limbs in global memory (AS_QUANT).
+//
+// A row group of four rows (16 limb rows) is one A tile, C of them per wave;
+// lane j + 16 q of a D fragment then holds the four limb sums of row 4c + q at
+// column j, so limbs are combined in the lane and waves exchange one int64 per
+// output.  The limb rows (up to 64 x K bytes) come from L2 for every block; the
+// weights come from HBM once, all U super-tiles of a wave in flight before the
+// first is used, and the A fragments of a super-tile are loaded while the MFMAs of
+// the one before run.  Unsigned nibbles enter the MFMA, 8 sum(X) is taken off at
+// the end: exact, so the result is that of any other GEMV of the row.
+// Bound by latency and the L2 reads of the limbs.  16 rows of E4B (one super-tile
+// at a time in flight, and limb rows whose fragment loads touched 64 separate
+// pieces, before): Gate|Up 19.4 -> 11.8 us, Down 21.7 -> 11.1; 13 x 2560 x 10240 with
+// its quantization 19.0 -> 12.2 us.  (With limb rows the new loop took 19.1 and
+// 21.5 us: the address unit, not memory, set the time.)
+// ------------------------------------------------------------------------------
+constexpr int kRowsU = 5;  // super-tiles per wave in flight
+
+template <int C, int P, int W, int EPI>
+__global__ __launch_bounds__(64 * W, W == 16 ? 4 : 2) void k_gemv_rows(GemvArgs a) {
+  constexpr int NT = 64 * W, U = kRowsU;
+  constexpr int NO = (EPI == EPI_SWIGLU ? 1 : P) * C * 64;  // outputs of the block
+  constexpr int IT = (NO + NT - 1) / NT;
+  __shared__ int64_t red[W * P * C * 64];
+  __shared__ int32_t row_s[16];
+  __shared__ int64_t row_x[16];
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int K = launder(a.K), M = launder(a.M);
+  const int nseg = launder(a.nseg);
+  const uint8_t *sw0 = launder(a.seg[0].w), *sw1 = launder(a.seg[1].w),
+                *sw2 = launder(a.seg[2].w);
+  const float ss0 = launder(a.seg[0].scale), ss1 = launder(a.seg[1].scale),
+              ss2 = launder(a.seg[2].scale);
+  const int sn0 = launder(a.seg[0].n_cols) >> 4;
+  const int sn1 = nseg > 1 ? launder(a.seg[1].n_cols) >> 4 : 0;
+  const int sn2 = nseg > 2 ? launder(a.seg[2].n_cols) >> 4 : 0;
+  const int sc0 = launder(a.seg[0].out_col0), sc1 = launder(a.seg[1].out_col0),
+            sc2 = launder(a.seg[2].out_col0);
+  const int ldo = launder(a.ldo);
+  float *out = launder(a.out);
+  const float *resid = EPI == EPI_RESID ? launder(a.resid) : nullptr;
+  const int8_t *limbs = launder(a.q.limbs);
+  const int32_t *shift = launder(a.q.shift);
+  const int64_t *xsum = launder(a.q.xsum);
+  const int KG = K / kSuperK, pg = blockIdx.x;
+
+  const uint8_t *wl[P];
+  float wsc[P];
+  int col[P];
+  bool wv[P];
+  __amdgpu_buffer_rsrc_t rw[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    gemv_slot<EPI>(sw0, sw1, sw2, ss0, ss1, ss2, sn0, sn1, sn2, sc0, sc1, sc2, K, P, pg, p,
+                   &wl[p], &wsc[p], &col[p], &wv[p]);
+    rw[p] = buffer_of(launder(wl[p]), K * 8);
+  }
+  // (row groups past M read zeros)
+  const __amdgpu_buffer_rsrc_t ra = buffer_of(limbs, (M + 3) / 4 * 16 * K);
+
+  // what the epilogue needs, before the weights queue up: the thread's output
+  // (slot p, row m, column j) of round it is o = tid + it NT
+  int32_t s_pre = 0;
+  int64_t x_pre = 0;
+  if (tid < M) {
+    s_pre = ldg<int32_t>(shift + tid);
+    x_pre = ldg<long long>(xsum + tid);
+  }
+  float resid_pre[IT];
+  if constexpr (EPI == EPI_RESID) {
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int o = tid + it * NT, p = o / (C * 64), m = 4 * (o / 64 % C) + (o % 64 >> 4);
+      static_assert(P == 1, "residual: one panel");
+      resid_pre[it] =
+          p < P && m < M && wv[0] ? ldg<float>(resid + (size_t)m * ldo + col[0] + (o & 15)) : 0.f;
+    }
+  }
+
+  v4i acc[P][C];
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+#pragma unroll
+    for (int c = 0; c < C; ++c) acc[p][c] = v4i{0, 0, 0, 0};
+  v4i af[2][C][2];
+  auto load_a = [&](int G, v4i(&f)[C][2]) {
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        f[c][h] = __builtin_bit_cast(
+            v4i, __builtin_amdgcn_raw_buffer_load_b128(ra, lane * 16,
+                                                       ((c * KG + G) * 2 + h) * 1024, 0));
+  };
+  // super-tiles wave, wave + W, ..; U of them per batch
+  for (int g0 = wave; g0 < KG; g0 += U * W) {
+    const int nt = min(U, (KG - g0 + W - 1) / W);
+    u32x4 q[U][P];
+    load_a(g0, af[0]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+        // (past the end of K: zeros without a memory access); streaming hint
+        q[u][p] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw[p], lane * 16,
+                                                         (g0 + u * W) * 1024, 2));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (u >= nt) break;
+      if (u + 1 < U && u + 1 < nt) load_a(g0 + (u + 1) * W, af[(u + 1) & 1]);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const uint32_t d0 = q[u][p][2 * h], d1 = q[u][p][2 * h + 1];
+          const v4i b = v4i{nib_u8(d0), nib_u8(d0 >> 4), nib_u8(d1), nib_u8(d1 >> 4)};
+#pragma unroll
+          for (int c = 0; c < C; ++c)
+            acc[p][c] =
+                __builtin_amdgcn_mfma_i32_16x16x64_i8(af[u & 1][c][h], b, acc[p][c], 0, 0, 0);
+        }
+    }
+  }
+  if (tid < 16) {
+    row_s[tid] = s_pre;
+    row_x[tid] = x_pre;
+  }
+#pragma unroll
+  for (int p = 0; p < P; ++p)
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+      red[((wave * P + p) * C + c) * 64 + lane] =
+          (int64_t)acc[p][c][0] + ((int64_t)acc[p][c][1] << 8) + ((int64_t)acc[p][c][2] << 16) +
+          ((int64_t)acc[p][c][3] << 24);
+  __syncthreads();
+  // sum_k X_k (n_k - 8) of row m at slot p, column j, scaled
+  auto value = [&](int p, int o) {
+    const int c = o / 64 % C, m = 4 * c + (o % 64 >> 4);
+    int64_t t = -8 * row_x[m];
+#pragma unroll
+    for (int w = 0; w < W; ++w) t += red[((w * P + p) * C + c) * 64 + o % 64];
+    return (float)((double)t * (double)ldexpf(1.0f, -row_s[m]) * (double)wsc[p]);
+  };
+  float v[IT];
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int o = tid + it * NT, m = 4 * (o / 64 % C) + (o % 64 >> 4), j = o & 15;
+    v[it] = 0.f;
+    if (o >= NO || m >= M) continue;
+    if constexpr (EPI == EPI_SWIGLU) {
+      // swiglu_inplace (kernels.mojo:519-532)
+      const float gt = value(0, o), up = value(1, o);
+      a.sw_out[(size_t)m * a.ldo_sw + col[0] + j] = up * gt * (1.0f / (1.0f + expf(-gt)));
+    } else {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        if (p != o / (C * 64) || !wv[p]) continue;
+        v[it] = value(p, o);
+        const size_t oi = (size_t)m * ldo + col[p] + j;
+        if constexpr (EPI == EPI_ARGMAX) {
+          if (out) out[oi] = v[it];  // logits (optional)
+        } else if constexpr (EPI == EPI_STORE) {
+          out[oi] = v[it];
+        } else if constexpr (EPI == EPI_ACCUMULATE) {
+          out[oi] += v[it];
+        } else {
+          // x = x + proj (gemma4_e4b.mojo:522,538)
+          const float x = resid_pre[it] + v[it];
+          out[oi] = x;
+          if (a.out2) a.out2[oi] = x;
+        }
+      }
+    }
+  }
+  if constexpr (EPI == EPI_ARGMAX) {
+    // the block's first index of the maximum per row
+    float *vals = reinterpret_cast<float *>(red);
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int o = tid + it * NT;
+      if (o < NO) vals[o] = v[it];
+    }
+    __syncthreads();
+    if (tid < M) {
+      float bv = -INFINITY;
+      int bi = 0x7fffffff;
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+        for (int j = 0; j < 16; ++j) {
+          const float x = vals[(p * C + (tid >> 2)) * 64 + (tid & 3) * 16 + j];
+          const int idx = col[p] + j;
+          if (x > bv || (x == bv && idx < bi)) {
+            bv = x;
+            bi = idx;
+          }
+        }
+      a.arg_val[(size_t)blockIdx.x * M + tid] = bv;
+      a.arg_idx[(size_t)blockIdx.x * M + tid] = bi;
+    }
+  }
+}
+
+// 5 to 16 rows from global limbs.
+static int launch_gemv_rows(const GemvArgs &a, long n_panels, hipStream_t st) {
+  const int KG = a.K / kSuperK, epi = a.epi;
+  // panels per block: gate and up; the head's four (its block maxima are laid out
+  // so); two where that leaves two blocks per CU (half the limb reads)
+  bool even = true;
+  for (int i = 0; i < a.nseg; ++i) even &= a.seg[i].n_cols % 32 == 0;
+  const int P = epi == EPI_SWIGLU ? 2 : epi == EPI_ARGMAX ? 4
+                : (epi == EPI_RESID || !even || n_panels < 1024) ? 1 : 2;
+  const long blocks = epi == EPI_SWIGLU ? a.seg[0].n_cols / 16 : n_panels / P;
+  // waves: as few as hold K in one batch each and give every SIMD one
+  int W = 4;
+  while (W < (P == 1 ? 16 : P == 2 ? 8 : 4) && (KG > kRowsU * W || blocks * W < 1024)) W *= 2;
+  GemvArgs b = a;
+  b.P = P;
+  bool ok = false;
+#define MS_ROWS(EP, PP, WW)                                                              \
+  if (!ok && epi == EP && P == PP && W == WW) {                                          \
+    if (a.M <= 8)                                                                        \
+      hipLaunchKernelGGL((k_gemv_rows<2, PP, WW, EP>), dim3(blocks), dim3(64 * WW), 0, st, b); \
+    else                                                                                 \
+      hipLaunchKernelGGL((k_gemv_rows<4, PP, WW, EP>), dim3(blocks), dim3(64 * WW), 0, st, b); \
+    ok = true;                                                                           \
+  }
+  MS_ROWS(EPI_STORE, 1, 4)
+  MS_ROWS(EPI_STORE, 1, 8)
+  MS_ROWS(EPI_STORE, 1, 16)
+  MS_ROWS(EPI_STORE, 2, 4)
+  MS_ROWS(EPI_STORE, 2, 8)
+  MS_ROWS(EPI_ACCUMULATE, 1, 4)
+  MS_ROWS(EPI_ACCUMULATE, 1, 8)
+  MS_ROWS(EPI_ACCUMULATE, 1, 16)
+  MS_ROWS(EPI_ACCUMULATE, 2, 4)
+  MS_ROWS(EPI_ACCUMULATE, 2, 8)
+  MS_ROWS(EPI_RESID, 1, 4)
+  MS_ROWS(EPI_RESID, 1, 8)
+  MS_ROWS(EPI_RESID, 1, 16)
+  MS_ROWS(EPI_SWIGLU, 2, 4)
+  MS_ROWS(EPI_SWIGLU, 2, 8)
+  MS_ROWS(EPI_ARGMAX, 4, 4)
+#undef MS_ROWS
+  MS_CHECK_ARG(ok, "GEMV: unsupported epilogue of quantized rows");
+  MS_HIP_TRY(hipGetLastError());
+  return MS_OK;
+}
+
 size_t gemv_lds_need(const GemvArgs &a) {
-  const int C = a.M <= 4 ? 1 : 4;
-  size_t b = gemv_lds_fixed(a.waves, a.P, C, a.M);
+  size_t b = gemv_lds_fixed(a.waves, a.P, 1, a.M);
   if (a.asrc == AS_ROWS || a.asrc == AS_ATTN || a.asrc == AS_WAVES)
     b += (size_t)4 * a.M * gemv_ldl(a.K);
   else if (a.asrc == AS_WSTREAM)
@@ -1626,10 +1894,14 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
   }
   if (a.epi == EPI_SWIGLU)
     MS_CHECK_ARG(a.seg[0].n_cols == a.seg[1].n_cols, "GEMV: gate/up widths differ");
+  if (a.asrc == AS_QUANT && a.M > 4) {
+    MS_CHECK_ARG(a.q.xsum, "GEMV: row sums missing");
+    return launch_gemv_rows(a, n_panels, st);
+  }
   const long blocks = (a.epi == EPI_SWIGLU) ? a.seg[0].n_cols / 16 : n_panels / a.P;
+  MS_CHECK_ARG(a.M <= 4, "GEMV: more than four rows come from global limbs");
   const size_t shmem = gemv_lds_need(a);
   MS_CHECK_ARG(shmem <= 160 * 1024 - 1024, "GEMV: LDS budget exceeded");
-  const int C = a.M <= 4 ? 1 : 4;
   bool ok = false;
   // Supported (epilogue, panels per block, activation source, waves).
 #define MS_GEMV_L(CC, EP, PP, AS, WW, RR) \
@@ -1638,8 +1910,7 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
   if (!ok && a.epi == EP && a.P == PP && a.asrc == AS && a.waves == WW) {        \
     constexpr int RP = WW > 8 ? 1 : 4;                                            \
     if (a.M == 1) MS_GEMV_L(1, EP, PP, AS, WW, 1);                                \
-    else if (C == 1) MS_GEMV_L(1, EP, PP, AS, WW, RP);                            \
-    else MS_GEMV_L(4, EP, PP, AS, WW, RP);                                        \
+    else MS_GEMV_L(1, EP, PP, AS, WW, RP);                                        \
     ok = true;                                                                    \
   }
   MS_GEMV(EPI_STORE, 1, AS_ROWS, 8)
@@ -1727,7 +1998,6 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
     ok = true;
   }
   if (!ok && a.epi == EPI_RESID && a.P == 1 && a.asrc == AS_QUANT && a.waves == 16) {
-    MS_CHECK_ARG(a.M <= 4, "GEMV: 16 waves over global limbs take at most 4 rows");
     if (a.M == 1) MS_GEMV_L(1, EPI_RESID, 1, AS_QUANT, 16, 1);
     else MS_GEMV_L(1, EPI_RESID, 1, AS_QUANT, 16, 4);
     ok = true;
