@@ -75,6 +75,10 @@ inline size_t attn_ctr_count(int max_seqs, int n_kv) { return (size_t)max_seqs *
 // query heads) merges the chunks into a.out [B][q_dim] (a.ctr: B * n_kv * 2
 // counters, zero between launches).
 int launch_attention_partials(const AttnArgs &a, hipStream_t st, bool merge = false);
+// The partials of a batch, one row of each sequence (RoPE factors from the tables
+// at each position), for launch_merge_quant (q4.h).  attn_batch_ok: shapes taken.
+bool attn_batch_ok(const AttnArgs &a);
+int launch_attention_batch(const AttnArgs &a, hipStream_t st);
 // Two to four rows of one sequence on a linear cache (attn_rows_ok): the
 // chunk scheme of the decode step per row (k_attn_rows), then the chunks
 // merged per row and query head into a.out [T][q_dim].  The partials need

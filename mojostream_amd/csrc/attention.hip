@@ -997,11 +997,13 @@ __global__ __launch_bounds__(256) void k_attn_decode(AttnArgs args) {
 // key, coalesced 16-byte pieces): the scores are its partial dots summed over
 // the key's lanes, then the chunk's softmax numerators (max and sum over its
 // keys), and o = sum_k e^(s_k - m) v_k over groups of keys (V through LDS),
-// stored with (m, l) per query head.  The consumer (the O projection) merges
-// the chunks, so no block waits for another.  Sixteen waves keep every SIMD
+// stored with (m, l) per query head.  The consumer (the O projection, or with
+// several sequences k_attn_rows_merge) merges the chunks, so no block waits for
+// another; MRG: the last block merges.  SEQ: RoPE factors from the tables at each
+// sequence's position.  Sixteen waves keep every SIMD
 // busy and every dependent step short.
 // ------------------------------------------------------------------------------
-template <int HD, int GQ, bool MRG>
+template <int HD, int GQ, bool MRG, bool SEQ = MRG>
 __global__ __launch_bounds__(1024) void k_attn_part(AttnArgs args) {
   extern __shared__ __align__(16) float lds[];
   __shared__ int s_last;
@@ -1081,7 +1083,7 @@ __global__ __launch_bounds__(1024) void k_attn_part(AttnArgs args) {
     const bool on = e < nq;
     qx[u] = ld1(rq, on, q0 + d);
     qy[u] = ld1(rq, on, q0 + rope_partner(p, d));
-    if constexpr (!MRG) {
+    if constexpr (!SEQ) {
       const bool rot = p.apply_rope && d < p.rot;
       const int ri = d < p.half ? d : d - p.half;
       const float cv = ld1(rr, rot, ri);
@@ -1096,7 +1098,7 @@ __global__ __launch_bounds__(1024) void k_attn_part(AttnArgs args) {
   const float ky = ld1(rq, tid < HD, k0 + rope_partner(p, df));
   const float vx = ld1(rq, tid < HD, p.q_dim + p.kv_dim + h * HD + df);
   float kc_ = 1.f, ks_ = 0.f;
-  if constexpr (!MRG) {
+  if constexpr (!SEQ) {
     const bool krot = p.apply_rope && df < p.rot;
     const int kri = df < p.half ? df : df - p.half;
     const float kcv = ld1(rr, krot, kri);
@@ -1118,7 +1120,7 @@ __global__ __launch_bounds__(1024) void k_attn_part(AttnArgs args) {
   const bool fresh_here = fslot < nslots && fslot / CH == c;
   const int kf = fslot - c * CH;  // key of the fresh row in this chunk
   const bool own_fresh = fresh_here && key == kf;
-  if constexpr (MRG) {
+  if constexpr (SEQ) {
     // the RoPE factors of this sequence's position, from the tables
 #pragma unroll
     for (int u = 0; u < QPT; ++u) rope_cs(p, (tid + NT * u) % HD, base, qc[u], qs[u]);
@@ -1571,8 +1573,9 @@ __global__ __launch_bounds__(1024) void k_attn_rows(AttnArgs args) {
 // w_c = e^(m_c - M) and l = sum_c l_c w_c come from wave reductions; chunks
 // past the row's last attended one are dropped by selects, so a stale
 // partial never enters the sum.
+// SEQ: row t is the one row of sequence t (k_attn_part), at its own position.
 constexpr int kMergeBatch = 8;
-template <int HD>
+template <int HD, bool SEQ>
 __global__ __launch_bounds__(128) void k_attn_rows_merge(AttnArgs args) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -1582,7 +1585,7 @@ __global__ __launch_bounds__(128) void k_attn_rows_merge(AttnArgs args) {
   const int cache_len = keep(args.cache_len), q_dim = keep(args.q_dim);
   const float *po = args.part + (size_t)t * kDecPartMaxChunks * nhq * (HD + 2);
   const float *pml = po + (size_t)kDecPartMaxChunks * nhq * HD;
-  const int base = aldg_lane<int32_t>(args.pos);
+  const int base = aldg_lane<int32_t>(args.pos + (SEQ ? t : 0));
   const __amdgpu_buffer_rsrc_t rml = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float *>(pml), 0, gc * nhq * 8, 0x00020000);
   const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
@@ -1595,7 +1598,7 @@ __global__ __launch_bounds__(128) void k_attn_rows_merge(AttnArgs args) {
   for (int u = 0; u < kMergeBatch; ++u)
     v[u] = __builtin_bit_cast(
         f32x4, __builtin_amdgcn_raw_buffer_load_b128(ro, (u * nhq + hq) * HD * 4 + od, 0, 0));
-  const int nslots = min(base + t + 1, cache_len);
+  const int nslots = min(base + (SEQ ? 0 : t) + 1, cache_len);
   const int n_act = min((nslots + kDecPartChunk - 1) / kDecPartChunk, gc);
   const bool on = lane < n_act;
   const float M = wave64_max(on ? ml.x : -INFINITY);
@@ -1628,6 +1631,20 @@ __global__ __launch_bounds__(128) void k_attn_rows_merge(AttnArgs args) {
   }
 }
 
+template <bool SEQ>
+static int launch_rows_merge(const AttnArgs &a, int rows, hipStream_t st) {
+  const dim3 grid(a.n_heads, rows);
+  const int nt = a.hd / 4 < 64 ? 64 : a.hd / 4;
+  if (a.hd == 128)
+    hipLaunchKernelGGL((k_attn_rows_merge<128, SEQ>), grid, dim3(nt), 0, st, a);
+  else if (a.hd == 256)
+    hipLaunchKernelGGL((k_attn_rows_merge<256, SEQ>), grid, dim3(nt), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_attn_rows_merge<512, SEQ>), grid, dim3(nt), 0, st, a);
+  MS_HIP_TRY(hipGetLastError());
+  return MS_OK;
+}
+
 bool attn_rows_ok(const AttnArgs &a) {
   const int G = a.n_kv > 0 ? a.n_heads / a.n_kv : 0;
   return a.B == 1 && a.T >= 2 && a.T <= kRowsMax && G >= 1 && G <= 4 && G != 3 &&
@@ -1654,13 +1671,7 @@ int launch_attention_rows(const AttnArgs &a, hipStream_t st) {
   else if (a.hd == 256) hipLaunchKernelGGL((k_attn_rows<256, GQ>), grid, dim3(1024), shmem, st, a2);
   else hipLaunchKernelGGL((k_attn_rows<512, GQ>), grid, dim3(1024), shmem, st, a2);
   MS_HIP_TRY(hipGetLastError());
-  const dim3 mgrid(a.n_heads, a.T);
-  const int mthreads = a.hd / 4 < 64 ? 64 : a.hd / 4;
-  if (a.hd == 128) hipLaunchKernelGGL(k_attn_rows_merge<128>, mgrid, dim3(mthreads), 0, st, a2);
-  else if (a.hd == 256) hipLaunchKernelGGL(k_attn_rows_merge<256>, mgrid, dim3(mthreads), 0, st, a2);
-  else hipLaunchKernelGGL(k_attn_rows_merge<512>, mgrid, dim3(mthreads), 0, st, a2);
-  MS_HIP_TRY(hipGetLastError());
-  return MS_OK;
+  return launch_rows_merge<false>(a2, a.T, st);
 }
 
 int dec_part_chunks(const AttnArgs &a) {
@@ -1695,6 +1706,33 @@ int launch_rope_cur(const AttnArgs &a, hipStream_t st) {
   return MS_OK;
 }
 
+// The merge in a launch of its own from this many chunk blocks on: the last-block
+// protocol makes every block wait for its stores and count itself, which few
+// blocks hide and many do not.  E4B steps, merge in the kernel against separate:
+// 4 sequences of 300 tokens (80 and 80 blocks) 1685 / 1696 us, 8 of 300 (160) 2445 /
+// 2435, 8 of 640 (256 and 320) 2675 / 2571, 16 of 640 (512 and 704) 3462 / 3091
+// (sliding layer 19.3 -> 10.3 + 4.6 us, full 53 -> 26 + 4.6).
+constexpr int kSepMergeBlocks = 160;
+
+bool attn_batch_ok(const AttnArgs &a) { return dec_part_ok(a) && a.n_heads == 4 * a.n_kv; }
+
+int launch_attention_batch(const AttnArgs &a, hipStream_t st) {
+  MS_CHECK_ARG(attn_batch_ok(a), "attention batch: unsupported shape");
+  MS_CHECK_ARG(a.qkv && a.part && a.pos && a.kc && a.vc && a.cos_t && a.sin_t,
+               "attention batch: missing buffers");
+  AttnArgs a2 = a;
+  a2.grid_chunks = dec_part_chunks(a);
+  constexpr int GQ = 4, CH = kDecPartChunk;
+  const dim3 grid(a2.grid_chunks, a.B * a.n_kv);
+  const size_t shmem = (size_t)(CH * a.hd + GQ * a.hd + a.hd + GQ * CH + 8) * 4 + 16384;
+  if (a.hd == 256)
+    hipLaunchKernelGGL((k_attn_part<256, GQ, false, true>), grid, dim3(1024), shmem, st, a2);
+  else
+    hipLaunchKernelGGL((k_attn_part<512, GQ, false, true>), grid, dim3(1024), shmem, st, a2);
+  MS_HIP_TRY(hipGetLastError());
+  return MS_OK;
+}
+
 int launch_attention_partials(const AttnArgs &a, hipStream_t st, bool merge) {
   MS_CHECK_ARG(dec_part_ok(a), "attention partials: unsupported shape");
   MS_CHECK_ARG(a.qkv && a.part && a.pos && a.kc && a.vc &&
@@ -1716,6 +1754,10 @@ int launch_attention_partials(const AttnArgs &a, hipStream_t st, bool merge) {
     constexpr int GQ4 = 4;
     const dim3 grid4(a2.grid_chunks, a.B * a.n_kv);
     const size_t shmem4 = (size_t)(CH * a.hd + GQ4 * a.hd + a.hd + GQ4 * CH + 8) * 4 + 16384;
+    if ((int)(grid4.x * grid4.y) >= kSepMergeBlocks) {
+      if (int rc = launch_attention_batch(a2, st)) return rc;
+      return launch_rows_merge<true>(a2, a.B, st);
+    }
     if (a.hd == 256) hipLaunchKernelGGL((k_attn_part<256, GQ4, true>), grid4, dim3(1024), shmem4, st, a2);
     else hipLaunchKernelGGL((k_attn_part<512, GQ4, true>), grid4, dim3(1024), shmem4, st, a2);
   } else if (merge) {

@@ -441,7 +441,16 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
     }
   }
   // 2. attention (chunks + merge/cache append)
-  bool merged_in_o = false;
+  bool merged_in_o = false, merged_in_quant = false;
+  AttnSrc o_src{};
+  o_src.part = m->attn_part;
+  o_src.pos = m->pos + rc.seq0;
+  o_src.hd = d.head_dim;
+  o_src.n_heads = d.n_heads;
+  o_src.circular = d.cache_kind == MS_CACHE_CIRCULAR;
+  o_src.cache_len = d.cache_len;
+  o_src.clamp = d.clamp_reads;
+  o_src.chunks = dec_part_chunks(attn);
   {
     AttnArgs a = attn;
     // KV bytes read at the current position are counted by bench.py
@@ -457,6 +466,11 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
       }
       if (int rc2 = launch_attention_partials(a, st)) return rc2;
       merged_in_o = true;
+    } else if (rc.T == 1 && attn_batch_ok(a) && merge_quant_ok(o_src, M, d.q_dim)) {
+      // five sequences or more: chunk partials; the O projection's quantization
+      // merges them
+      if (int rc2 = launch_attention_batch(a, st)) return rc2;
+      merged_in_quant = true;
     } else if (rc.T == 1 && dec_part_ok(a)) {
       // one row per sequence (a batch decode step, a one-row forward): the
       // same chunk blocks, merged by the last block of each (sequence, kv
@@ -500,17 +514,13 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
       // the attention chunks merged per head in the O projection's prologue
       a.asrc = AS_ATTN;
       a.waves = 8;
-      a.at.part = m->attn_part;
-      a.at.pos = m->pos + rc.seq0;
-      a.at.hd = d.head_dim;
-      a.at.n_heads = d.n_heads;
-      a.at.circular = d.cache_kind == MS_CACHE_CIRCULAR;
-      a.at.cache_len = d.cache_len;
-      a.at.clamp = d.clamp_reads;
-      AttnArgs pa{};
-      pa.cache_len = d.cache_len;
-      pa.pos_bound = rc.pos_bound;
-      a.at.chunks = dec_part_chunks(pa);
+      a.at = o_src;
+      if (int rc2 = launch_gemv_rec(a, st)) return rc2;
+    } else if (merged_in_quant) {
+      a.asrc = AS_QUANT;
+      a.q = quant_rows_view(m->quant, M, d.q_dim);
+      a.waves = 4;
+      if (int rc2 = launch_merge_quant(o_src, M, d.q_dim, a.q, st)) return rc2;
       if (int rc2 = launch_gemv_rec(a, st)) return rc2;
     } else if (int rc2 = launch_proj_row(m, rc, a, r, 8, 8, st)) {
       return rc2;
@@ -866,10 +876,10 @@ extern "C" int ms_model_create(const ms_model_desc *desc, const ms_layer_desc *l
     const int G = ld.n_heads / ld.n_kv_heads;
     max_part = std::max(max_part, attn_part_floats(d.max_seqs, ld.n_kv_heads, Ly.n_chunks,
                                                    attn_rows, G, ld.head_dim));
-    // a batch-1 decode step's chunk partials, merged in the O projection, or
-    // those of two to four rows of one sequence
-    max_part = std::max(max_part, dec_part_floats(std::min(d.max_rows, 4), ld.n_heads,
-                                                  ld.head_dim));
+    // a decode step's chunk partials of every sequence, or those of two to four
+    // rows of one
+    max_part = std::max(max_part, dec_part_floats(std::max(std::min(d.max_rows, 4), d.max_seqs),
+                                                  ld.n_heads, ld.head_dim));
     m->qkv_max = std::max(m->qkv_max, ncols_qkv);
     m->q_max = std::max(m->q_max, ld.q_dim);
     m->quant_k = std::max(m->quant_k, std::max(std::max(d.hidden, d.ffn), ld.q_dim));

@@ -176,6 +176,10 @@ QuantRows quant_rows_view(void *buf, int M, int K);
 // rows.  The view fits in a buffer of quant_rows_bytes(Mp, K).
 QuantRows quant_rows3_view(void *buf, int Mp, int K);
 int launch_quant_rows3(const RowSrc &r, int M, int K, const QuantRows &q, hipStream_t st);
+// 5 to 16 rows merged from the chunk partials of a decode batch (at.pos: the rows'
+// positions) and quantized, as attention, merge and launch_quant_rows would.
+bool merge_quant_ok(const AttnSrc &at, int M, int K);
+int launch_merge_quant(const AttnSrc &at, int M, int K, const QuantRows &q, hipStream_t st);
 int pack_device(uint8_t *dst, const uint8_t *src, int K, int N, hipStream_t st);
 int launch_argmax_fin(const ArgmaxFin &f, hipStream_t st);
 int launch_gemm(const GemmArgs &g, hipStream_t st);
