@@ -79,6 +79,7 @@ int launch_attention_partials(const AttnArgs &a, hipStream_t st, bool merge = fa
 // at each position), for launch_merge_quant (q4.h).  attn_batch_ok: shapes taken.
 bool attn_batch_ok(const AttnArgs &a);
 int launch_attention_batch(const AttnArgs &a, hipStream_t st);
+int launch_attention_batch_merged(const AttnArgs &a, hipStream_t st);
 // Two to four rows of one sequence on a linear cache (attn_rows_ok): the
 // chunk scheme of the decode step per row (k_attn_rows), then the chunks
 // merged per row and query head into a.out [T][q_dim].  The partials need

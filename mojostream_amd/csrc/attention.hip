@@ -988,7 +988,7 @@ __global__ __launch_bounds__(256) void k_attn_decode(AttnArgs args) {
 // ------------------------------------------------------------------------------
 // k_attn_part: the decode attention of one row per sequence without the merge.
 // Block (c, b x h), 1024 threads: cache slots 32c..32c+31 of sequence b, kv
-// head h, for its G <= 4 query heads.  The chunk's cached rows, q, the fresh
+// head h, for its G <= GQ query heads (five of eight in the 14B class).  The chunk's cached rows, q, the fresh
 // k, v and the RoPE factors prepared for the position are loaded before the
 // position arrives (branch-free range-checked loads; the host launches only
 // the chunks below its bound on the position); rows past the attended ones
@@ -1003,6 +1003,12 @@ __global__ __launch_bounds__(256) void k_attn_decode(AttnArgs args) {
 // sequence's position.  Sixteen waves keep every SIMD
 // busy and every dependent step short.
 // ------------------------------------------------------------------------------
+constexpr int part_ml(int gq) { return gq < 4 ? 4 : gq; }
+// LDS: sv, sq, sf, ss, sm, sl, so (16 KB at every head dim)
+constexpr size_t part_lds(int hd, int gq) {
+  return (size_t)(kDecPartChunk * hd + gq * hd + hd + gq * kDecPartChunk + 2 * part_ml(gq)) * 4 +
+         16384;
+}
 template <int HD, int GQ, bool MRG, bool SEQ = MRG>
 __global__ __launch_bounds__(1024) void k_attn_part(AttnArgs args) {
   extern __shared__ __align__(16) float lds[];
@@ -1018,7 +1024,7 @@ __global__ __launch_bounds__(1024) void k_attn_part(AttnArgs args) {
   constexpr int NU = GQ * H4;                   // P.V float4 units (head, dims)
   constexpr int NKG = NT / NU;                  // key groups of the P.V sums
   constexpr int KPG = CH / NKG;                 // keys per group
-  static_assert(NF >= 1 && NKG >= 1 && CH % NKG == 0, "head dim 256 or 512");
+  static_assert(NF >= 1 && NKG >= 1 && CH % NKG == 0, "head dim 128, 256 or 512");
   constexpr uint32_t kOut = 0x80000000u;
   const AttnP p = load_params(args);
   const int tid = threadIdx.x;
@@ -1040,8 +1046,8 @@ __global__ __launch_bounds__(1024) void k_attn_part(AttnArgs args) {
   float *sf = sq + GQ * HD;      // [HD] fresh key, rotated
   float *ss = sf + HD;           // [GQ][CH] scores -> numerators
   float *sm = ss + GQ * CH;      // [GQ]
-  float *sl = sm + 4;            // [GQ]
-  float4 *so = reinterpret_cast<float4 *>(sl + 4);  // [NKG][NU] partial o
+  float *sl = sm + part_ml(GQ);  // [GQ]
+  float4 *so = reinterpret_cast<float4 *>(sl + part_ml(GQ));  // [NKG][NU] partial o
   const size_t cbase = (size_t)b * p.cache_seq_stride;
   const float *qrow = p.qkv + (size_t)b * p.ld;
 
@@ -1714,7 +1720,13 @@ int launch_rope_cur(const AttnArgs &a, hipStream_t st) {
 // (sliding layer 19.3 -> 10.3 + 4.6 us, full 53 -> 26 + 4.6).
 constexpr int kSepMergeBlocks = 160;
 
-bool attn_batch_ok(const AttnArgs &a) { return dec_part_ok(a) && a.n_heads == 4 * a.n_kv; }
+bool attn_batch_ok(const AttnArgs &a) {
+  const int G = a.n_kv > 0 ? a.n_heads / a.n_kv : 0;
+  return a.T == 1 && G >= 1 && a.n_heads % a.n_kv == 0 &&
+         (a.hd == 128 ? G <= 8 : (a.hd == 256 || a.hd == 512) && G <= 4) && a.rot % 2 == 0 &&
+         a.rot <= a.hd && a.ld >= a.q_dim + 2 * a.kv_dim &&
+         dec_part_chunks(a) <= kDecPartMaxChunks;
+}
 
 int launch_attention_batch(const AttnArgs &a, hipStream_t st) {
   MS_CHECK_ARG(attn_batch_ok(a), "attention batch: unsupported shape");
@@ -1722,15 +1734,30 @@ int launch_attention_batch(const AttnArgs &a, hipStream_t st) {
                "attention batch: missing buffers");
   AttnArgs a2 = a;
   a2.grid_chunks = dec_part_chunks(a);
-  constexpr int GQ = 4, CH = kDecPartChunk;
   const dim3 grid(a2.grid_chunks, a.B * a.n_kv);
-  const size_t shmem = (size_t)(CH * a.hd + GQ * a.hd + a.hd + GQ * CH + 8) * 4 + 16384;
-  if (a.hd == 256)
-    hipLaunchKernelGGL((k_attn_part<256, GQ, false, true>), grid, dim3(1024), shmem, st, a2);
-  else
-    hipLaunchKernelGGL((k_attn_part<512, GQ, false, true>), grid, dim3(1024), shmem, st, a2);
+#define MS_BATCH(HD, GQ)                                                                     \
+  hipLaunchKernelGGL((k_attn_part<HD, GQ, false, true>), grid, dim3(1024), part_lds(HD, GQ), \
+                     st, a2)
+  if (a.hd == 128 && a.n_heads > 4 * a.n_kv) MS_BATCH(128, 8);
+  else if (a.hd == 128) MS_BATCH(128, 4);
+  else if (a.hd == 256) MS_BATCH(256, 4);
+  else MS_BATCH(512, 4);
+#undef MS_BATCH
   MS_HIP_TRY(hipGetLastError());
   return MS_OK;
+}
+
+// The same merged into a.out by a second launch.  14B class (five query heads of
+// 128 per kv head), one layer, against
+// k_attn_decode's 16-key chunks of 256 threads: 16 sequences of 640 tokens 31 (and 12
+// for the merge in O's quantization) against 215 us, one of 1400 7.5 + 4.6 against
+// 26.6; a step of four layers and the head 1871 -> 853 us and 471 -> 411.
+int launch_attention_batch_merged(const AttnArgs &a, hipStream_t st) {
+  MS_CHECK_ARG(a.out, "attention batch: missing output");
+  if (int rc = launch_attention_batch(a, st)) return rc;
+  AttnArgs a2 = a;
+  a2.grid_chunks = dec_part_chunks(a);
+  return launch_rows_merge<true>(a2, a.B, st);
 }
 
 int launch_attention_partials(const AttnArgs &a, hipStream_t st, bool merge) {
@@ -1745,18 +1772,15 @@ int launch_attention_partials(const AttnArgs &a, hipStream_t st, bool merge) {
   const int G = a.n_heads / a.n_kv;
   const int ns = G > GQ ? G / GQ : 1;
   const dim3 grid(a2.grid_chunks, a.B * a.n_kv * ns);
-  constexpr int CH = kDecPartChunk;
-  // sv, sq, sf, ss, sm / sl (4 + 4 floats), so (16 KB at every head dim)
-  const size_t shmem = (size_t)(CH * a.hd + GQ * a.hd + a.hd + GQ * CH + 8) * 4 + 16384;
+  const size_t shmem = part_lds(a.hd, GQ);
   if (merge && G == 4) {
     // the merging kernel on all four query heads of a kv head per block (half
     // the blocks, each K/V row loaded once): batch 4 2,429 -> 2,436 tok/s
     constexpr int GQ4 = 4;
     const dim3 grid4(a2.grid_chunks, a.B * a.n_kv);
-    const size_t shmem4 = (size_t)(CH * a.hd + GQ4 * a.hd + a.hd + GQ4 * CH + 8) * 4 + 16384;
+    const size_t shmem4 = part_lds(a.hd, GQ4);
     if ((int)(grid4.x * grid4.y) >= kSepMergeBlocks) {
-      if (int rc = launch_attention_batch(a2, st)) return rc;
-      return launch_rows_merge<true>(a2, a.B, st);
+      return launch_attention_batch_merged(a, st);
     }
     if (a.hd == 256) hipLaunchKernelGGL((k_attn_part<256, GQ4, true>), grid4, dim3(1024), shmem4, st, a2);
     else hipLaunchKernelGGL((k_attn_part<512, GQ4, true>), grid4, dim3(1024), shmem4, st, a2);

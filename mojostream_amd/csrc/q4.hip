@@ -1578,7 +1578,7 @@ int launch_argmax_fin(const ArgmaxFin &f, hipStream_t st) {
 // merge and the quantization apart (a step of 16 sequences 3091 -> 3008 us, of six
 // 2371 -> 2233).
 // ------------------------------------------------------------------------------
-constexpr int kMergeHeads = 32;
+constexpr int kMergeHeads = 48;
 template <int HD>
 __global__ __launch_bounds__(1024) void k_merge_quant(AttnSrc at, int K, QuantRows q) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -1674,7 +1674,7 @@ __global__ __launch_bounds__(1024) void k_merge_quant(AttnSrc at, int K, QuantRo
 }
 
 bool merge_quant_ok(const AttnSrc &at, int M, int K) {
-  return M > 4 && M <= kGemvMaxM && (at.hd == 256 || at.hd == 512) &&
+  return M > 4 && M <= kGemvMaxM && (at.hd == 128 || at.hd == 256 || at.hd == 512) &&
          at.n_heads <= kMergeHeads && K == at.n_heads * at.hd && K <= 8192;
 }
 
@@ -1683,7 +1683,9 @@ int launch_merge_quant(const AttnSrc &at, int M, int K, const QuantRows &q, hipS
                    at.chunks <= kDecPartMaxChunks && at.cache_len > 0,
                "merge and quantize: unsupported shape");
   MS_CHECK_ARG(q.limbs && q.shift && q.xsum, "merge and quantize: missing buffers");
-  if (at.hd == 256)
+  if (at.hd == 128)
+    hipLaunchKernelGGL(k_merge_quant<128>, dim3(M), dim3(1024), 0, st, at, K, q);
+  else if (at.hd == 256)
     hipLaunchKernelGGL(k_merge_quant<256>, dim3(M), dim3(1024), 0, st, at, K, q);
   else
     hipLaunchKernelGGL(k_merge_quant<512>, dim3(M), dim3(1024), 0, st, at, K, q);
