@@ -28,7 +28,7 @@ enum GemvEpilogue {
 // are combined in int64 and scaled by 2^-s and the tensor scale once per output.
 enum GemvASource {
   AS_ROWS = 0,   // prologue: every block quantizes the fp32 rows into LDS
-  AS_QUANT = 1,  // limbs prepared in global memory by launch_quant_rows
+  AS_QUANT = 1,  // limbs prepared in global memory by launch_quant_rows (k_gemv_rows)
   AS_ATTN = 2,   // one row: the attention chunks of k_attn_part, merged per
                  // query head by the wave that owns the head's K range
   AS_WAVES = 3,  // one to four rows: each wave quantizes its own contiguous
@@ -77,12 +77,9 @@ struct RowSrc {
   float *x_out;        // copy of x [M][K] (same writer) or null
 };
 
-// Quantized rows in global memory: limb l of row m at
-// limbs[(4m + l) * K + limb position of k] (MFMA fragment order per 128-row
-// super-tile), shift[m] = s; more than four rows: whole MFMA fragments (frag_pos
-// in q4.hip).  The GEMM's operand (launch_quant_rows3) has
-// three limbs in planes: limb l of row m at limbs[(l * plane_rows + m) * K +
-// limb position of k].
+// Quantized rows in global memory, whole MFMA fragments (frag_pos in q4.hip),
+// shift[m] = s.  The GEMM's operand (launch_quant_rows3) has three limbs in
+// planes: limb l of row m at limbs[(l * plane_rows + m) * K + limb position of k].
 struct QuantRows {
   int8_t *limbs;
   int32_t *shift;

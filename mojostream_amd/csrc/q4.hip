@@ -392,8 +392,8 @@ __device__ inline void row_finish(const RowSrc &r, int K, int m, bool writer,
 }
 
 // One row per block of NT threads, NG groups of 8 values per thread
-// (K <= 8 NG NT).  LIMBS 3: the GEMM's planes; FRAG: k_gemv_rows' fragments.
-template <bool GAM, int NT, int LIMBS = 4, int NG = 2, bool FRAG = false>
+// (K <= 8 NG NT).  LIMBS 4: k_gemv_rows' fragments; 3: the GEMM's planes.
+template <bool GAM, int NT, int LIMBS, int NG = 2>
 __global__ __launch_bounds__(NT) void k_quant_rows(RowSrc r, int K, QuantRows q) {
   __shared__ __align__(8) float sh[32];  // also 16 doubles (row sum)
   RowRegs<NT, NG, GAM> R;
@@ -401,7 +401,7 @@ __global__ __launch_bounds__(NT) void k_quant_rows(RowSrc r, int K, QuantRows q)
   row_load<NT, NG, GAM>(r, K, m, R);
   int s;
   double xs;
-  row_finish<NT, NG, GAM, true, LIMBS, FRAG>(r, K, m, true, R, q.limbs, K, sh, &s, &xs, true,
+  row_finish<NT, NG, GAM, true, LIMBS, LIMBS == 4>(r, K, m, true, R, q.limbs, K, sh, &s, &xs, true,
                                        q.plane_rows);
   if (threadIdx.x == 0) {
     q.shift[m] = s;
@@ -466,21 +466,12 @@ int launch_quant_rows(const RowSrc &r, int M, int K, const QuantRows &q, hipStre
                "quant: row length must be a multiple of 8 in [8, 16384]");
   MS_CHECK_ARG(r.x && r.ld >= K && q.limbs && q.shift && q.xsum, "quant: missing buffers");
   MS_CHECK_ARG(M <= kGemvMaxM, "quant: four limbs for at most 16 rows");
-  if (M > 4) {
-    if (K <= 16 * 256 && !r.gamma)
-      hipLaunchKernelGGL((k_quant_rows<false, 256, 4, 2, true>), dim3(M), dim3(256), 0, st, r, K,
-                         q);
-    else if (r.gamma)
-      hipLaunchKernelGGL((k_quant_rows<true, 1024, 4, 2, true>), dim3(M), dim3(1024), 0, st, r,
-                         K, q);
-    else
-      hipLaunchKernelGGL((k_quant_rows<false, 1024, 4, 2, true>), dim3(M), dim3(1024), 0, st, r,
-                         K, q);
-  } else if (r.gamma) {
-    hipLaunchKernelGGL((k_quant_rows<true, 1024>), dim3(M), dim3(1024), 0, st, r, K, q);
-  } else {
-    hipLaunchKernelGGL((k_quant_rows<false, 1024>), dim3(M), dim3(1024), 0, st, r, K, q);
-  }
+  if (K <= 16 * 256 && M > 4 && !r.gamma)
+    hipLaunchKernelGGL((k_quant_rows<false, 256, 4>), dim3(M), dim3(256), 0, st, r, K, q);
+  else if (r.gamma)
+    hipLaunchKernelGGL((k_quant_rows<true, 1024, 4>), dim3(M), dim3(1024), 0, st, r, K, q);
+  else
+    hipLaunchKernelGGL((k_quant_rows<false, 1024, 4>), dim3(M), dim3(1024), 0, st, r, K, q);
   MS_HIP_TRY(hipGetLastError());
   return MS_OK;
 }
@@ -525,19 +516,12 @@ __device__ inline void gemv_slot(const uint8_t *w0, const uint8_t *w1, const uin
 // lane j + 16*(i/4), element i%4).
 __device__ inline int dfrag(int i, int j) { return (j + 16 * (i >> 2)) * 4 + (i & 3); }
 
-// Super-tiles each wave keeps in flight per batch: A fragments of a global-A
-// GEMV live in registers next to the weights, so it holds fewer.  Ten per
-// wave lets the decode shapes (E4B gate|up: 5 per panel at W = 4) finish
+// Super-tiles each wave keeps in flight per batch.  Ten per wave lets the
+// decode shapes (E4B gate|up: 5 per panel at W = 4) finish
 // in one batch.
-template <int C, int P, int AS, int W>
+template <int C, int P>
 constexpr int gemv_batch() {
-  // one to four rows from global limbs in 16 waves (the Down projection at
-  // batch 2-4): five super-tiles per wave take K <= 10240 in one batch
-  if (AS == AS_QUANT && C == 1 && P == 1 && W == 16) return 5;
-  // four panels per block from global limbs (the LM head): two super-tiles per
-  // batch (one: 0.2% slower per decode step, three to five: no faster)
-  if (AS == AS_QUANT && C == 1 && P == 4 && W == 4) return 2;
-  constexpr int u = (AS == AS_QUANT ? 4 / C : 10 / C) / P;
+  constexpr int u = 10 / C / P;
   return u < 1 ? 1 : u;
 }
 
@@ -973,7 +957,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
   constexpr bool WS = AS == AS_WSTREAM;
   constexpr int U = AS == AS_ATTN    ? attn_hd(RP) / 128
                     : (AS == AS_WAVES || WS) ? waves_tpw(RP)
-                                     : gemv_batch<C, P, AS, W>();
+                                     : gemv_batch<C, P>();
   // rows a WAVE_K epilogue finishes (AS_ATTN: one)
   constexpr int MR = (AS == AS_WAVES || WS) ? waves_rows(RP) : 1;
   constexpr int NSL = AS == AS_WAVES ? waves_nsl(RP) : 1;
@@ -1002,8 +986,6 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
   float *out2 = (EPI == EPI_RESID) ? launder(a.out2) : nullptr;
   float *sw_out = (EPI == EPI_SWIGLU) ? launder(a.sw_out) : nullptr;
   const int ldo_sw = (EPI == EPI_SWIGLU) ? launder(a.ldo_sw) : 0;
-  float *arg_val = (EPI == EPI_ARGMAX) ? launder(a.arg_val) : nullptr;
-  int32_t *arg_idx = (EPI == EPI_ARGMAX) ? launder(a.arg_idx) : nullptr;
   // the decode attention's RoPE factors (one-row Q|K|V projection)
   constexpr bool PF = AS == AS_WAVES && waves_pf(RP);
   static_assert(!PF || (EPI == EPI_STORE && P == 1 && MR == 1), "AttnPrep: one row, store");
@@ -1023,7 +1005,6 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
     pf_base = ldg<int32_t>(launder(a.pf.pos) + z);
   }
   RowSrc rs{};
-  QuantRows qr{};
   if (AS == AS_ROWS || AS == AS_WAVES || WS) {
     rs.x = launder(a.rows.x);
     rs.ld = launder(a.rows.ld);
@@ -1031,9 +1012,6 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
     rs.norm = launder(a.rows.norm);
     rs.y_out = launder(a.rows.y_out);
     rs.x_out = launder(a.rows.x_out);
-  } else if (AS == AS_QUANT) {
-    qr.limbs = launder(a.q.limbs);
-    qr.shift = launder(a.q.shift);
   }
 
   const int KG = K / kSuperK;
@@ -1065,7 +1043,6 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
         resid_pre[m] = ldg<float>(resid + (size_t)m * ldo + col[p] + j);
   }
   int32_t *red = reinterpret_cast<int32_t *>(lds);
-  float *vals = reinterpret_cast<float *>(lds + gemv_lds_red(W, P, C));
   int32_t *row_s = reinterpret_cast<int32_t *>(lds + gemv_lds_red(W, P, C) + (size_t)P * M * 64);
   int8_t *limbs = reinterpret_cast<int8_t *>(lds + gemv_lds_fixed(W, P, C, M));
   const int ldl = gemv_ldl(K);
@@ -1078,7 +1055,6 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
 
   uint4 q[U][P];
   float pf_cs[2];  // PF: cos, sin at the position (block 0)
-  v4i af[AS == AS_QUANT ? U : 1][C][2];
   float yv[MR][NSL][8];  // AS_WAVES: the wave's y values (for the normalized rows)
   float ys[WS ? U : 1][8];  // AS_WSTREAM: the lane's group of each super-tile
   int ws_s = 0;             // AS_WSTREAM: the lane's row shift
@@ -1110,18 +1086,6 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
         } else if (tile_on(bt, u)) {
           const u32x4 v = ldg_nt<u32x4>(wl[p] + (size_t)Gu * 1024 + lane * 16);
           q[u][p] = uint4{v.x, v.y, v.z, v.w};
-        }
-      }
-      if constexpr (AS == AS_QUANT) {
-#pragma unroll
-        for (int c = 0; c < C; ++c) {
-          af[u][c][0] = v4i{0, 0, 0, 0};
-          af[u][c][1] = v4i{0, 0, 0, 0};
-          if (a_on[c]) {
-            const int8_t *ar = qr.limbs + (size_t)(16 * c + i) * K + Gu * 128 + 32 * g;
-            af[u][c][0] = ldg<v4i>(ar);
-            af[u][c][1] = ldg<v4i>(ar + 16);
-          }
         }
       }
     }
@@ -1195,9 +1159,6 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
       pf_cs[1] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_, ro, 0, 0));
       __builtin_amdgcn_sched_barrier(0);
     }
-  } else {
-    if ((int)threadIdx.x < M) row_s[threadIdx.x] = ldg<int32_t>(qr.shift + threadIdx.x);
-    issue(0);
   }
 
   // Weights enter the MFMA as unsigned nibbles n (one mask per four bytes);
@@ -1255,8 +1216,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
             const v4i b = v4i{nib_u8(d0), nib_u8(d0 >> 4), nib_u8(d1), nib_u8(d1 >> 4)};
 #pragma unroll
             for (int c = 0; c < C; ++c) {
-              const v4i av = (AS == AS_QUANT) ? af[u][c][h] : al[c][h];
-              acc[p][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, b, acc[p][c], 0, 0, 0);
+              acc[p][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[c][h], b, acc[p][c], 0, 0, 0);
             }
           }
         }
@@ -1265,8 +1225,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
         for (int h = 0; h < 2; ++h)
 #pragma unroll
           for (int c = 0; c < C; ++c) {
-            const v4i av = (AS == AS_QUANT) ? af[u][c][h] : al[c][h];
-            accz[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, kMinus8, accz[c], 0, 0, 0);
+            accz[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[c][h], kMinus8, accz[c], 0, 0, 0);
           }
       }
     }
@@ -1437,37 +1396,6 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
       const float gt = value(0, m, j), up = value(1, m, j);
       const float y = up * gt * (1.0f / (1.0f + expf(-gt)));
       sw_out[(size_t)m * ldo_sw + col[0] + j] = y;
-    }
-  } else if constexpr (EPI == EPI_ARGMAX) {
-#pragma unroll
-    for (int p = 0; p < P; ++p)
-      for (int o = threadIdx.x; o < M * 16; o += NT) vals[p * M * 16 + o] = value(p, o >> 4, o & 15);
-    __syncthreads();
-    // logits (optional) and the block's first index of the maximum per row
-    if (out) {
-#pragma unroll
-      for (int p = 0; p < P; ++p)
-        for (int o = threadIdx.x; o < M * 16; o += NT) {
-          const int m = o >> 4, j = o & 15;
-          out[(size_t)m * ldo + col[p] + j] = vals[p * M * 16 + o];
-        }
-    }
-    if ((int)threadIdx.x < M) {
-      const int m = threadIdx.x;
-      float bv = -INFINITY;
-      int bi = 0x7fffffff;
-#pragma unroll
-      for (int p = 0; p < P; ++p)
-        for (int j = 0; j < 16; ++j) {
-          const float v = vals[(p * M + m) * 16 + j];
-          const int idx = col[p] + j;
-          if (v > bv || (v == bv && idx < bi)) {
-            bv = v;
-            bi = idx;
-          }
-        }
-      arg_val[(size_t)blockIdx.x * M + m] = bv;
-      arg_idx[(size_t)blockIdx.x * M + m] = bi;
     }
   }
 }
@@ -1694,7 +1622,7 @@ int launch_merge_quant(const AttnSrc &at, int M, int K, const QuantRows &q, hipS
 }
 
 // ------------------------------------------------------------------------------
-// GEMV of 5 to 16 rows, limbs in global memory (AS_QUANT).
+// GEMV of up to 16 rows, limbs in global memory (AS_QUANT).
 //
 // A row group of four rows (16 limb rows) is one A tile, C of them per wave;
 // lane j + 16 q of a D fragment then holds the four limb sums of row 4c + q at
@@ -1752,8 +1680,9 @@ __global__ __launch_bounds__(64 * W, W == 16 ? 4 : 2) void k_gemv_rows(GemvArgs 
                    &wl[p], &wsc[p], &col[p], &wv[p]);
     rw[p] = buffer_of(launder(wl[p]), K * 8);
   }
-  // (row groups past M read zeros)
+  // (row groups past M, and of a single group the limb rows past it, read zeros)
   const __amdgpu_buffer_rsrc_t ra = buffer_of(limbs, (M + 3) / 4 * 16 * K);
+  const uint32_t ao = C > 1 || (lane & 15) < 4 * M ? lane * 16 : 0x80000000u;
 
   // what the epilogue needs, before the weights queue up: the thread's output
   // (slot p, row m, column j) of round it is o = tid + it NT
@@ -1786,7 +1715,7 @@ __global__ __launch_bounds__(64 * W, W == 16 ? 4 : 2) void k_gemv_rows(GemvArgs 
 #pragma unroll
       for (int h = 0; h < 2; ++h)
         f[c][h] = __builtin_bit_cast(
-            v4i, __builtin_amdgcn_raw_buffer_load_b128(ra, lane * 16,
+            v4i, __builtin_amdgcn_raw_buffer_load_b128(ra, ao,
                                                        ((c * KG + G) * 2 + h) * 1024, 0));
   };
   // super-tiles wave, wave + W, ..; U of them per batch
@@ -1899,7 +1828,6 @@ __global__ __launch_bounds__(64 * W, W == 16 ? 4 : 2) void k_gemv_rows(GemvArgs 
   }
 }
 
-// 5 to 16 rows from global limbs.
 static int launch_gemv_rows(const GemvArgs &a, long n_panels, hipStream_t st) {
   const int KG = a.K / kSuperK, epi = a.epi;
   // panels per block: gate and up; the head's four (its block maxima are laid out
@@ -1917,7 +1845,9 @@ static int launch_gemv_rows(const GemvArgs &a, long n_panels, hipStream_t st) {
   bool ok = false;
 #define MS_ROWS(EP, PP, WW)                                                              \
   if (!ok && epi == EP && P == PP && W == WW) {                                          \
-    if (a.M <= 8)                                                                        \
+    if (a.M <= 4)                                                                        \
+      hipLaunchKernelGGL((k_gemv_rows<1, PP, WW, EP>), dim3(blocks), dim3(64 * WW), 0, st, b); \
+    else if (a.M <= 8)                                                                   \
       hipLaunchKernelGGL((k_gemv_rows<2, PP, WW, EP>), dim3(blocks), dim3(64 * WW), 0, st, b); \
     else                                                                                 \
       hipLaunchKernelGGL((k_gemv_rows<4, PP, WW, EP>), dim3(blocks), dim3(64 * WW), 0, st, b); \
@@ -2010,7 +1940,7 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
                      a.at.chunks <= kDecPartMaxChunks && a.at.cache_len > 0,
                  "GEMV: attention source: one head of 128/256/512 per wave, K = heads * hd");
   } else {
-    MS_CHECK_ARG(a.q.limbs && a.q.shift, "GEMV: quantized rows missing");
+    MS_CHECK_ARG(a.q.limbs && a.q.shift && a.q.xsum, "GEMV: quantized rows missing");
   }
   long n_panels = 0;
   for (int i = 0; i < a.nseg; ++i) {
@@ -2023,10 +1953,7 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
   }
   if (a.epi == EPI_SWIGLU)
     MS_CHECK_ARG(a.seg[0].n_cols == a.seg[1].n_cols, "GEMV: gate/up widths differ");
-  if (a.asrc == AS_QUANT && a.M > 4) {
-    MS_CHECK_ARG(a.q.xsum, "GEMV: row sums missing");
-    return launch_gemv_rows(a, n_panels, st);
-  }
+  if (a.asrc == AS_QUANT) return launch_gemv_rows(a, n_panels, st);
   const long blocks = (a.epi == EPI_SWIGLU) ? a.seg[0].n_cols / 16 : n_panels / a.P;
   MS_CHECK_ARG(a.M <= 4, "GEMV: more than four rows come from global limbs");
   const size_t shmem = gemv_lds_need(a);
@@ -2043,14 +1970,9 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
     ok = true;                                                                    \
   }
   MS_GEMV(EPI_STORE, 1, AS_ROWS, 8)
-  MS_GEMV(EPI_STORE, 1, AS_QUANT, 4)
-  MS_GEMV(EPI_STORE, 4, AS_QUANT, 4)
-  MS_GEMV(EPI_ACCUMULATE, 1, AS_QUANT, 4)
-  MS_GEMV(EPI_ACCUMULATE, 4, AS_QUANT, 4)
   MS_GEMV(EPI_RESID, 1, AS_ROWS, 4)
   MS_GEMV(EPI_RESID, 1, AS_ROWS, 8)
   MS_GEMV(EPI_RESID, 1, AS_ROWS, 16)
-  MS_GEMV(EPI_RESID, 1, AS_QUANT, 4)
   if (!ok && a.asrc == AS_WAVES) {
     // RP = 10 * row bound + super-tiles per wave; one row has instantiations
     // of its own (fewer registers)
@@ -2126,15 +2048,8 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
     else MS_GEMV_L(1, EPI_RESID, 1, AS_ATTN, 8, 416);
     ok = true;
   }
-  if (!ok && a.epi == EPI_RESID && a.P == 1 && a.asrc == AS_QUANT && a.waves == 16) {
-    if (a.M == 1) MS_GEMV_L(1, EPI_RESID, 1, AS_QUANT, 16, 1);
-    else MS_GEMV_L(1, EPI_RESID, 1, AS_QUANT, 16, 4);
-    ok = true;
-  }
   MS_GEMV(EPI_SWIGLU, 2, AS_ROWS, 8)
   MS_GEMV(EPI_SWIGLU, 2, AS_ROWS, 4)
-  MS_GEMV(EPI_SWIGLU, 2, AS_QUANT, 4)
-  MS_GEMV(EPI_ARGMAX, 4, AS_QUANT, 4)
 #undef MS_GEMV
 #undef MS_GEMV_L
   MS_CHECK_ARG(ok, "GEMV: unsupported (epilogue, P, waves, activation source) combination");
