@@ -476,9 +476,11 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
       // same chunk blocks, merged by the last block of each (sequence, kv
       // head, head pair), the RoPE factors from the tables at each position
       if (int rc2 = launch_attention_partials(a, st, true)) return rc2;
-    } else if (rc.T == 1 && attn_batch_ok(a) && dec_part_chunks(a) > 1) {
-      // other one-row shapes: chunk partials and their merge (a single chunk takes
-      // one launch below: demo model, one row at position 0 758 against 846 us)
+    } else if (rc.T == 1 && attn_batch_ok(a) && dec_part_chunks(a) > 2) {
+      // other one-row shapes: chunk partials and their merge (below 64 positions,
+      // the first bucket of a captured step, one launch is faster while a single
+      // chunk is attended: demo model, one row at position 0 758 against 846 us, at
+      // 60 872 against 843, at 200 907 against 854)
       if (int rc2 = launch_attention_batch_merged(a, st)) return rc2;
     } else if (attn_rows_ok(a)) {
       // two to four rows of one sequence: chunk partials per row, merged
