@@ -1433,16 +1433,25 @@ __global__ __launch_bounds__(1024) void k_argmax_fin(ArgmaxFin f) {
       bv[r] = -INFINITY;
       bi[r] = 0x7fffffff;
     }
-    for (int b = threadIdx.x; b < nb; b += 1024)
+    // four blocks a thread in flight (a head of 262144 ids has 4096)
+    for (int b0 = threadIdx.x; b0 < nb; b0 += 4 * 1024)
 #pragma unroll
       for (int r = 0; r < kFinRows; ++r) {
         if (m0 + r >= f.M) break;
-        const float v = f.arg_val[(size_t)b * f.M + m0 + r];
-        const int idx = f.arg_idx[(size_t)b * f.M + m0 + r];
-        if (v > bv[r] || (v == bv[r] && idx < bi[r])) {
-          bv[r] = v;
-          bi[r] = idx;
+        float v[4];
+        int idx[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const size_t o = (size_t)min(b0 + 1024 * i, nb - 1) * f.M + m0 + r;
+          v[i] = ldg<float>(f.arg_val + o);
+          idx[i] = ldg<int32_t>(f.arg_idx + o);
         }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (v[i] > bv[r] || (v[i] == bv[r] && idx[i] < bi[r])) {
+            bv[r] = v[i];
+            bi[r] = idx[i];
+          }
       }
 #pragma unroll
     for (int r = 0; r < kFinRows; ++r) {
@@ -1638,11 +1647,14 @@ int launch_merge_quant(const AttnSrc &at, int M, int K, const QuantRows &q, hipS
 // its quantization 19.0 -> 12.2 us.  (With limb rows the new loop took 19.1 and
 // 21.5 us: the address unit, not memory, set the time.)
 // ------------------------------------------------------------------------------
-constexpr int kRowsU = 5;  // super-tiles per wave in flight
+// Super-tiles per wave in flight.  The head at one to four rows is bound by HBM with
+// its thousands of blocks: two leave more of them resident (one row 55.3 against 57.8
+// us with five).
+constexpr int rows_u(int c, int p) { return c == 1 && p == 4 ? 2 : 5; }
 
 template <int C, int P, int W, int EPI>
 __global__ __launch_bounds__(64 * W, W == 16 ? 4 : 2) void k_gemv_rows(GemvArgs a) {
-  constexpr int NT = 64 * W, U = kRowsU;
+  constexpr int NT = 64 * W, U = rows_u(C, P);
   constexpr int NO = (EPI == EPI_SWIGLU ? 1 : P) * C * 64;  // outputs of the block
   constexpr int IT = (NO + NT - 1) / NT;
   __shared__ int64_t red[W * P * C * 64];
@@ -1839,7 +1851,7 @@ static int launch_gemv_rows(const GemvArgs &a, long n_panels, hipStream_t st) {
   const long blocks = epi == EPI_SWIGLU ? a.seg[0].n_cols / 16 : n_panels / P;
   // waves: as few as hold K in one batch each and give every SIMD one
   int W = 4;
-  while (W < (P == 1 ? 16 : P == 2 ? 8 : 4) && (KG > kRowsU * W || blocks * W < 1024)) W *= 2;
+  while (W < (P == 1 ? 16 : P == 2 ? 8 : 4) && (KG > rows_u(4, P) * W || blocks * W < 1024)) W *= 2;
   GemvArgs b = a;
   b.P = P;
   bool ok = false;
