@@ -526,6 +526,10 @@ int launch_gemm(const GemmArgs &g, hipStream_t st) {
     grid.z = g.ksplit;
     const dim3 cgrid((g.ldo + 255) / 256, g.M);
     hipLaunchKernelGGL((k_gemm<EPI_PART, 1, 4>), grid, dim3(kGNT), gemm_lds(1, 4), st, g);
+    if (g.parts_only) {
+      MS_HIP_TRY(hipGetLastError());
+      return MS_OK;
+    }
     if (g.epi == EPI_STORE)
       hipLaunchKernelGGL(k_gemm_kcombine<EPI_STORE>, cgrid, dim3(256), 0, st, g);
     else if (g.epi == EPI_ACCUMULATE)

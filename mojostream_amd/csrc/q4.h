@@ -75,6 +75,14 @@ struct RowSrc {
   const float *gamma;  // or null
   float *y_out;        // y [M][K] (written once: block 0 or the quant kernel) or null
   float *x_out;        // copy of x [M][K] (same writer) or null
+  // ks > 0: the rows are a split GEMM's, not yet combined (launch_quant_rows3):
+  // x = resid + the scaled sum of its parts, as k_gemm_kcombine forms it
+  int ks;
+  const int64_t *kpart;   // [ks][M][K]
+  const float *kresid;    // [M][K]
+  const int32_t *kshift;  // [M] of that GEMM's operand
+  const int64_t *kxsum;
+  float kscale;
 };
 
 // Quantized rows in global memory, whole MFMA fragments (frag_pos in q4.hip),
@@ -145,6 +153,7 @@ struct GemmArgs {
   // combine kernel adds them and scales (the same value as without the split)
   int ksplit;
   int64_t *kpart;
+  int parts_only;  // leave the combine to the next launch_quant_rows3 (RowSrc::ks)
 };
 
 constexpr int kGemvMaxM = 16;

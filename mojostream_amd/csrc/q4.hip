@@ -234,9 +234,48 @@ struct RowRegs {
 // Issue the loads of row m.  Threads past the end of the row load nothing (a
 // clamped duplicate address would send every idle thread of every block to
 // the same cache line).
-template <int NT, int NG, bool GAM>
-__device__ inline void row_load(const RowSrc &r, int K, int m, RowRegs<NT, NG, GAM> &R) {
+// KP: the row from the parts of a split GEMM of M rows (RowSrc::ks), four parts'
+// loads in flight.
+template <int NT, int NG, bool GAM, bool KP = false>
+__device__ inline void row_load(const RowSrc &r, int K, int m, RowRegs<NT, NG, GAM> &R,
+                                int M = 0) {
   const int nq = K >> 3;
+  if constexpr (KP) {
+    typedef long long i64x2 __attribute__((ext_vector_type(2)));
+    const double z8 = (double)(8 * ldg<long long>(r.kxsum + m));
+    const double sc = (double)ldexpf(1.0f, -ldg<int32_t>(r.kshift + m));
+#pragma unroll
+    for (int gi = 0; gi < NG; ++gi) {
+      const int q = (int)threadIdx.x + gi * NT;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) R.v[gi][e] = 0.f;
+      if (q >= nq) continue;
+      const float *p = r.kresid + (size_t)m * K + 8 * q;
+      const float4 a = ldg<float4>(p), b = ldg<float4>(p + 4);
+      const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      long long t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      for (int z0 = 0; z0 < r.ks; z0 += 4) {
+        i64x2 d[4][4];
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            d[z][e] = ldg<i64x2>(r.kpart + ((size_t)min(z0 + z, r.ks - 1) * M + m) * K + 8 * q +
+                                 2 * e);
+#pragma unroll
+        for (int z = 0; z < 4; ++z)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            t[2 * e] += z0 + z < r.ks ? d[z][e].x : 0;
+            t[2 * e + 1] += z0 + z < r.ks ? d[z][e].y : 0;
+          }
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        R.v[gi][e] = x[e] + (float)(((double)t[e] - z8) * sc * (double)r.kscale);
+    }
+    return;
+  }
 #pragma unroll
   for (int gi = 0; gi < NG; ++gi) {
     const int q = (int)threadIdx.x + gi * NT;
@@ -393,12 +432,12 @@ __device__ inline void row_finish(const RowSrc &r, int K, int m, bool writer,
 
 // One row per block of NT threads, NG groups of 8 values per thread
 // (K <= 8 NG NT).  LIMBS 4: k_gemv_rows' fragments; 3: the GEMM's planes.
-template <bool GAM, int NT, int LIMBS, int NG = 2>
+template <bool GAM, int NT, int LIMBS, int NG = 2, bool KP = false>
 __global__ __launch_bounds__(NT) void k_quant_rows(RowSrc r, int K, QuantRows q) {
   __shared__ __align__(8) float sh[32];  // also 16 doubles (row sum)
   RowRegs<NT, NG, GAM> R;
   const int m = blockIdx.x;
-  row_load<NT, NG, GAM>(r, K, m, R);
+  row_load<NT, NG, GAM, KP>(r, K, m, R, gridDim.x);
   int s;
   double xs;
   row_finish<NT, NG, GAM, true, LIMBS, LIMBS == 4>(r, K, m, true, R, q.limbs, K, sh, &s, &xs, true,
@@ -438,8 +477,22 @@ QuantRows quant_rows3_view(void *buf, int Mp, int K) {
 int launch_quant_rows3(const RowSrc &r, int M, int K, const QuantRows &q, hipStream_t st) {
   MS_CHECK_ARG(M >= 1 && K >= 8 && K % 8 == 0 && K <= kQuantMaxK,
                "quant: row length must be a multiple of 8 in [8, 16384]");
-  MS_CHECK_ARG(r.x && r.ld >= K && q.limbs && q.shift && q.xsum && q.plane_rows >= M,
+  MS_CHECK_ARG((r.ks > 0 || (r.x && r.ld >= K)) && q.limbs && q.shift && q.xsum &&
+                   q.plane_rows >= M,
                "quant: missing buffers");
+  if (r.ks > 0) {
+    MS_CHECK_ARG(r.kpart && r.kresid && r.kshift && r.kxsum && !r.gamma && q.shift != r.kshift,
+                 "quant: split rows: missing buffers");
+    // (the thread counts of rows in memory: a row's norm sums in the same order)
+    if (K <= 16 * 256 && M >= 64)
+      hipLaunchKernelGGL((k_quant_rows<false, 256, 3, 2, true>), dim3(M), dim3(256), 0, st, r, K,
+                         q);
+    else
+      hipLaunchKernelGGL((k_quant_rows<false, 1024, 3, 2, true>), dim3(M), dim3(1024), 0, st, r,
+                         K, q);
+    MS_HIP_TRY(hipGetLastError());
+    return MS_OK;
+  }
   if (K <= 16 * 256 && M >= 64) {
     if (r.gamma)
       hipLaunchKernelGGL((k_quant_rows<true, 256, 3>), dim3(M), dim3(256), 0, st, r, K, q);
