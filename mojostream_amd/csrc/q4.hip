@@ -498,6 +498,10 @@ int launch_quant_rows3(const RowSrc &r, int M, int K, const QuantRows &q, hipStr
       hipLaunchKernelGGL((k_quant_rows<true, 256, 3>), dim3(M), dim3(256), 0, st, r, K, q);
     else
       hipLaunchKernelGGL((k_quant_rows<false, 256, 3>), dim3(M), dim3(256), 0, st, r, K, q);
+  } else if (K <= 24 * 256 && M >= 64 && !r.gamma) {
+    // (the 14B class's rows of 5120: 1024-thread blocks fit two per CU, 1000 rows took
+    // two rounds, 16.8 us against 12.0)
+    hipLaunchKernelGGL((k_quant_rows<false, 256, 3, 3>), dim3(M), dim3(256), 0, st, r, K, q);
   } else if (K <= 40 * 256 && M >= 64 && !r.gamma && !r.norm) {
     // long rows without a norm (the Down input, K = 10240): 256 threads of
     // five groups, so that more rows of a prompt chunk are resident at once
@@ -505,6 +509,10 @@ int launch_quant_rows3(const RowSrc &r, int M, int K, const QuantRows &q, hipStr
     // the maximum and the exact sum of X are reduced, so the limbs, shift
     // and sum equal those of the 1024-thread kernel.
     hipLaunchKernelGGL((k_quant_rows<false, 256, 3, 5>), dim3(M), dim3(256), 0, st, r, K, q);
+  } else if (K <= 56 * 256 && M >= 64 && !r.gamma && !r.norm) {
+    // (the same for the 14B class's Down input, K = 13824: 22.5 us at 1000 rows before,
+    // 18.1 now)
+    hipLaunchKernelGGL((k_quant_rows<false, 256, 3, 7>), dim3(M), dim3(256), 0, st, r, K, q);
   } else if (r.gamma) {
     hipLaunchKernelGGL((k_quant_rows<true, 1024, 3>), dim3(M), dim3(1024), 0, st, r, K, q);
   } else {
