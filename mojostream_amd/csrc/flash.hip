@@ -30,6 +30,10 @@
 //                 softmax needs two lane swaps a tile.
 //  k_flash_merge  log-sum-exp merge of the key splits.
 //
+// Error against 64 bits (relative 2-norm, normal q, k and v, scores up to 0.3 to 3 times
+// sqrt(hd)): 1.0e-7 to 1.3e-6 at 300 to 2048 rows, 1.2e-7 to 1.8e-6 for the fp32 MFMA
+// kernel before it; 0.8e-7 to 3.2e-7 at 17 rows against 0.6e-7 to 4.6e-7.
+//
 // Measured (E4B, 2048 rows; the fp32 MFMA kernel before it): sliding layer 45
 // + 13 (prep) against 135 + 17 us (RoPE and append launches), full layer 190 + 32
 // + 14 (merge) against 515 + 29; 14B class, 1000 rows, one layer: 62 + 16

@@ -86,3 +86,35 @@ def test_sample_odd_values(gpu):
     assert ms.sample(dl, V, 0.7, dh, 0, 1.0, 1) == V - 1
     dl.free()
     dh.free()
+
+
+@pytest.mark.parametrize("V", [3000, 262144])
+def test_sample_flat_tail(gpu, oracle, V):
+    """One id holds nearly all the mass in the middle of the row: draws on it, and
+    draws whose target lies within rounding of many slices of next to none (the
+    head and the tail of the row): the first index whose running sum, slice by
+    slice, reaches the target."""
+    ms = gpu
+    say(f"sample flat tail V={V}")
+    dh = ms.DeviceBuffer.from_array(np.zeros(1, np.int32))
+    v = np.full(V, -6.0, np.float32)
+    v[V // 2] = 18.0 + np.log(V)
+    dl = ms.DeviceBuffer(V * 4)
+    per = (V + 1023) // 1024
+    targets = sorted((oracle.sample_target(s), s) for s in range(400000))
+    for t, seed in targets[:6] + targets[200000:200002] + targets[-6:]:
+        dl.upload(v)
+        gid = ms.sample(dl, V, 1.0, dh, 0, 1.0, seed)
+        p = dl.download(np.float32, V)
+        want, base = V - 1, np.float32(0)
+        for c in range(0, V, per):
+            run = base + np.zeros(1, np.float32)
+            cum = np.cumsum(np.concatenate([run, p[c:c + per]]), dtype=np.float32)[1:]
+            hit = np.flatnonzero(cum >= np.float32(t))
+            if hit.size:
+                want = c + int(hit[0])
+                break
+            base = np.float32(base + np.cumsum(p[c:c + per], dtype=np.float32)[-1])
+        assert gid == want, (t, gid, want)
+    dl.free()
+    dh.free()
