@@ -8,8 +8,8 @@
 // value with a per-row power-of-two scale, so the dot product sum X*(n-8) is
 // exact integer arithmetic; it is scaled by 2^-s and the tensor scale once per
 // output.  For M <= 4 the 4M limb rows share one MFMA, so one MFMA covers
-// 1024 weights.  Prefill rows (M > 16) go through the GEMM in gemm.hip, which
-// uses the same operands and therefore gives the same values.
+// 1024 weights (k_gemv; k_gemv_rows for more rows and for limbs in global
+// memory).  Prefill rows (M > 16) go through the GEMM in gemm.hip on three limbs.
 #include "attention.h"
 #include "devutil.h"
 #include "q4.h"
