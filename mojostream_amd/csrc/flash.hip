@@ -329,8 +329,11 @@ __device__ inline void wait_loads() {
   __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
   asm volatile("" ::: "memory");
 }
+// A barrier behind this wave's LDS reads (lgkmcnt(0), vmcnt free): the loads issued
+// after it, by any wave, refill buffers that the reads before it used.
 __device__ inline void block_sync() {
   asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xC07F);
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }
