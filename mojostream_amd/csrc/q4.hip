@@ -1788,8 +1788,8 @@ __global__ __launch_bounds__(64 * W, W == 16 ? 4 : 2) void k_gemv_rows(GemvArgs 
 #pragma unroll
       for (int h = 0; h < 2; ++h)
         f[c][h] = __builtin_bit_cast(
-            v4i, __builtin_amdgcn_raw_buffer_load_b128(ra, ao,
-                                                       ((c * KG + G) * 2 + h) * 1024, 0));
+            v4i, __builtin_amdgcn_raw_buffer_load_b128(ra, ao + ((c * KG + G) * 2 + h) * 1024,
+                                                       0, 0));
   };
   // super-tiles wave, wave + W, ..; U of them per batch
   for (int g0 = wave; g0 < KG; g0 += U * W) {
@@ -1800,10 +1800,11 @@ __global__ __launch_bounds__(64 * W, W == 16 ? 4 : 2) void k_gemv_rows(GemvArgs 
     for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int p = 0; p < P; ++p)
-        // (past the end of K: zeros without a memory access); streaming hint
+        // (past the end of K: zeros without a memory access, the whole offset in the
+        // operand that the range check covers); streaming hint
         q[u][p] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw[p], lane * 16,
-                                                         (g0 + u * W) * 1024, 2));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw[p], (g0 + u * W) * 1024 + lane * 16,
+                                                         0, 2));
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (u >= nt) break;

@@ -101,3 +101,18 @@ def test_lds_reads_done_at_barriers(source, kernel):
         assert n and max(n) == 0, f"{name}: LDS accesses in flight at its barriers: {n}"
         seen += 1
     assert seen >= 4
+
+
+def test_range_checked_loads_check_the_whole_offset():
+    """The GEMV kernels rely on range-checked loads that return zeros past the end of an
+    operand.  The check need not cover the scalar offset, so it has to be zero."""
+    seen = 0
+    for name, lines in _asm("q4").items():
+        for ln in lines:
+            if not ln.startswith("buffer_load"):
+                continue
+            ops = [o.strip() for o in ln.split(None, 1)[1].split(",")]
+            soff = ops[-1].split()[0]
+            assert soff == "0", f"{name}: {ln}"
+            seen += "k_gemv_rows" in name
+    assert seen > 100
