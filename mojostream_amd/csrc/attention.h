@@ -107,9 +107,7 @@ struct FlashBuf {
   int nkt, n_qt;          // 32-key tiles; tiles of 64 queries per kv head
   int st_tiles, maxs;     // key tiles per split, splits per query tile (1: none)
   int append;             // k_flash_prep appends the rows to the cache
-  _Float16 *q, *k, *v;    // split operands in MFMA fragment order
-  int32_t *qe;            // their exponents, per query
-  int2 *kve;              // and per key tile (k, v)
+  __bf16 *q, *k, *v;      // operands in three parts, in MFMA fragment order
   float *part;            // per split block: o [64][hd], then (max, sum) [64][2]
 };
 size_t flash_bytes(const AttnArgs &a);

@@ -1,14 +1,16 @@
 // Prefill attention: many rows of one sequence, causal GQA over the cached
 // keys and the rows' own (semantics in attention.hip).
 //
-// Operands in two fp16 parts.  A value y = x 2^-e (e per query, per 32-key
-// tile of K and of V, chosen so that the largest |y| lies in [2^13, 2^14)) is
-// held as hi = fp16(y) and lo = fp16(y - hi): 2^-24 relative, what an fp32
-// value carries, down to 2^-38 of the largest, below which the parts are
-// fixed point.  A product takes three v_mfma_f32_16x16x32_f16 (hi hi, hi lo,
-// lo hi; lo lo is below 2^-24 of the product) with fp32 sums.  On gfx950 one
-// fp32 16x16x4 MFMA takes as long as a fp16 16x16x32: three of the latter do
-// the work of eight of the former.
+// Operands in three bf16 parts.  A value is h + m + l, h its rounding to bf16, m that
+// of the rest and l what is left: 8 + 8 + 8 bits and two signs hold the 24 bits of a
+// fp32 value (of at least 2^-109 or zero; below, to 2^-133), and every part has fp32's
+// range, so no exponent is shared between values: a row's result does not depend on
+// the size of others in its tile.  A product takes six v_mfma_f32_16x16x32_bf16 (hh, hm,
+// mh, hl, mm, lh) with fp32 sums; what is dropped (ml, lm, ll) is below 2^-25 of the
+// product and 2^-28 of it in the mean.  On gfx950 one fp32 16x16x4 MFMA takes as
+// long as a bf16 16x16x32: six of the latter do the work of eight of the former.
+// (Two fp16 parts with an exponent per tile, three MFMAs: 23 bits near the tile's
+// maximum and fewer below 2^-15 of it.)
 //
 //  k_flash_prep   q and k after RoPE, v, and the cached keys the rows attend
 //                 to, split and written in MFMA fragment order (lane l of a
@@ -31,15 +33,18 @@
 //  k_flash_merge  log-sum-exp merge of the key splits.
 //
 // Error against 64 bits (relative 2-norm, normal q, k and v, scores up to 0.3 to 3 times
-// sqrt(hd)): 1.0e-7 to 1.3e-6 at 300 to 2048 rows, 1.2e-7 to 1.8e-6 for the fp32 MFMA
-// kernel before it; 0.8e-7 to 3.2e-7 at 17 rows against 0.6e-7 to 4.6e-7.
+// sqrt(hd)): 0.6e-7 to 1.2e-6 at 300 to 2048 rows, 0.5e-7 to 2.0e-7 at 17 rows, below
+// that of an fp32 MFMA kernel with one running sum in each of 18 cells (1.2e-7 to 1.8e-6,
+// 0.6e-7 to 4.6e-7).  The two fp16 parts took 0.7 of this kernel's time, 1.0e-7 to 1.3e-6
+// on these inputs, 0.8e-7 to 3.2e-7 at 17 rows, and 1e-5 to 5e-5 in rows or dims beside
+// values 2^24 times theirs.
 //
-// Measured (E4B, 2048 rows; the fp32 MFMA kernel before it): sliding layer 45
-// + 13 (prep) against 135 + 17 us (RoPE and append launches), full layer 190 + 32
-// + 14 (merge) against 515 + 29; 14B class, 1000 rows, one layer: 62 + 16
-// against 5.0 ms of chunk launches.  Bound by the fragment reads and MFMAs of one
-// wave per SIMD; a short prompt by latency (77 rows: 10.5 + 7.4 against 22.5 +
-// 9.5 us).
+// Measured (E4B, 2048 rows; the fp32 kernel before): sliding layer 64 to 70 + 16 (prep)
+// against 135 + 17 us (RoPE and append launches), full layer 263 to 295 + 40 + 13.5
+// (merge) against 515 + 29; 14B class, 1000 rows, one layer: 81 + 17.5 against 5.0 ms of
+// chunk launches.  Bound by the fragment reads of one wave per SIMD and by its softmax:
+// the matrix cores are busy 38% of the time at head dim 256.  A short prompt by latency
+// (77 rows: 14.5 + 6.3 against 22.5 + 9.5 us).
 #include <algorithm>
 #include <cmath>
 
@@ -49,15 +54,14 @@
 namespace ms {
 namespace {
 
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
-typedef int i2 __attribute__((ext_vector_type(2)));
 
 constexpr int kQB = 64;   // queries per block: 16 per wave
 constexpr int kKT = 32;   // keys per tile
 constexpr int kFlashMaxSplits = 32;
 constexpr int kFlashMaxBlocks = 512;  // blocks of a split launch
-constexpr int kPBits = 14;            // P is scaled by 2^14 before its split
+constexpr int kFrag = 3 * 512;        // values of a fragment: three parts of 1 KiB
 
 // First and last key that the row at position pos attends to.
 __host__ __device__ inline void key_span(int circular, int clamp, int cache_len, int pos, int *lo,
@@ -84,26 +88,27 @@ __host__ __device__ inline int split_count(const FlashBuf &f, int nt) {
   return f.maxs == 1 ? 1 : (n < f.maxs ? n : f.maxs);
 }
 
-// |x| for the tile's scale; what is not finite does not set it
-__device__ inline float fin_abs(float x) {
-  const float v = fabsf(x);
-  return v < INFINITY ? v : 0.f;
-}
-// e with 2^-e * m in [2^13, 2^14); 0 for m = 0
-__device__ inline int scale_exp(float m) {
-  return m > 0.f ? __builtin_amdgcn_frexp_expf(m) - 14 : 0;
-}
-// hi and lo of x[0..7] 2^-e to dst and dst + 512 (halves)
-__device__ inline void store_split(const float *x, int e, _Float16 *dst) {
-  h8 hi, lo;
+// The parts of eight values.  (A value that rounds past the largest bf16 is cut off
+// instead; what is not finite has itself and zeros as its parts.)
+__device__ inline void split3(const float *x, bf8 &h, bf8 &m, bf8 &l) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const float y = ldexpf(x[j], -e);
-    hi[j] = (_Float16)y;
-    lo[j] = (_Float16)(y - (float)hi[j]);
+    const bool fin = fabsf(x[j]) < INFINITY;
+    h[j] = (__bf16)x[j];
+    if (fin && !(fabsf((float)h[j]) < INFINITY))
+      h[j] = (__bf16)__uint_as_float(__float_as_uint(x[j]) & 0xFFFF0000u);
+    const float r = fin ? x[j] - (float)h[j] : 0.f;
+    m[j] = (__bf16)r;
+    l[j] = (__bf16)(r - (float)m[j]);
   }
-  *reinterpret_cast<h8 *>(dst) = hi;
-  *reinterpret_cast<h8 *>(dst + 512) = lo;
+}
+// the parts of x[0..7] to dst, dst + 512 and dst + 1024
+__device__ inline void store_split(const float *x, __bf16 *dst) {
+  bf8 h, m, l;
+  split3(x, h, m, l);
+  *reinterpret_cast<bf8 *>(dst) = h;
+  *reinterpret_cast<bf8 *>(dst + 512) = m;
+  *reinterpret_cast<bf8 *>(dst + 1024) = l;
 }
 
 // Dims d0 .. d0 + 7 of a head row at src, after RoPE at position pos where
@@ -162,7 +167,6 @@ __global__ __launch_bounds__(prep_threads<HD>()) void k_flash_prep(AttnArgs a, F
   constexpr int KS = HD / 32;      // 32-dim MFMA steps
   __shared__ const float *krow[kKT], *vrow[kKT];
   __shared__ int kslot[kKT], kind[kKT];  // kind: 0 no key, 1 cached, 2 one of the rows
-  __shared__ float red[2][16];
   const int tid = threadIdx.x;
   const int G = a.n_heads / a.n_kv;
   int blk = blockIdx.x;
@@ -176,20 +180,13 @@ __global__ __launch_bounds__(prep_threads<HD>()) void k_flash_prep(AttnArgs a, F
       const int q = blk / a.n_kv * 32 + (tid + NT * i) / PK, d8 = (tid + NT * i) % PK;
       const int row = q / G, head = h * G + q - row * G;
       const bool ok = row < a.T;
-      float x[8], m = 0.f;
+      float x[8];
       load_rope8(a, a.qkv + (ok ? (size_t)row * a.ld + head * HD : 0), 8 * d8, ok, f.base + row,
                  x);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        x[j] = ok ? x[j] : 0.f;
-        m = fmaxf(m, fin_abs(x[j]));
-      }
-#pragma unroll
-      for (int o = 1; o < PK; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
-      const int e = scale_exp(m);
-      if (d8 == 0) f.qe[h * nq + q] = e;
-      store_split(x, e, f.q + (h * nq + (q & ~15)) * HD * 2 + (d8 >> 2) * 1024 +
-                            ((d8 & 3) * 16 + (q & 15)) * 8);
+      for (int j = 0; j < 8; ++j) x[j] = ok ? x[j] : 0.f;
+      store_split(x, f.q + ((h * nq + (q & ~15)) * HD / 512 + (d8 >> 2)) * kFrag +
+                         ((d8 & 3) * 16 + (q & 15)) * 8);
     }
     return;
   }
@@ -211,7 +208,7 @@ __global__ __launch_bounds__(prep_threads<HD>()) void k_flash_prep(AttnArgs a, F
     kslot[tid] = kd == 2 && (circ ? r >= a.T - a.cache_len : slot < a.cache_len) ? slot : -1;
   }
   __syncthreads();
-  float x[NP][8], v[NP][8], mk = 0.f, mv = 0.f;
+  float x[NP][8], v[NP][8];
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
     // V piece (dim, lk): keys 4 lk + 0..3 and 16 + 4 lk + 0..3
@@ -224,35 +221,16 @@ __global__ __launch_bounds__(prep_threads<HD>()) void k_flash_prep(AttnArgs a, F
     for (int j = 0; j < 8; ++j) {
       x[i][j] = kind[kk] ? x[i][j] : 0.f;
       v[i][j] = kind[4 * lk + (j & 3) + 4 * (j & 4)] ? v[i][j] : 0.f;
-      mk = fmaxf(mk, fin_abs(x[i][j]));
-      mv = fmaxf(mv, fin_abs(v[i][j]));
     }
   }
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    mk = fmaxf(mk, __shfl_xor(mk, o, 64));
-    mv = fmaxf(mv, __shfl_xor(mv, o, 64));
-  }
-  if ((tid & 63) == 0) {
-    red[0][tid >> 6] = mk;
-    red[1][tid >> 6] = mv;
-  }
-  __syncthreads();
-#pragma unroll 1
-  for (int w = 0; w < NT / 64; ++w) {
-    mk = fmaxf(mk, red[0][w]);
-    mv = fmaxf(mv, red[1][w]);
-  }
-  const int ek = scale_exp(mk), ev = scale_exp(mv);
-  if (tid == 0) f.kve[h * f.nkt + kt] = int2{ek, ev};
-  const size_t tile = ((size_t)h * f.nkt + kt) * HD * 64;  // halves per tile and operand
+  const size_t tile = ((size_t)h * f.nkt + kt) * HD / 16 * kFrag;
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
     const int dim = (tid + NT * i) % HD, lk = (tid + NT * i) / HD;
     const int kk = (tid + NT * i) / PK, d8 = (tid + NT * i) % PK;
-    store_split(x[i], ek, f.k + tile + ((kk >> 4) * KS + (d8 >> 2)) * 1024 +
-                              ((d8 & 3) * 16 + (kk & 15)) * 8);
-    store_split(v[i], ev, f.v + tile + (dim >> 4) * 1024 + (lk * 16 + (dim & 15)) * 8);
+    store_split(x[i], f.k + tile + ((kk >> 4) * KS + (d8 >> 2)) * kFrag +
+                          ((d8 & 3) * 16 + (kk & 15)) * 8);
+    store_split(v[i], f.v + tile + (dim >> 4) * kFrag + (lk * 16 + (dim & 15)) * 8);
     if (!f.append) continue;
     if (kslot[kk] >= 0) {
       float *d = a.kc + (size_t)kslot[kk] * a.kv_dim + hc + 8 * d8;
@@ -308,49 +286,42 @@ __device__ inline float exp_neg(float d) {
 }
 
 // Instruction order of a product phase of `reads` fragment reads feeding `mfmas`
-// MFMAs: eight reads ahead, then four per six MFMAs.  (Left to itself the
-// compiler reads each fragment right before its use and waits for it; with one
-// wave per SIMD nothing else covers that.)
-template <int READS, int MFMAS>
+// MFMAs: nine reads ahead, then three per six MFMAs, and `valus` vector instructions
+// (the softmax beside the scores) behind each MFMA.  (Left to itself the compiler
+// reads each fragment right before its use and waits for it; with one wave per SIMD
+// nothing else covers that.)
+template <int READS, int MFMAS, int VALUS>
 __device__ inline void interleave() {
-  constexpr int kMfma = 0x008, kRead = 0x100;
-  __builtin_amdgcn_sched_group_barrier(kRead, 8, 0);
+  constexpr int kMfma = 0x008, kRead = 0x100, kValu = 0x002;
+  __builtin_amdgcn_sched_group_barrier(kRead, 9, 0);
 #pragma unroll
-  for (int i = 8; i < READS; i += 4) {
-    __builtin_amdgcn_sched_group_barrier(kMfma, 6, 0);
-    __builtin_amdgcn_sched_group_barrier(kRead, 4, 0);
+  for (int i = 9; i < READS; i += 3) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+      __builtin_amdgcn_sched_group_barrier(kMfma, 1, 0);
+      if (k & 1) __builtin_amdgcn_sched_group_barrier(kRead, 1, 0);
+      if (VALUS > 0) __builtin_amdgcn_sched_group_barrier(kValu, VALUS, 0);
+    }
   }
   __builtin_amdgcn_sched_group_barrier(kMfma, MFMAS, 0);
 }
 
-// vmcnt(n), every other counter free
-template <int N>
-__device__ inline void wait_loads() {
-  __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-  asm volatile("" ::: "memory");
-}
-// A barrier behind this wave's LDS reads (lgkmcnt(0), vmcnt free): the loads issued
-// after it, by any wave, refill buffers that the reads before it used.
-__device__ inline void block_sync() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
-
-// Head dims up to 256 keep two K and two V tiles in LDS (DB): the scores of
-// tile t + 1 are computed beside the softmax and P V of tile t, one barrier a
-// tile.  At 512 one tile of each fits (128 KiB): V(t) arrives during the
-// scores, K(t + 1) during P V.
+// Keys and values go through a ring of three LDS stages of up to 48 KiB: a K or V
+// tile (half of one at head dim 512: 16 keys of K, 256 dims of V).  Two stages are
+// in flight while one is read.  Head dims up to 256 take them in the order K0, K1, V0,
+// K2, V1, .. (AHEAD): the scores of tile t + 1 are computed beside the softmax of
+// tile t.
 template <int HD>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD <= 256 ? 2 : 1, HD <= 256 ? 2 : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(HD <= 128 ? 2 : 1, HD <= 128 ? 2 : 1)))
 void k_flash(AttnArgs a, FlashBuf f) {
   constexpr int KS = HD / 32, DT = HD / 16;
-  constexpr int TB = HD * 128;         // bytes of a K or V tile
-  constexpr bool DB = HD <= 256;
-  constexpr int NLD = TB / 4096;       // 1 KiB loads per wave and tile
+  constexpr int TB = HD * 192;         // bytes of a K or V tile
+  constexpr bool AHEAD = HD <= 256;
+  constexpr int NST = AHEAD ? 1 : 2;   // stages of a tile
+  constexpr int SB = TB / NST;         // bytes of a stage
+  constexpr int NLD = SB / 4096;       // 1 KiB loads per wave and stage
+  constexpr int ND = AHEAD ? 4 : 2;    // 16-dim tiles of O in one go
   extern __shared__ __align__(16) uint8_t lds[];
-  uint8_t *kb = lds, *vb = lds + (DB ? 2 : 1) * TB;
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int li = lane & 15, lk = lane >> 4;
@@ -366,6 +337,7 @@ void k_flash(AttnArgs a, FlashBuf f) {
   if (sp >= nsplit) return;
   t0 += sp * f.st_tiles;
   if (sp < nsplit - 1) t1 = t0 + f.st_tiles - 1;
+  const int n = t1 - t0 + 1, n_stages = 2 * NST * n;
 
   const size_t nq = (size_t)f.n_qt * kQB;
   const int qi = qt * kQB + wave * 16 + li, row = qi / G;
@@ -374,165 +346,190 @@ void k_flash(AttnArgs a, FlashBuf f) {
   key_span(circ, a.clamp, a.cache_len, f.base + row, &lo, &hi);
   lo = valid ? lo - f.kbase : 1;
   hi = valid ? hi - f.kbase : 0;
-  const int qe = ldg<int32_t>(f.qe + h * nq + qi);
-  h8 qh[KS], ql[KS];
+  bf8 qh[KS], qm[KS], ql[KS];
   {
-    const _Float16 *qp = f.q + (h * nq + qt * kQB + wave * 16) * HD * 2 + lane * 8;
+    const __bf16 *qp = f.q + (h * nq + qt * kQB + wave * 16) * HD / 512 * kFrag + lane * 8;
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
-      qh[s] = ldg<h8>(qp + s * 1024);
-      ql[s] = ldg<h8>(qp + s * 1024 + 512);
+      qh[s] = ldg<bf8>(qp + s * kFrag);
+      qm[s] = ldg<bf8>(qp + s * kFrag + 512);
+      ql[s] = ldg<bf8>(qp + s * kFrag + 1024);
     }
   }
-  const __amdgpu_buffer_rsrc_t kg =
-      buffer_of(reinterpret_cast<const uint8_t *>(f.k) + (size_t)h * f.nkt * TB, f.nkt * TB);
-  const __amdgpu_buffer_rsrc_t vg =
-      buffer_of(reinterpret_cast<const uint8_t *>(f.v) + (size_t)h * f.nkt * TB, f.nkt * TB);
-  // tile t of a K or V array into LDS: this wave's NLD kilobytes
+  const uint8_t *kg = reinterpret_cast<const uint8_t *>(f.k) + (size_t)h * f.nkt * TB;
+  const uint8_t *vg = reinterpret_cast<const uint8_t *>(f.v) + (size_t)h * f.nkt * TB;
+  // this wave's NLD kilobytes of stage i, if there is one, into a slot of the ring
   const int voff = wave * (NLD * 1024) + lane * 16;
-  auto issue = [&](const __amdgpu_buffer_rsrc_t src, int t, uint8_t *dst) {
+  auto issue = [&](int i, int slot) {
+    if (i >= n_stages) return;
+    int t, half = 0;
+    bool is_v;
+    if constexpr (AHEAD) {
+      t = (i - 1) >> 1;
+      is_v = i > 0 && (t == n - 1 || !(i & 1));
+      t += is_v ? 0 : 1;  // (stage 0: K of tile 0)
+    } else {
+      t = i >> 2;
+      is_v = i & 2;
+      half = i & 1;
+    }
+    const int src = (t0 + t) * TB + half * SB;
+    const __amdgpu_buffer_rsrc_t r = buffer_of(is_v ? vg : kg, f.nkt * TB);
+    uint8_t *dst = lds + slot * SB + wave * NLD * 1024;
 #pragma unroll
-    for (int i = 0; i < NLD; ++i)
-      load_lds16(src, dst + (wave * NLD + i) * 1024, voff, t * TB + i * 1024);
+    for (int u = 0; u < NLD; ++u) load_lds16(r, dst + u * 1024, voff, src + u * 1024);
   };
-  // S^T of the tile at kt: s[u], keys 16 u + 4 lk + e of query li
+  // Stage `stage` (in ring slot `slot`) becomes readable; stage + 2 goes into the
+  // slot of stage - 1: the barrier comes after this wave's loads of `stage` (those
+  // of stage + 1 may be in flight) and after its reads of stage - 1.
+  int stage = -1, slot = 2;
+  auto next = [&]() {
+    ++stage;
+    slot = slot == 2 ? 0 : slot + 1;
+    asm volatile("" ::: "memory");
+    if (stage + 1 < n_stages)
+      __builtin_amdgcn_s_waitcnt(0x0070 | (NLD & 15) | ((NLD >> 4) << 14));
+    else
+      __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue(stage + 2, slot == 0 ? 2 : slot - 1);
+    return (const uint8_t *)(lds + slot * SB + lane * 16);
+  };
+  // S^T of NU x 16 keys (fragments from kt): keys 4 lk + e of query li.  Sums of the
+  // small products apart, added last; no MFMA feeds one of the next two.
+  constexpr int NU = 2 / NST;
   auto scores = [&](const uint8_t *kt, f4 *s) {
-    f4 x[2];  // the small products, added last
+    f4 x[NU], y[NU], z[NU];
 #pragma unroll
-    for (int u = 0; u < 2; ++u) s[u] = x[u] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < NU; ++u) s[u] = x[u] = y[u] = z[u] = f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int d = 0; d < KS; ++d)
+    for (int d = 0; d < KS; ++d) {
+      bf8 kh[NU], km[NU], kl[NU];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const h8 kh = *reinterpret_cast<const h8 *>(kt + (u * KS + d) * 2048 + lane * 16);
-        const h8 kl = *reinterpret_cast<const h8 *>(kt + (u * KS + d) * 2048 + 1024 + lane * 16);
-        s[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, qh[d], s[u], 0, 0, 0);
-        x[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh, ql[d], x[u], 0, 0, 0);
-        x[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl, qh[d], x[u], 0, 0, 0);
+      for (int u = 0; u < NU; ++u) {
+        kh[u] = *reinterpret_cast<const bf8 *>(kt + (u * KS + d) * 3072);
+        km[u] = *reinterpret_cast<const bf8 *>(kt + (u * KS + d) * 3072 + 1024);
+        kl[u] = *reinterpret_cast<const bf8 *>(kt + (u * KS + d) * 3072 + 2048);
       }
-    interleave<4 * KS, 6 * KS>();
+#define MS_QK(k, q, r)              \
+  _Pragma("unroll") for (int u = 0; u < NU; ++u) r[u] = \
+      __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[u], q[d], r[u], 0, 0, 0)
+      MS_QK(kh, qh, s);
+      MS_QK(kh, qm, x);
+      MS_QK(km, qh, y);
+      MS_QK(kh, ql, z);
+      MS_QK(km, qm, x);
+      MS_QK(kl, qh, y);
+#undef MS_QK
+    }
+    if constexpr (!AHEAD) interleave<3 * NU * KS, 6 * NU * KS, 0>();
 #pragma unroll
-    for (int u = 0; u < 2; ++u) s[u] += x[u];
+    for (int u = 0; u < NU; ++u) s[u] += (x[u] + y[u]) + z[u];
   };
   f4 o[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d) o[d] = f4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
-  int E = -(1 << 20);  // o is in units of 2^(E - 14), E the largest V exponent so far
-  // exponents of tile t's K and V, loaded through a vector register: scalar
-  // loads in flight would turn every wait for an LDS read into one for all
-  auto exps = [&](int t) {
-    int z;
-    asm volatile("v_mov_b32 %0, 0" : "=v"(z));
-    return ldg<i2>(f.kve + h * f.nkt + t + z);
-  };
-  // softmax of the scores of tile t against the running maximum: p in its two
-  // parts, o and l rescaled
-  auto softmax = [&](int t, const i2 kve, const f4 *s, h8 &ph, h8 &pl) {
-    const int ke = __builtin_amdgcn_readfirstlane(kve.x);
-    const int ve = __builtin_amdgcn_readfirstlane(kve.y);
-    const float sf = ldexpf(a.scale, qe + ke);
+  // softmax of the scores of tile t against the running maximum: p in its
+  // parts, l rescaled; returns the factor of o
+  auto softmax = [&](int t, const f4 *s, bf8 &ph, bf8 &pm, bf8 &pl) {
     const int k0 = t * kKT;
     float x[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) x[i] = s[i >> 2][i & 3] * sf;
-    if (!__all(lo <= k0 && hi >= k0 + kKT - 1)) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const int k = k0 + 16 * (i >> 2) + 4 * lk + (i & 3);
-        x[i] = k >= lo && k <= hi ? x[i] : -INFINITY;
-      }
-    }
-    float mt = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
-                     fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
-    const float mn = fmaxf(m, max_rows(mt));
-    const float safe = mn == -INFINITY ? 0.f : mn;
-    if (ve > E || __any(mn != m)) {
-      const int En = ve > E ? ve : E;
-      const float c = m == -INFINITY ? 0.f : exp_neg(m - safe);
-      const float oc = ldexpf(c, E - En);
-      l *= c;
-#pragma unroll
-      for (int d = 0; d < DT; ++d) o[d] *= oc;
-      m = mn;
-      E = En;
-    }
-    const int pe = kPBits + ve - E;
+    for (int i = 0; i < 8; ++i) x[i] = s[i >> 2][i & 3] * a.scale;
+    // (no branch for tiles without a masked key: the next tile's MFMAs run beside this)
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
-      const float p = exp_neg(x[i] - safe);
-      l += p;
-      const float y = ldexpf(p, pe);
-      ph[i] = (_Float16)y;
-      pl[i] = (_Float16)(y - (float)ph[i]);
+      const int k = k0 + 16 * (i >> 2) + 4 * lk + (i & 3);
+      x[i] = k >= lo && k <= hi ? x[i] : -INFINITY;
     }
+    const float mt = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
+                           fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+    const float mn = fmaxf(m, max_rows(mt));
+    const float safe = mn == -INFINITY ? 0.f : mn;
+    const float c = exp_neg(m - safe);  // (0 before the first key)
+    m = mn;
+    float ps = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      x[i] = exp_neg(x[i] - safe);
+      ps += x[i];
+    }
+    l = l * c + ps;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      ph[i] = (__bf16)x[i];
+      const float r = x[i] - (float)ph[i];
+      pm[i] = (__bf16)r;
+      pl[i] = (__bf16)(r - (float)pm[i]);
+    }
+    // (in place: not behind the next barrier, where no MFMAs cover it)
+    asm volatile("" : "+v"(ph), "+v"(pm), "+v"(pl), "+v"(l));
+    return c;
   };
-  // O^T += V^T P^T
-  auto pv = [&](const uint8_t *vt, const h8 ph, const h8 pl) {
+  // O^T = c O^T + V^T P^T for the dims of a stage, the tile's sum apart (one rounding
+  // of o per tile)
+  auto pv = [&](const uint8_t *vt, int d0, float c, const bf8 ph, const bf8 pm, const bf8 pl) {
 #pragma unroll
-    for (int d = 0; d < DT; d += 4) {
-      h8 vh[4], vl[4];
+    for (int d = 0; d < DT / NST; d += ND) {
+      bf8 vh[ND], vm[ND], vl[ND];
+      f4 r[ND];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        vh[i] = *reinterpret_cast<const h8 *>(vt + (d + i) * 2048 + lane * 16);
-        vl[i] = *reinterpret_cast<const h8 *>(vt + (d + i) * 2048 + 1024 + lane * 16);
+      for (int i = 0; i < ND; ++i) {
+        vh[i] = *reinterpret_cast<const bf8 *>(vt + (d + i) * 3072);
+        vm[i] = *reinterpret_cast<const bf8 *>(vt + (d + i) * 3072 + 1024);
+        vl[i] = *reinterpret_cast<const bf8 *>(vt + (d + i) * 3072 + 2048);
+        r[i] = f4{0.f, 0.f, 0.f, 0.f};
       }
+#define MS_PV(v, p)              \
+  _Pragma("unroll") for (int i = 0; i < ND; ++i) r[i] = \
+      __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[i], p, r[i], 0, 0, 0)
+      MS_PV(vl, ph);
+      MS_PV(vm, pm);
+      MS_PV(vh, pl);
+      MS_PV(vm, ph);
+      MS_PV(vh, pm);
+      MS_PV(vh, ph);
+#undef MS_PV
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        o[d + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[i], ph, o[d + i], 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        o[d + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[i], pl, o[d + i], 0, 0, 0);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        o[d + i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[i], ph, o[d + i], 0, 0, 0);
+      for (int i = 0; i < ND; ++i) o[d0 + d + i] = o[d0 + d + i] * c + r[i];
     }
-    interleave<2 * DT, 3 * DT>();
+    interleave<3 * DT / NST, 6 * DT / NST, 0>();
   };
 
-  h8 ph, pl;
-  if constexpr (DB) {
-    i2 e = exps(t0);
-    issue(kg, t0, kb);
-    issue(vg, t0, vb);
-    wait_loads<0>();
-    block_sync();
-    if (t0 < t1) issue(kg, t0 + 1, kb + TB);
+  bf8 ph, pm, pl;
+  issue(0, 0);
+  issue(1, 1);
+  if constexpr (AHEAD) {
     f4 s[2];
-    scores(kb, s);
-    for (int t = t0, b = 0; t <= t1; ++t, b ^= 1) {
-      // K(t + 1) and V(t) have landed, and no wave still reads the buffers
-      // that the next loads fill
-      wait_loads<0>();
-      block_sync();
-      const i2 en = exps(t < t1 ? t + 1 : t);
-      if (t + 2 <= t1) issue(kg, t + 2, kb + b * TB);
-      if (t + 1 <= t1) issue(vg, t + 1, vb + (b ^ 1) * TB);
+    const uint8_t *st = next();
+    scores(st, s);
+#pragma unroll 1
+    for (int t = 0; t < n; ++t) {
+      if (t < n - 1) st = next();
       f4 sn[2];
-      scores(kb + (b ^ 1) * TB, sn);  // past the last tile: not used
-      softmax(t, e, s, ph, pl);
-      pv(vb + b * TB, ph, pl);
+      scores(st, sn);  // past the last tile: not used
+      const float c = softmax(t0 + t, s, ph, pm, pl);
+      interleave<6 * KS, 12 * KS, 32 / KS>();
+      st = next();
+      pv(st, 0, c, ph, pm, pl);
       s[0] = sn[0];
       s[1] = sn[1];
-      e = en;
     }
   } else {
-    issue(kg, t0, kb);
-    for (int t = t0; t <= t1; ++t) {
-      const i2 e = exps(t);
-      issue(vg, t, vb);
-      wait_loads<NLD>();
-      block_sync();
+#pragma unroll 1
+    for (int t = 0; t < n; ++t) {
       f4 s[2];
-      scores(kb, s);
-      block_sync();
-      if (t < t1) issue(kg, t + 1, kb);
-      softmax(t, e, s, ph, pl);
-      if (t < t1) wait_loads<NLD>();
-      else wait_loads<0>();
-      block_sync();
-      pv(vb, ph, pl);
-      block_sync();
+      const uint8_t *st = next();
+      scores(st, s);
+      st = next();
+      scores(st, s + 1);
+      const float c = softmax(t0 + t, s, ph, pm, pl);
+      st = next();
+      pv(st, 0, c, ph, pm, pl);
+      st = next();
+      pv(st, DT / 2, c, ph, pm, pl);
     }
   }
   // the query's sum over its four lanes
@@ -544,10 +541,7 @@ void k_flash(AttnArgs a, FlashBuf f) {
     float *op = a.out + (size_t)row * a.q_dim + (h * G + qi - row * G) * HD + 4 * lk;
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
-      f4 v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = ldexpf(o[d][e], E - kPBits) * w;
-      *reinterpret_cast<f4 *>(op + 16 * d) = v;
+      *reinterpret_cast<f4 *>(op + 16 * d) = o[d] * w;
     }
     return;
   }
@@ -555,12 +549,7 @@ void k_flash(AttnArgs a, FlashBuf f) {
   float *pb = f.part + (size_t)j * kQB * (HD + 2);
   float *po = pb + (wave * 16 + li) * HD + 4 * lk;
 #pragma unroll
-  for (int d = 0; d < DT; ++d) {
-    f4 v;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = ldexpf(o[d][e], E - kPBits);
-    *reinterpret_cast<f4 *>(po + 16 * d) = v;
-  }
+  for (int d = 0; d < DT; ++d) *reinterpret_cast<f4 *>(po + 16 * d) = o[d];
   if (lk == 0) {
     float *pm = pb + kQB * HD + (wave * 16 + li) * 2;
     pm[0] = m;
@@ -656,11 +645,9 @@ FlashBuf flash_view(const AttnArgs &a, int base, void *buf, size_t *bytes) {
     off += up256(b);
     return r;
   };
-  f.q = reinterpret_cast<_Float16 *>(take(nq * a.hd * 4));
-  f.k = reinterpret_cast<_Float16 *>(take(nk * a.hd * 4));
-  f.v = reinterpret_cast<_Float16 *>(take(nk * a.hd * 4));
-  f.qe = reinterpret_cast<int32_t *>(take(nq * 4));
-  f.kve = reinterpret_cast<int2 *>(take((size_t)a.n_kv * f.nkt * 8));
+  f.q = reinterpret_cast<__bf16 *>(take(nq * a.hd * 6));
+  f.k = reinterpret_cast<__bf16 *>(take(nk * a.hd * 6));
+  f.v = reinterpret_cast<__bf16 *>(take(nk * a.hd * 6));
   f.part = reinterpret_cast<float *>(
       take(f.maxs > 1 ? (size_t)f.maxs * f.n_qt * a.n_kv * kQB * (a.hd + 2) * 4 : 0));
   *bytes = off;
@@ -669,7 +656,7 @@ FlashBuf flash_view(const AttnArgs &a, int base, void *buf, size_t *bytes) {
 
 template <int HD>
 void launch_hd(const AttnArgs &a, const FlashBuf &f, hipStream_t st) {
-  constexpr int lds = HD * 128 * (HD <= 256 ? 4 : 2);
+  constexpr int lds = 3 * 192 * (HD <= 256 ? HD : HD / 2);
   hipLaunchKernelGGL(k_flash_prep<HD>, dim3((f.nkt + 2 * f.n_qt) * a.n_kv),
                      dim3(prep_threads<HD>()), 0, st, a, f);
   hipLaunchKernelGGL(k_flash<HD>, dim3(f.maxs * f.n_qt * a.n_kv), dim3(256), lds, st, a, f);
@@ -691,7 +678,7 @@ size_t flash_bytes_max(const AttnArgs &a) {
   const size_t nq = (size_t)a.n_kv * ((a.T * G + kQB - 1) / kQB) * kQB;
   const size_t keys = a.cache_kind == MS_CACHE_CIRCULAR ? (size_t)a.cache_len + a.T : a.cache_len;
   const size_t nk = (size_t)a.n_kv * (keys + 2 * kKT);
-  return nq * a.hd * 4 + 2 * nk * a.hd * 4 + nq * 4 + nk + 8 * 256 +
+  return nq * a.hd * 6 + 2 * nk * a.hd * 6 + 8 * 256 +
          (size_t)kFlashMaxBlocks * kQB * (a.hd + 2) * 4;
 }
 

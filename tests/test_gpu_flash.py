@@ -3,11 +3,11 @@ numbers of query heads per kv head that do not divide the 64-query tiles, every
 head size, rows and positions at the edges of the 32-key tiles, key splits, a
 window shorter than the rows, and the cache contents afterwards.
 
-Bound: q, k, v and p are held to 2^-24 of each value, products of the small
-parts are dropped (2^-24), sums are fp32.  A score's error is then below about
-3 * 2^-24 * sum |q k| scale, at |q|, |k| ~ 2 and hd <= 512 below 1e-5 absolute,
-and moves a probability by as much relatively; the outputs' relative RMSE is
-held to 2e-6 (an fp32 evaluation shows 1e-7 .. 5e-7)."""
+Bound: q, k, v and p enter exactly (three bf16 parts), each product lacks less than
+2^-24 of itself, sums are fp32.  A score's error is then below about 3 * 2^-24 * sum |q
+k| scale, at |q|, |k| ~ 2 and hd <= 512 below 1e-5 absolute, and moves a probability by
+as much relatively; the outputs' relative RMSE is held to 2e-6 (an fp32 evaluation shows
+1e-7 .. 5e-7)."""
 import ctypes as C
 
 import numpy as np
@@ -54,8 +54,7 @@ def test_prefill_attention(gpu, case, scale):
     rng = np.random.default_rng(T * 7 + base)
     qd, kvd, G = nh * hd, nkv * hd, nh // nkv
     kc = (rng.standard_normal((clen, kvd)) * 2).astype(np.float32)
-    # values of very different size by position, and k and q whose product keeps
-    # its size: the tiles' exponents must not lose the small ones
+    # v of different size by position, and k and q whose product keeps its size
     vc = (rng.standard_normal((clen, kvd)) * scale).astype(np.float32)
     q = (rng.standard_normal((T, qd)) * 2 / scale).astype(np.float32)
     kc *= np.float32(scale)
@@ -119,3 +118,84 @@ def test_prefill_attention_nan_row_stays_in_its_tile(gpu):
     assert np.abs(got[:-1] - mean[:-1, None]).max() < 1e-6
     assert np.abs(got[-1, 1:] - mean[-1]).max() < 1e-6
     assert np.isnan(got[-1, 0]).all()
+
+
+def attend(ms, nh, nkv, hd, circ, clen, q, kn, vn, base=0):
+    """ms_attention on fresh rows after zero caches (base 0)."""
+    T = len(q)
+    desc = ms.LayerDesc(q_dim=nh * hd, kv_dim=nkv * hd, head_dim=hd, n_heads=nh, n_kv_heads=nkv,
+                        rot_dim=hd, theta=1e4, cache_kind=circ, cache_len=clen, clamp_reads=0)
+    bufs = [ms.DeviceBuffer.from_array(np.ascontiguousarray(a.reshape(T, -1), np.float32))
+            for a in (q, kn, vn)]
+    caches = [ms.DeviceBuffer.from_array(np.zeros((clen, nkv * hd), np.float32)) for _ in "kv"]
+    out = ms.DeviceBuffer(T * nh * hd * 4)
+    ms.check(ms.lib().ms_attention(C.byref(desc), *(b.ptr for b in bufs + caches), T, base,
+                                   out.ptr))
+    got = out.download(np.float32, (T, nh, hd))
+    for b in bufs + caches + [out]:
+        b.free()
+    return got
+
+
+SPREADS = [("k-row", 128), ("k-row", 512), ("v-row", 256), ("v-row", 512), ("v-dims", 64),
+           ("v-dims", 256), ("v-dims", 512), ("k-dims", 128), ("k-dims", 512)]
+
+
+@pytest.mark.parametrize("kind,hd", SPREADS)
+def test_prefill_attention_magnitudes(gpu, kind, hd):
+    """Values 2^24 apart in one tile: a key, or a value, of no weight beside ordinary
+    ones, and dims of very different size.  Every row, head and dim is held to the
+    error of an fp32 evaluation by itself: the operands are exact and a sum of n
+    products in fp32 is off by about sqrt(n) 2^-25 of its terms' 2-norm, below 1e-6 here
+    for the scores (|s| ~ 1) and the outputs."""
+    ms = gpu
+    T, nh, nkv = 150, 4, 2
+    print(f"[flash] magnitudes {kind} hd={hd}", flush=True)
+    rng = np.random.default_rng(hd)
+    q = rng.standard_normal((T, nh, hd))
+    k = rng.standard_normal((T, nkv, hd))
+    v = rng.standard_normal((T, nkv, hd)) + 0.5
+    big = 2.0 ** 24
+    if kind in ("k-row", "v-row"):
+        # key 40 scores far below every other and has no weight
+        q[:, :, 0] = np.abs(q[:, :, 0]) + 1
+        k[40] = 0
+        k[40, :, 0] = -big if kind == "k-row" else -2000.0 * np.sqrt(hd)
+        if kind == "v-row":
+            v[40] *= big
+        rows = np.r_[0:40, 41:T]  # (row 40's first keys are ordinary as well)
+    else:
+        f = np.exp2(24.0 * np.arange(hd) / hd - 12).astype(np.float32)
+        if kind == "v-dims":
+            v *= f
+        else:
+            k, q = k * f, q / f
+        rows = np.arange(T)
+    q, k, v = (a.astype(np.float32) for a in (q, k, v))
+    got = attend(ms, nh, nkv, hd, 0, 256, q, k, v).astype(np.float64)
+    pos = np.arange(T)
+    ref = reference(q.astype(np.float64), k.astype(np.float64), v.astype(np.float64), nh // nkv,
+                    np.zeros(T, int), pos, 0)
+    e, r = (got - ref)[rows], ref[rows]
+    row_err = np.sqrt((e ** 2).mean(2) / (r ** 2).mean(2))
+    dim_err = np.sqrt((e ** 2).mean(0) / (r ** 2).mean(0))
+    print(f"[flash]   worst row {row_err.max():.2e}, worst dim {dim_err.max():.2e}", flush=True)
+    if kind != "v-dims":
+        assert row_err.max() < 2e-6
+    assert dim_err.max() < 2e-6
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256, 512])
+def test_prefill_attention_rows_do_not_depend_on_later_ones(gpu, hd):
+    """Later rows change no bit of an earlier row's output, whatever their size."""
+    ms = gpu
+    rng = np.random.default_rng(hd)
+    T, nh, nkv = 70, 4, 2
+    q, k, v = (rng.standard_normal((T, n, hd)).astype(np.float32) for n in (nh, nkv, nkv))
+    a = attend(ms, nh, nkv, hd, 0, 128, q, k, v)
+    for r in (5, 37, 69):
+        k2, v2 = k.copy(), v.copy()
+        k2[r:] *= np.float32(3e4)
+        v2[r:] *= np.float32(3e-5)
+        b = attend(ms, nh, nkv, hd, 0, 128, q, k2, v2)
+        assert np.array_equal(a[:r], b[:r])
