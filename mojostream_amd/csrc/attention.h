@@ -108,6 +108,7 @@ struct FlashBuf {
   int st_tiles, maxs;     // key tiles per split, splits per query tile (1: none)
   int append;             // k_flash_prep appends the rows to the cache
   __bf16 *q, *k, *v;      // operands in three parts, in MFMA fragment order
+  int32_t *bad;           // per key tile: k or v holds a value that is not finite
   float *part;            // per split block: o [64][hd], then (max, sum) [64][2]
 };
 size_t flash_bytes(const AttnArgs &a);

@@ -30,6 +30,8 @@
 //                 half tile), which are the B operand of the second product
 //                 as they are (V^T is stored with the same key order), and the
 //                 softmax needs two lane swaps a tile.
+//                 A block whose tiles hold a value that is not finite
+//                 (k_flash_prep's flags) goes key by key instead.
 //  k_flash_merge  log-sum-exp merge of the key splits.
 //
 // Error against 64 bits (relative 2-norm, normal q, k and v, scores up to 0.3 to 3 times
@@ -223,6 +225,14 @@ __global__ __launch_bounds__(prep_threads<HD>()) void k_flash_prep(AttnArgs a, F
       v[i][j] = kind[4 * lk + (j & 3) + 4 * (j & 4)] ? v[i][j] : 0.f;
     }
   }
+  int bad = 0;
+#pragma unroll
+  for (int i = 0; i < NP; ++i)
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      bad |= !(fabsf(x[i][j]) < INFINITY) || !(fabsf(v[i][j]) < INFINITY);
+  bad = __syncthreads_or(bad);
+  if (tid == 0) f.bad[h * f.nkt + kt] = bad;
   const size_t tile = ((size_t)h * f.nkt + kt) * HD / 16 * kFrag;
 #pragma unroll
   for (int i = 0; i < NP; ++i) {
@@ -306,6 +316,77 @@ __device__ inline void interleave() {
   __builtin_amdgcn_sched_group_barrier(kMfma, MFMAS, 0);
 }
 
+// Value j of the fragment piece at p, from its parts.
+__device__ inline float whole(const __bf16 *p, int j) {
+  return ((float)p[j] + (float)p[512 + j]) + (float)p[1024 + j];
+}
+
+// The queries of one wave over key tiles t0 .. t1, key by key in fp32: for blocks whose
+// tiles hold values that are not finite.  There the products of parts, and those with
+// the weights of masked keys (0 NaN), would reach rows that do not attend to the value.
+// Lanes take 64 keys for the scores and HD / 64 dims each for the output.
+template <int HD, class Store>
+__device__ inline void flash_plain(const AttnArgs &a, const FlashBuf &f, int h, int q0, int t0,
+                                   int t1, int lane, Store store) {
+  constexpr int KS = HD / 32, ND = HD / 64;
+  const int G = a.n_heads / a.n_kv, circ = a.cache_kind == MS_CACHE_CIRCULAR;
+  const size_t nq = (size_t)f.n_qt * kQB, tile = (size_t)HD / 16 * kFrag;
+  const __bf16 *kb = f.k + h * f.nkt * tile, *vb = f.v + h * f.nkt * tile;
+#pragma unroll 1
+  for (int q = q0; q < q0 + 16; ++q) {
+    int lo = 1, hi = 0;
+    if (q / G < a.T) {
+      key_span(circ, a.clamp, a.cache_len, f.base + q / G, &lo, &hi);
+      lo = max(lo - f.kbase, t0 * kKT);
+      hi = min(hi - f.kbase, t1 * kKT + kKT - 1);
+    }
+    const __bf16 *qp = f.q + (h * nq + q0) * HD / 512 * kFrag + (q - q0) * 8;
+    float m = -INFINITY, l = 0.f, o[ND];
+#pragma unroll
+    for (int j = 0; j < ND; ++j) o[j] = 0.f;
+#pragma unroll 1
+    for (int k0 = lo; k0 <= hi; k0 += 64) {
+      const bool on = k0 + lane <= hi;
+      const int k = on ? k0 + lane : hi, kk = k % kKT;
+      const __bf16 *kp = kb + k / kKT * tile + (kk >> 4) * KS * kFrag + (kk & 15) * 8;
+      float s = 0.f;
+#pragma unroll 1
+      for (int d8 = 0; d8 < HD / 8; ++d8) {
+        const int p = (d8 >> 2) * kFrag + (d8 & 3) * 128;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s = __builtin_fmaf(whole(qp + p, j), whole(kp + p, j), s);
+      }
+      const float x = on ? s * a.scale : -INFINITY;
+      float mn = x;
+#pragma unroll
+      for (int i = 1; i < 64; i <<= 1) mn = fmaxf(mn, __shfl_xor(mn, i, 64));
+      mn = fmaxf(m, mn);
+      const float safe = mn == -INFINITY ? 0.f : mn;
+      const float p = on ? expf(x - safe) : 0.f, c = m == -INFINITY ? 0.f : expf(m - safe);
+      float ps = p;
+#pragma unroll
+      for (int i = 1; i < 64; i <<= 1) ps += __shfl_xor(ps, i, 64);
+      l = l * c + ps;
+      m = mn;
+#pragma unroll
+      for (int j = 0; j < ND; ++j) o[j] *= c;
+#pragma unroll 1
+      for (int u = k0; u <= min(hi, k0 + 63); ++u) {
+        const float pu = __shfl(p, u - k0, 64);
+        const int uk = u % kKT;
+        const __bf16 *vp = vb + u / kKT * tile + ((uk >> 2) & 3) * 128;
+#pragma unroll
+        for (int j = 0; j < ND; ++j) {
+          const int d = lane + 64 * j;
+          o[j] = __builtin_fmaf(pu, whole(vp + (d >> 4) * kFrag + (d & 15) * 8,
+                                          (uk & 3) + (uk >> 4) * 4), o[j]);
+        }
+      }
+    }
+    store(q, m, l, o);
+  }
+}
+
 // Keys and values go through a ring of three LDS stages of up to 48 KiB: a K or V
 // tile (half of one at head dim 512: 16 keys of K, 256 dims of V).  Two stages are
 // in flight while one is read.  Head dims up to 256 take them in the order K0, K1, V0,
@@ -346,6 +427,8 @@ void k_flash(AttnArgs a, FlashBuf f) {
   key_span(circ, a.clamp, a.cache_len, f.base + row, &lo, &hi);
   lo = valid ? lo - f.kbase : 1;
   hi = valid ? hi - f.kbase : 0;
+  int bad = 0;
+  for (int t = t0 + lane; t <= t1; t += 64) bad |= ldg<int32_t>(f.bad + h * f.nkt + t);
   bf8 qh[KS], qm[KS], ql[KS];
   {
     const __bf16 *qp = f.q + (h * nq + qt * kQB + wave * 16) * HD / 512 * kFrag + lane * 8;
@@ -498,6 +581,7 @@ void k_flash(AttnArgs a, FlashBuf f) {
     interleave<3 * DT / NST, 6 * DT / NST, 0>();
   };
 
+  float *pb = f.part + (size_t)j * kQB * (HD + 2);
   bf8 ph, pm, pl;
   issue(0, 0);
   issue(1, 1);
@@ -532,6 +616,24 @@ void k_flash(AttnArgs a, FlashBuf f) {
       pv(st, DT / 2, c, ph, pm, pl);
     }
   }
+  if (__any(bad)) {
+    // (here, where its registers cost the loops nothing)
+    flash_plain<HD>(a, f, h, qt * kQB + wave * 16, t0, t1, lane,
+                    [&](int q, float m1, float l1, const float *o1) {
+      const int row1 = q / G, ql = q % kQB;
+      if (nsplit == 1 && row1 >= a.T) return;
+      float *d = nsplit == 1 ? a.out + (size_t)row1 * a.q_dim + (h * G + q - row1 * G) * HD
+                             : pb + ql * HD;
+      const float w = nsplit == 1 ? 1.0f / l1 : 1.0f;
+#pragma unroll
+      for (int i = 0; i < HD / 64; ++i) d[lane + 64 * i] = o1[i] * w;
+      if (nsplit > 1 && lane == 0) {
+        pb[kQB * HD + 2 * ql] = m1;
+        pb[kQB * HD + 2 * ql + 1] = l1;
+      }
+    });
+    return;
+  }
   // the query's sum over its four lanes
   l += __shfl_xor(l, 16, 64);
   l += __shfl_xor(l, 32, 64);
@@ -546,7 +648,6 @@ void k_flash(AttnArgs a, FlashBuf f) {
     return;
   }
   // partial of this split: o, then (max, sum), per query
-  float *pb = f.part + (size_t)j * kQB * (HD + 2);
   float *po = pb + (wave * 16 + li) * HD + 4 * lk;
 #pragma unroll
   for (int d = 0; d < DT; ++d) *reinterpret_cast<f4 *>(po + 16 * d) = o[d];
@@ -648,6 +749,7 @@ FlashBuf flash_view(const AttnArgs &a, int base, void *buf, size_t *bytes) {
   f.q = reinterpret_cast<__bf16 *>(take(nq * a.hd * 6));
   f.k = reinterpret_cast<__bf16 *>(take(nk * a.hd * 6));
   f.v = reinterpret_cast<__bf16 *>(take(nk * a.hd * 6));
+  f.bad = reinterpret_cast<int32_t *>(take((size_t)a.n_kv * f.nkt * 4));
   f.part = reinterpret_cast<float *>(
       take(f.maxs > 1 ? (size_t)f.maxs * f.n_qt * a.n_kv * kQB * (a.hd + 2) * 4 : 0));
   *bytes = off;
@@ -678,7 +780,7 @@ size_t flash_bytes_max(const AttnArgs &a) {
   const size_t nq = (size_t)a.n_kv * ((a.T * G + kQB - 1) / kQB) * kQB;
   const size_t keys = a.cache_kind == MS_CACHE_CIRCULAR ? (size_t)a.cache_len + a.T : a.cache_len;
   const size_t nk = (size_t)a.n_kv * (keys + 2 * kKT);
-  return nq * a.hd * 6 + 2 * nk * a.hd * 6 + 8 * 256 +
+  return nq * a.hd * 6 + 2 * nk * a.hd * 6 + nk + 8 * 256 +
          (size_t)kFlashMaxBlocks * kQB * (a.hd + 2) * 4;
 }
 

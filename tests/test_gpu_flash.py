@@ -199,3 +199,77 @@ def test_prefill_attention_rows_do_not_depend_on_later_ones(gpu, hd):
         v2[r:] *= np.float32(3e-5)
         b = attend(ms, nh, nkv, hd, 0, 128, q, k2, v2)
         assert np.array_equal(a[:r], b[:r])
+
+
+@pytest.mark.parametrize("hd,T", [(64, 70), (128, 150), (256, 300), (512, 600)])
+@pytest.mark.parametrize("kind", ["v-nan", "v-inf", "k-inf", "k-weightless"])
+def test_prefill_attention_not_finite(gpu, kind, hd, T):
+    """A value that is not finite reaches the rows that attend to its key with a weight,
+    in its dim, and no other: not earlier rows of its tile, and not through the parts of
+    the operands.  (The last case has keys in several splits.)"""
+    ms = gpu
+    print(f"[flash] {kind} hd={hd} T={T}", flush=True)
+    nh, nkv, r = 4, 2, T // 2 + 9
+    rng = np.random.default_rng(hd)
+    q, k, v = (rng.standard_normal((T, n, hd)).astype(np.float32) for n in (nh, nkv, nkv))
+    q[:, :, 3] = np.abs(q[:, :, 3]) + np.float32(0.1)
+    pos = np.arange(T)
+    zero = np.zeros(T, int)
+    f64 = [a.astype(np.float64) for a in (q, k, v)]
+    if kind == "k-weightless":
+        # a score of -inf in kv head 1: the same as without the key
+        k[r, 1, 3] = -np.inf
+        ref = reference(*f64, nh // nkv, zero, pos, 0)
+        rest = np.delete(pos, r)
+        with_r = reference(f64[0][r:], f64[1][rest], f64[2][rest], nh // nkv, zero[r:],
+                           pos[r:] - 1, 0)
+        ref[r:, 2:] = with_r[:, 2:]
+        hit = np.zeros((T, nh, hd), bool)
+        value = None
+    else:
+        ref = reference(*f64, nh // nkv, zero, pos, 0)
+        hit = np.zeros((T, nh, hd), bool)
+        if kind == "k-inf":
+            k[r, 1, 3] = np.inf  # the softmax of an infinite score: NaN
+            hit[r:, 2:] = True
+            value = np.isnan
+        else:
+            v[r, 1, 5] = np.nan if kind == "v-nan" else np.inf
+            hit[r:, 2:, 5] = True
+            value = np.isnan if kind == "v-nan" else np.isposinf
+    got = attend(ms, nh, nkv, hd, 0, 1024, q, k, v)
+    if value is not None:
+        assert value(got[hit]).all()
+    e, w = got[~hit] - ref[~hit], ref[~hit]
+    assert np.isfinite(e).all()
+    err = np.sqrt(np.mean(e ** 2) / np.mean(w ** 2))
+    print(f"[flash]   rel rmse {err:.2e}", flush=True)
+    assert err < 2e-6
+
+
+def test_prefill_attention_not_finite_outside_the_window(gpu):
+    """Cached keys that the window has left, in the first tile of the rows, are not
+    finite: no row sees them."""
+    ms = gpu
+    nh, nkv, hd, clen, T, base = 4, 2, 128, 96, 40, 150
+    rng = np.random.default_rng(5)
+    q, kn, vn = (rng.standard_normal((T, n * hd)).astype(np.float32) for n in (nh, nkv, nkv))
+    kc, vc = (rng.standard_normal((clen, nkv * hd)).astype(np.float32) for _ in "kv")
+    pos = base + np.arange(T)
+    lo = pos - clen + 1
+    old = np.arange(lo[0], base)
+    # (keys 32 .. 54 share a tile with key 55, the first that a row attends to; their
+    # slots now hold keys 128 .. 149 and one that is to come)
+    slot = (lo[0] - 1) % clen
+    kc[slot], vc[slot] = np.nan, np.inf
+    k = np.concatenate([kc[old % clen], kn]).astype(np.float64).reshape(-1, nkv, hd)
+    v = np.concatenate([vc[old % clen], vn]).astype(np.float64).reshape(-1, nkv, hd)
+    ref = reference(q.astype(np.float64).reshape(T, nh, hd), k, v, nh // nkv, lo, pos, lo[0])
+    desc = ms.LayerDesc(q_dim=nh * hd, kv_dim=nkv * hd, head_dim=hd, n_heads=nh, n_kv_heads=nkv,
+                        rot_dim=hd, theta=1e4, cache_kind=1, cache_len=clen, clamp_reads=0)
+    bufs = [ms.DeviceBuffer.from_array(a) for a in (q, kn, vn, kc, vc)]
+    out = ms.DeviceBuffer(T * nh * hd * 4)
+    ms.check(ms.lib().ms_attention(C.byref(desc), *(b.ptr for b in bufs), T, base, out.ptr))
+    got = out.download(np.float32, (T, nh, hd))
+    assert np.isfinite(got).all()
+    assert np.sqrt(np.mean((got - ref) ** 2) / np.mean(ref ** 2)) < 2e-6
