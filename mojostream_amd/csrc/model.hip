@@ -58,6 +58,8 @@ enum { PC_QKV, PC_ATTN, PC_O, PC_GATEUP, PC_DOWN, PC_LM, PC_PREP, PC_OTHER };
 static const char *kProfNames[MS_PROF_CLASSES] = {"qkv_gemv", "attention", "o_gemv",
                                                   "gateup_gemv", "down_gemv", "lm_head",
                                                   "embed_prep", "other"};
+// launchers of the one-row attention (launch_attn_rec)
+enum { AT_CHUNKS, AT_PART, AT_PART_MERGED, AT_BATCH, AT_BATCH_MERGED };
 struct Prof {
   bool on = false;
   long launches[MS_PROF_CLASSES] = {};
@@ -79,8 +81,13 @@ struct Prof {
   AttnArgs last_attn[2] = {};
   int last_attn_layer[2] = {};
   bool have_attn[2] = {};
-  bool attn_part[2] = {};  // that launch left its chunks to the O projection
+  int attn_how[2] = {};  // its launcher
   int layer = -1;
+  const void *model = nullptr;  // whose launches were recorded last
+  void forget() {
+    for (bool &h : have) h = false;
+    for (bool &h : have_attn) h = false;
+  }
 };
 static Prof g_prof;
 
@@ -392,6 +399,28 @@ static const float *layer_input(ms_model *m, const RunCfg &rc, int l) {
   return l == rc.first_layer ? rc.in_rows : m->xs;
 }
 
+static int launch_attn(int how, const AttnArgs &a, hipStream_t st) {
+  switch (how) {
+    case AT_PART: return launch_attention_partials(a, st);
+    case AT_PART_MERGED: return launch_attention_partials(a, st, true);
+    case AT_BATCH: return launch_attention_batch(a, st);
+    case AT_BATCH_MERGED: return launch_attention_batch_merged(a, st);
+    default: return launch_attention(a, st);
+  }
+}
+
+// Layer l's attention launch, recorded for ms_prof_sweep where it is a decode step's.
+static int launch_attn_rec(int how, const AttnArgs &a, int l, hipStream_t st) {
+  if (g_prof.on && a.T == 1) {
+    const int k = a.cache_kind == MS_CACHE_CIRCULAR ? 1 : 0;
+    g_prof.last_attn[k] = a;
+    g_prof.last_attn_layer[k] = l;
+    g_prof.have_attn[k] = true;
+    g_prof.attn_how[k] = how;
+  }
+  return launch_attn(how, a, st);
+}
+
 static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
   Layer &Ly = m->L[l];
   g_prof.layer = l;
@@ -493,31 +522,24 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
     ProfScope ps(PC_ATTN, 0.0, st);
     if (use_part) {
       // chunk partials only; the O projection below merges them
-      if (g_prof.on) {
-        const int k = d.cache_kind == MS_CACHE_CIRCULAR ? 1 : 0;
-        g_prof.last_attn[k] = a;
-        g_prof.last_attn_layer[k] = l;
-        g_prof.have_attn[k] = true;
-        g_prof.attn_part[k] = true;
-      }
-      if (int rc2 = launch_attention_partials(a, st)) return rc2;
+      if (int rc2 = launch_attn_rec(AT_PART, a, l, st)) return rc2;
       merged_in_o = true;
     } else if (rc.T == 1 && attn_batch_ok(a) && merge_quant_ok(o_src, M, d.q_dim)) {
       // five sequences or more: chunk partials; the O projection's quantization
       // merges them
-      if (int rc2 = launch_attention_batch(a, st)) return rc2;
+      if (int rc2 = launch_attn_rec(AT_BATCH, a, l, st)) return rc2;
       merged_in_quant = true;
     } else if (rc.T == 1 && dec_part_ok(a)) {
       // one row per sequence (a batch decode step, a one-row forward): the
       // same chunk blocks, merged by the last block of each (sequence, kv
       // head, head pair), the RoPE factors from the tables at each position
-      if (int rc2 = launch_attention_partials(a, st, true)) return rc2;
+      if (int rc2 = launch_attn_rec(AT_PART_MERGED, a, l, st)) return rc2;
     } else if (rc.T == 1 && attn_batch_ok(a) && dec_part_chunks(a) > 2) {
       // other one-row shapes: chunk partials and their merge (below 64 positions,
       // the first bucket of a captured step, one launch is faster while a single
       // chunk is attended: demo model, one row at position 0 758 against 846 us, at
       // 60 872 against 843, at 200 907 against 854)
-      if (int rc2 = launch_attention_batch_merged(a, st)) return rc2;
+      if (int rc2 = launch_attn_rec(AT_BATCH_MERGED, a, l, st)) return rc2;
     } else if (attn_rows_ok(a)) {
       // two to four rows of one sequence: chunk partials per row, merged
       if (int rc2 = launch_attention_rows(a, st)) return rc2;
@@ -525,14 +547,7 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
       // prefill rows of one sequence: flash attention
       if (int rc2 = launch_attention_prefill(a, m->flash, m->flash_bytes, st)) return rc2;
     } else {
-      if (g_prof.on && rc.T == 1) {
-        const int k = d.cache_kind == MS_CACHE_CIRCULAR ? 1 : 0;
-        g_prof.last_attn[k] = a;
-        g_prof.last_attn_layer[k] = l;
-        g_prof.have_attn[k] = true;
-        g_prof.attn_part[k] = false;
-      }
-      if (int rc2 = launch_attention(a, st)) return rc2;
+      if (int rc2 = launch_attn_rec(AT_CHUNKS, a, l, st)) return rc2;
     }
   }
   // 3. x2 = x + attn . Wo (residual epilogue)
@@ -758,6 +773,7 @@ static int run_layers(ms_model *m, const RunCfg &rc, hipStream_t st) {
   const bool streaming = !m->d.resident;
   const int l0 = rc.first_layer, l1 = rc.first_layer + rc.n_layers;
   m->kpend.ks = 0;
+  if (g_prof.on) g_prof.model = m;
   if (streaming) {
     // timing of this pass ([copy start, copy end] per layer and compute
     // waits), added to the statistics of the API call (reset at its start)
@@ -1033,6 +1049,7 @@ extern "C" int ms_model_destroy(ms_model *m) {
   (void)hipStreamSynchronize(ctx().stream);
   (void)hipStreamSynchronize(ctx().copy_stream);
   drop_graphs(m);
+  if (g_prof.model == m) g_prof.forget();  // they point into its buffers
   if (m->h_pos_pin) (void)hipHostFree(m->h_pos_pin);
   for (auto &Ly : m->L)
     for (int i = 0; i < 7; ++i)
@@ -1612,6 +1629,7 @@ extern "C" int ms_model_stream_stats(ms_model *m, ms_stream_stats *out) {
 
 extern "C" int ms_prof_enable(int on) {
   g_prof.on = on != 0;
+  if (on) g_prof.forget();  // (a sweep takes launches of this recording)
   for (int i = 0; i < MS_PROF_CLASSES; ++i) {
     g_prof.launches[i] = 0;
     g_prof.ms[i] = 0;
@@ -1662,7 +1680,7 @@ static int attn_sweep(ms_model *m, int passes, double *avg_us, double *bytes_per
   double bytes = 0;
   long n = 0;
   int rc = MS_OK;
-  if (g_prof.attn_part[k]) {
+  if (g_prof.attn_how[k] == AT_PART) {
     // the RoPE factors of the swept layers (one table for the kind)
     AttnArgs a = base;
     a.cos_t = m->ropes[Lr.rope].cs;
@@ -1682,9 +1700,7 @@ static int attn_sweep(ms_model *m, int passes, double *avg_us, double *bytes_per
       a.cache_len = Ly.d.cache_len;
       a.clamp = Ly.d.clamp_reads;
       a.write_cache = 0;
-      if ((rc = g_prof.attn_part[k] ? launch_attention_partials(a, st)
-                                     : launch_attention(a, st)))
-        break;
+      if ((rc = launch_attn(g_prof.attn_how[k], a, st))) break;
       for (int b = 0; b < a.B; ++b) {
         const int keys = std::min(pos[b] + 1, Ly.d.cache_len);
         bytes += 2.0 * keys * Ly.d.kv_dim * 4;

@@ -92,3 +92,49 @@ def test_14b_batch_equals_prefill(gpu, lens):
         d = np.linalg.norm(got[b] - ref) / np.linalg.norm(ref)
         assert d < 1e-5, (b, d)
     one.close()
+
+
+@pytest.mark.parametrize("kind,B", [("14b", 1), ("14b", 6), ("e4b", 1), ("e4b", 3), ("e4b", 6)])
+def test_attention_sweep_of_each_decode_path(gpu, kind, B):
+    """ms_prof_sweep re-runs the attention launch of the profiled step, whichever path the
+    step takes: on every layer of its kind, with the K and V rows of every attended key as
+    bytes, and without a trace in what the model decodes next."""
+    ms = gpu
+    say(f"attention sweep {kind} B={B}")
+    V, n = 4096, 90
+    arch = (ms.arch_14b(max_len=256, n_layers=3, vocab=V) if kind == "14b"
+            else ms.arch_e4b(max_full_seq=256, n_layers=6, vocab=V))
+    m = ms.Model(arch, max_seqs=B, max_rows=1, max_pos=256)
+    m.fill_synthetic(42)
+    rng = np.random.default_rng(B)
+    prompts = [rng.integers(0, V, n + b).tolist() for b in range(B)]
+    nxt = rng.integers(0, V, B).tolist()
+
+    def run(sweep):
+        m.reset()
+        for b, p in enumerate(prompts):
+            m.prefill(p, 0, b)
+        ms.prof_enable(sweep)
+        ids = [m.decode(nxt, [len(p) for p in prompts], 2, use_graph=False)]
+        ms.prof_enable(False)
+        if sweep:
+            sw = ms.prof_sweep(m, "attention", passes=2)
+            # (the E4B's sliding layers, five of six)
+            layers = [d for d in arch.layers if kind == "14b" or d.cache_kind == 1]
+            d = layers[0]
+            # (positions after the two steps)
+            keys = sum(min(len(p) + 3, d.cache_len) for p in prompts)
+            assert sw["launches"] == 2 * len(layers) and sw["avg_us"] > 0
+            assert sw["bytes_per_launch"] == 2.0 * keys * d.kv_dim * 4
+        ids.append(m.decode_continue(3, B, use_graph=False))
+        return np.concatenate(ids)
+
+    a, b = run(False), run(True)
+    m.close()
+    assert np.array_equal(a, b)
+    with pytest.raises(Exception):
+        other = ms.Model(arch, max_seqs=1, max_rows=1, max_pos=256)
+        try:
+            ms.prof_sweep(other, "attention")  # nothing recorded: its launches are gone
+        finally:
+            other.close()
