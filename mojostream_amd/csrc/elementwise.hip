@@ -250,8 +250,7 @@ extern "C" int ms_lm_head_argmax(const float *d_x, int M, int D, const uint8_t *
   MS_CHECK_ARG(D % 128 == 0 && D <= kQuantMaxK && vocab % 64 == 0,
                "lm_head: D % 128 (D <= 16384), vocab % 64");
   hipStream_t st = ctx().stream;
-  const int P = 4;
-  const long blocks = vocab / 16 / P;
+  const long blocks = vocab / 64;  // four panels each
   const size_t qb = (quant_rows_bytes(M, D) + 255) & ~(size_t)255;
   const size_t need = qb + (size_t)blocks * M * 8 + 64;
   void *buf = nullptr;
@@ -272,8 +271,6 @@ extern "C" int ms_lm_head_argmax(const float *d_x, int M, int D, const uint8_t *
   a.q = q;
   a.seg[0] = GemvSeg{d_packed, scale, vocab, 0};
   a.nseg = 1;
-  a.P = P;
-  a.waves = 4;
   a.out = d_logits;
   a.ldo = vocab;
   a.arg_val = bv;

@@ -356,9 +356,6 @@ static int launch_proj(ms_model *m, GemvArgs a, const RowSrc &r, int waves, hipS
   a.asrc = AS_QUANT;
   a.rows = RowSrc{};
   a.q = quant_rows_view(m->quant, a.M, a.K);
-  // one to four rows of a long residual projection (Down at batch 2-4): 16
-  // waves, every super-tile of a wave in one batch
-  a.waves = (a.M <= 4 && a.P == 1 && a.epi == EPI_RESID && waves == 16) ? 16 : 4;
   if (int rc = launch_quant_rows(r, a.M, a.K, a.q, st)) return rc;
   return launch_gemv_rec(a, st);
 }
@@ -578,7 +575,6 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
     } else if (merged_in_quant) {
       a.asrc = AS_QUANT;
       a.q = quant_rows_view(m->quant, M, d.q_dim);
-      a.waves = 4;
       if (int rc2 = launch_merge_quant(o_src, M, d.q_dim, a.q, st)) return rc2;
       if (int rc2 = launch_gemv_rec(a, st)) return rc2;
     } else if (int rc2 = launch_proj_row(m, rc, a, r, 8, 8, st)) {
@@ -711,8 +707,6 @@ static int enqueue_lm(ms_model *m, const RunCfg &rc, int row0, int M, const Argm
   a.q = quant_rows_view(m->quant, M, D);
   a.seg[0] = GemvSeg{m->lm_w, m->lm_scale, m->d.vocab, 0};
   a.nseg = 1;
-  a.P = 4;
-  a.waves = 4;
   a.out = m->sampling ? m->logits + (size_t)rc.seq0 * m->d.vocab : m->tap_logits;
   a.ldo = m->d.vocab;
   a.arg_val = m->arg_val;

@@ -106,8 +106,8 @@ struct GemvArgs {
   AttnPrep pf;    // AS_WAVES, one row, store epilogue: the decode attention's inputs
   GemvSeg seg[3];
   int nseg;
-  int P;          // panels per block (EPI_SWIGLU: 2, gate and up)
-  int waves;      // waves per block
+  int P;          // panels per block (EPI_SWIGLU: 2, gate and up) and waves per
+  int waves;      // block; with AS_QUANT the launcher chooses both
   float *out;     // [M][ldo]
   int ldo;
   float *sw_out;  // EPI_SWIGLU: [M][ldo_sw]

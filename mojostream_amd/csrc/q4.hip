@@ -578,24 +578,17 @@ __device__ inline void gemv_slot(const uint8_t *w0, const uint8_t *w1, const uin
 __device__ inline int dfrag(int i, int j) { return (j + 16 * (i >> 2)) * 4 + (i & 3); }
 
 // Super-tiles each wave keeps in flight per batch.  Ten per wave lets the
-// decode shapes (E4B gate|up: 5 per panel at W = 4) finish
-// in one batch.
-template <int C, int P>
-constexpr int gemv_batch() {
-  constexpr int u = 10 / C / P;
-  return u < 1 ? 1 : u;
-}
+// decode shapes (E4B gate|up: 5 per panel at W = 4) finish in one batch.
+constexpr int gemv_batch(int p) { return 10 / p < 1 ? 1 : 10 / p; }
 
-// LDS layout: int partial sums [W][P][C][256], output values [P][M][16],
+// LDS layout: int partial sums [W][P][256], output values [P][M][16],
 // shifts, then (AS_ROWS, AS_ATTN, AS_WAVES) limb rows [4M][K + 16] (16-byte
 // aligned).
-__host__ __device__ inline size_t gemv_lds_red(int W, int P, int C) {
-  return (size_t)W * P * C * 256 * 4;
-}
+__host__ __device__ inline size_t gemv_lds_red(int W, int P) { return (size_t)W * P * 256 * 4; }
 // shifts: one per row, or per (row, wave) with AS_WAVES (4 rows x 16 waves)
 constexpr int kRowShiftSlots = 64;
-__host__ __device__ inline size_t gemv_lds_fixed(int W, int P, int C, int M) {
-  return gemv_lds_red(W, P, C) + (size_t)P * M * 16 * 4 + (size_t)kRowShiftSlots * 4;
+__host__ __device__ inline size_t gemv_lds_fixed(int W, int P, int M) {
+  return gemv_lds_red(W, P) + (size_t)P * M * 16 * 4 + (size_t)kRowShiftSlots * 4;
 }
 __host__ __device__ inline int gemv_ldl(int K) { return K + 16; }
 
@@ -997,7 +990,7 @@ __device__ inline int wave_stream_load(const RowSrc &rs, int M, int32_t *row_s, 
   return s;
 }
 
-// C: 16-row MFMA groups (4 limb rows per activation row: M <= 4C).
+// One to four rows (4 limb rows per activation row, one 16-row MFMA group).
 // P: panels per block.  AS: GemvASource.  W: waves per block.  EPI: epilogue.
 // RP: activation rows whose loads the AS_ROWS prologue issues at once
 // (AS_ATTN: head dim and load batch, attn_hd / attn_nj; AS_WAVES: row bound
@@ -1007,7 +1000,7 @@ __device__ inline int wave_stream_load(const RowSrc &rs, int M, int32_t *row_s, 
 // w, w+W, ...; each batch issues U of them (P panels each) before any is
 // consumed, and the first batch is issued before the prologue so that the
 // weight stream overlaps the activation quantization.
-template <int C, int P, int AS, int W, int EPI, int RP>
+template <int P, int AS, int W, int EPI, int RP>
 __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
   extern __shared__ __align__(16) uint8_t lds[];
   // reduction scratch (AS_WAVES: a sum of squares per (row, wave))
@@ -1018,7 +1011,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
   constexpr bool WS = AS == AS_WSTREAM;
   constexpr int U = AS == AS_ATTN    ? attn_hd(RP) / 128
                     : (AS == AS_WAVES || WS) ? waves_tpw(RP)
-                                     : gemv_batch<C, P>();
+                                     : gemv_batch(P);
   // rows a WAVE_K epilogue finishes (AS_ATTN: one)
   constexpr int MR = (AS == AS_WAVES || WS) ? waves_rows(RP) : 1;
   constexpr int NSL = AS == AS_WAVES ? waves_nsl(RP) : 1;
@@ -1104,15 +1097,13 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
         resid_pre[m] = ldg<float>(resid + (size_t)m * ldo + col[p] + j);
   }
   int32_t *red = reinterpret_cast<int32_t *>(lds);
-  int32_t *row_s = reinterpret_cast<int32_t *>(lds + gemv_lds_red(W, P, C) + (size_t)P * M * 64);
-  int8_t *limbs = reinterpret_cast<int8_t *>(lds + gemv_lds_fixed(W, P, C, M));
+  int32_t *row_s = reinterpret_cast<int32_t *>(lds + gemv_lds_red(W, P) + (size_t)P * M * 64);
+  int8_t *limbs = reinterpret_cast<int8_t *>(lds + gemv_lds_fixed(W, P, M));
   const int ldl = gemv_ldl(K);
 
-  // A operand of this lane: row i of MFMA group c is limb row 16c + i
+  // A operand of this lane: limb row i
   const int i = lane & 15, g = lane >> 4;
-  bool a_on[C];
-#pragma unroll
-  for (int c = 0; c < C; ++c) a_on[c] = 16 * c + i < 4 * M;
+  const bool a_on = i < 4 * M;
 
   uint4 q[U][P];
   float pf_cs[2];  // PF: cos, sin at the position (block 0)
@@ -1162,7 +1153,7 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
     // its share of the quantization: at most four loads per wave go out
     // before it, the rest after the prologue.
     constexpr int kEarly = (4 / P) < 1 ? 1 : ((4 / P) < U ? (4 / P) : U);
-    if constexpr (RP == 4 && C == 1) {
+    if constexpr (RP == 4) {
       // two to four rows: side by side, one wave group per row
       rows_to_waves<W>(rs, K, M, limbs, ldl, row_s, sh, [&] { issue_part(0, 0, kEarly); });
     } else {
@@ -1227,13 +1218,9 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
   // panel's sums after the K loop (exact: each term stays in int32).
   const v4i kMinus8 = v4i{(int)0xF8F8F8F8u, (int)0xF8F8F8F8u, (int)0xF8F8F8F8u,
                           (int)0xF8F8F8F8u};
-  v4i acc[P][C], accz[C];
+  v4i acc[P], accz = v4i{0, 0, 0, 0};
 #pragma unroll
-  for (int p = 0; p < P; ++p)
-#pragma unroll
-    for (int c = 0; c < C; ++c) acc[p][c] = v4i{0, 0, 0, 0};
-#pragma unroll
-  for (int c = 0; c < C; ++c) accz[c] = v4i{0, 0, 0, 0};
+  for (int p = 0; p < P; ++p) acc[p] = v4i{0, 0, 0, 0};
 
   for (int bt = 0; bt < nb; ++bt) {
     if (bt > 0) issue(bt);
@@ -1254,19 +1241,12 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
                 uint2{lo[l], hi[l]};
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
-        v4i al[C][2];
-        if constexpr (AS == AS_ROWS || WAVE_K) {
-#pragma unroll
-          for (int c = 0; c < C; ++c) {
-            al[c][0] = v4i{0, 0, 0, 0};
-            al[c][1] = v4i{0, 0, 0, 0};
-            if (a_on[c]) {
-              const int8_t *ar = WS ? wb + (size_t)(16 * c + i) * kWsLd + 32 * g
-                                    : limbs + (size_t)(16 * c + i) * ldl + Gu * 128 + 32 * g;
-              al[c][0] = *reinterpret_cast<const v4i *>(ar);
-              al[c][1] = *reinterpret_cast<const v4i *>(ar + 16);
-            }
-          }
+        v4i al[2] = {v4i{0, 0, 0, 0}, v4i{0, 0, 0, 0}};
+        if (a_on) {
+          const int8_t *ar =
+              WS ? wb + (size_t)i * kWsLd + 32 * g : limbs + (size_t)i * ldl + Gu * 128 + 32 * g;
+          al[0] = *reinterpret_cast<const v4i *>(ar);
+          al[1] = *reinterpret_cast<const v4i *>(ar + 16);
         }
 #pragma unroll
         for (int p = 0; p < P; ++p) {
@@ -1275,35 +1255,23 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
           for (int h = 0; h < 2; ++h) {
             const uint32_t d0 = dw[2 * h], d1 = dw[2 * h + 1];
             const v4i b = v4i{nib_u8(d0), nib_u8(d0 >> 4), nib_u8(d1), nib_u8(d1 >> 4)};
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-              acc[p][c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[c][h], b, acc[p][c], 0, 0, 0);
-            }
+            acc[p] = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[h], b, acc[p], 0, 0, 0);
           }
         }
         // the zero point: sum_k limb(k) * (-8), once for all panels
 #pragma unroll
         for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int c = 0; c < C; ++c) {
-            accz[c] = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[c][h], kMinus8, accz[c], 0, 0, 0);
-          }
+          accz = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[h], kMinus8, accz, 0, 0, 0);
       }
     }
   }
   // acc = sum_k limb(k) * n_k + sum_k limb(k) * (-8) = sum_k limb(k) * (n_k - 8)
 #pragma unroll
-  for (int p = 0; p < P; ++p)
-#pragma unroll
-    for (int c = 0; c < C; ++c) acc[p][c] += accz[c];
+  for (int p = 0; p < P; ++p) acc[p] += accz;
 
 #pragma unroll
   for (int p = 0; p < P; ++p)
-#pragma unroll
-    for (int c = 0; c < C; ++c) {
-      int32_t *r = red + (((size_t)wave * P + p) * C + c) * 256 + lane * 4;
-      *reinterpret_cast<v4i *>(r) = acc[p][c];
-    }
+    *reinterpret_cast<v4i *>(red + ((size_t)wave * P + p) * 256 + lane * 4) = acc[p];
   __syncthreads();
 
   // output (slot p, row m, column j): sum the waves per limb row (exact int32:
@@ -1319,7 +1287,6 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
     static_assert(EPI == EPI_STORE || EPI == EPI_ACCUMULATE || EPI == EPI_RESID ||
                       EPI == EPI_SWIGLU,
                   "per-wave shifts: store, accumulate, residual or SwiGLU epilogue");
-    static_assert(C == 1, "per-wave shifts: at most four rows");
     const int t = threadIdx.x;
     const int w = t % W, p = (t / W) % P, j = t / (W * P);
     const bool on = t < 16 * P * W;
@@ -1418,13 +1385,12 @@ __global__ __launch_bounds__(64 * W, W == 4 ? 3 : 1) void k_gemv(GemvArgs a) {
     return;
   }
   auto value = [&](int p, int m, int j) {
-    const int c = m >> 2, r0 = 4 * (m & 3);
     long long t = 0;
 #pragma unroll
     for (int l = 0; l < 4; ++l) {
       int d = 0;
       for (int w = 0; w < W; ++w)
-        d += red[(((size_t)w * P + p) * C + c) * 256 + dfrag(r0 + l, j)];
+        d += red[((size_t)w * P + p) * 256 + dfrag(4 * m + l, j)];
       t += (long long)d << (8 * l);
     }
     return (float)((double)t * (double)ldexpf(1.0f, -row_s[m]) * (double)wsc[p]);
@@ -1910,6 +1876,8 @@ static int launch_gemv_rows(const GemvArgs &a, long n_panels, hipStream_t st) {
   for (int i = 0; i < a.nseg; ++i) even &= a.seg[i].n_cols % 32 == 0;
   const int P = epi == EPI_SWIGLU ? 2 : epi == EPI_ARGMAX ? 4
                 : (epi == EPI_RESID || !even || n_panels < 1024) ? 1 : 2;
+  MS_CHECK_ARG(epi == EPI_SWIGLU || n_panels % P == 0,
+               "GEMV: the head's width must be a multiple of 64");
   const long blocks = epi == EPI_SWIGLU ? a.seg[0].n_cols / 16 : n_panels / P;
   // waves: as few as hold K in one batch each and give every SIMD one
   int W = 4;
@@ -1950,7 +1918,7 @@ static int launch_gemv_rows(const GemvArgs &a, long n_panels, hipStream_t st) {
 }
 
 size_t gemv_lds_need(const GemvArgs &a) {
-  size_t b = gemv_lds_fixed(a.waves, a.P, 1, a.M);
+  size_t b = gemv_lds_fixed(a.waves, a.P, a.M);
   if (a.asrc == AS_ROWS || a.asrc == AS_ATTN || a.asrc == AS_WAVES)
     b += (size_t)4 * a.M * gemv_ldl(a.K);
   else if (a.asrc == AS_WSTREAM)
@@ -1983,7 +1951,8 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
                "GEMV: bad activation source");
   MS_CHECK_ARG(a.nseg >= 1 && a.nseg <= 3, "GEMV: 1 to 3 segments");
   MS_CHECK_ARG(a.epi != EPI_RESID || (a.resid && a.out), "GEMV: residual epilogue needs rows");
-  MS_CHECK_ARG(a.epi != EPI_SWIGLU || (a.P == 2 && a.nseg == 2 && a.sw_out),
+  MS_CHECK_ARG(a.epi != EPI_SWIGLU ||
+                   ((a.P == 2 || a.asrc == AS_QUANT) && a.nseg == 2 && a.sw_out),
                "GEMV: SwiGLU epilogue needs P=2, two segments and an output");
   MS_CHECK_ARG(a.epi != EPI_ARGMAX || (a.arg_val && a.arg_idx),
                "GEMV: argmax epilogue needs block-max buffers");
@@ -2021,7 +1990,7 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
     MS_CHECK_ARG(a.seg[i].w && a.seg[i].n_cols > 0 && a.seg[i].n_cols % 16 == 0,
                  "GEMV: segment width % 16 != 0");
     n_panels += a.seg[i].n_cols / 16;
-    if (a.epi != EPI_SWIGLU)
+    if (a.epi != EPI_SWIGLU && a.asrc != AS_QUANT)
       MS_CHECK_ARG((a.seg[i].n_cols / 16) % a.P == 0,
                    "GEMV: panels per block must divide every segment");
   }
@@ -2034,13 +2003,13 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
   MS_CHECK_ARG(shmem <= 160 * 1024 - 1024, "GEMV: LDS budget exceeded");
   bool ok = false;
   // Supported (epilogue, panels per block, activation source, waves).
-#define MS_GEMV_L(CC, EP, PP, AS, WW, RR) \
-  hipLaunchKernelGGL((k_gemv<CC, PP, AS, WW, EP, RR>), dim3(blocks), dim3(64 * WW), shmem, st, a)
+#define MS_GEMV_L(EP, PP, AS, WW, RR) \
+  hipLaunchKernelGGL((k_gemv<PP, AS, WW, EP, RR>), dim3(blocks), dim3(64 * WW), shmem, st, a)
 #define MS_GEMV(EP, PP, AS, WW)                                                   \
   if (!ok && a.epi == EP && a.P == PP && a.asrc == AS && a.waves == WW) {        \
     constexpr int RP = WW > 8 ? 1 : 4;                                            \
-    if (a.M == 1) MS_GEMV_L(1, EP, PP, AS, WW, 1);                                \
-    else MS_GEMV_L(1, EP, PP, AS, WW, RP);                                        \
+    if (a.M == 1) MS_GEMV_L(EP, PP, AS, WW, 1);                                \
+    else MS_GEMV_L(EP, PP, AS, WW, RP);                                        \
     ok = true;                                                                    \
   }
   MS_GEMV(EPI_STORE, 1, AS_ROWS, 8)
@@ -2057,14 +2026,14 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
                        (tpw == 5 || tpw == 2) && a.pf.pos && a.pf.cos_t && a.pf.sin_t &&
                        a.pf.half >= 0 && a.pf.half <= 256 && a.pf.rope_rows >= 1,
                    "GEMV: attention preparation: one row, store, 4 waves, K = 1024 or 2560");
-      if (tpw == 5) MS_GEMV_L(1, EPI_STORE, 1, AS_WAVES, 4, 115);
-      else MS_GEMV_L(1, EPI_STORE, 1, AS_WAVES, 4, 112);
+      if (tpw == 5) MS_GEMV_L(EPI_STORE, 1, AS_WAVES, 4, 115);
+      else MS_GEMV_L(EPI_STORE, 1, AS_WAVES, 4, 112);
       ok = true;
     }
 #define MS_GEMV_W(EP, PP, WW, T)                                       \
   if (!ok && a.epi == EP && a.waves == WW && tpw == T) {               \
-    if (a.M == 1) MS_GEMV_L(1, EP, PP, AS_WAVES, WW, 10 + T);          \
-    else MS_GEMV_L(1, EP, PP, AS_WAVES, WW, 10 * kWaveRowsMax + T);     \
+    if (a.M == 1) MS_GEMV_L(EP, PP, AS_WAVES, WW, 10 + T);          \
+    else MS_GEMV_L(EP, PP, AS_WAVES, WW, 10 * kWaveRowsMax + T);     \
     ok = true;                                                         \
   }
     MS_GEMV_W(EPI_STORE, 1, 4, 5)
@@ -2089,7 +2058,7 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
     const int tpw = a.K / (a.waves * kSuperK);
 #define MS_GEMV_S(EP, PP, WW, T)                                            \
   if (!ok && a.epi == EP && a.waves == WW && tpw == T) {                    \
-    MS_GEMV_L(1, EP, PP, AS_WSTREAM, WW, 10 * kWaveRowsMax + T);            \
+    MS_GEMV_L(EP, PP, AS_WSTREAM, WW, 10 * kWaveRowsMax + T);            \
     ok = true;                                                              \
   }
     MS_GEMV_S(EPI_STORE, 1, 4, 5)
@@ -2114,12 +2083,12 @@ int launch_gemv(const GemvArgs &a, hipStream_t st) {
     // the row-prologue template slot carries the head dim and the load pairs
     // per batch (a pair covers 512 / hd chunks)
     const int pairs = (a.at.chunks * a.at.hd + 511) / 512;
-    if (a.at.hd == 128) MS_GEMV_L(1, EPI_RESID, 1, AS_ATTN, 8, 104);
-    else if (a.at.hd == 256 && pairs <= 4) MS_GEMV_L(1, EPI_RESID, 1, AS_ATTN, 8, 204);
-    else if (a.at.hd == 256) MS_GEMV_L(1, EPI_RESID, 1, AS_ATTN, 8, 208);
-    else if (pairs <= 4) MS_GEMV_L(1, EPI_RESID, 1, AS_ATTN, 8, 404);
-    else if (pairs <= 8) MS_GEMV_L(1, EPI_RESID, 1, AS_ATTN, 8, 408);
-    else MS_GEMV_L(1, EPI_RESID, 1, AS_ATTN, 8, 416);
+    if (a.at.hd == 128) MS_GEMV_L(EPI_RESID, 1, AS_ATTN, 8, 104);
+    else if (a.at.hd == 256 && pairs <= 4) MS_GEMV_L(EPI_RESID, 1, AS_ATTN, 8, 204);
+    else if (a.at.hd == 256) MS_GEMV_L(EPI_RESID, 1, AS_ATTN, 8, 208);
+    else if (pairs <= 4) MS_GEMV_L(EPI_RESID, 1, AS_ATTN, 8, 404);
+    else if (pairs <= 8) MS_GEMV_L(EPI_RESID, 1, AS_ATTN, 8, 408);
+    else MS_GEMV_L(EPI_RESID, 1, AS_ATTN, 8, 416);
     ok = true;
   }
   MS_GEMV(EPI_SWIGLU, 2, AS_ROWS, 8)
@@ -2291,31 +2260,23 @@ static int q4_matmul_impl(float *d_C, const float *d_A, const uint8_t *d_packed,
       if (wave_shape_ok(a) && gemv_lds_need(a) <= 150 * 1024) return launch_gemv(a, st);
     }
   }
-  const int chunk = kGemvMaxM;
-  const int P = (N / 16) % 4 == 0 && N >= 4 * 16 * 512 ? 4 : 1;
-  const QuantRows q = quant_rows_view(buf, chunk, K);
-  for (int m0 = 0; m0 < M; m0 += chunk) {
-    const int mm = (M - m0 < chunk) ? M - m0 : chunk;
-    RowSrc r{};
-    r.x = d_A + (size_t)m0 * K;
-    r.ld = K;
-    r.pre_scale = 1.f;
-    if (int rc = launch_quant_rows(r, mm, K, q, st)) return rc;
-    GemvArgs a{};
-    a.epi = accumulate ? EPI_ACCUMULATE : EPI_STORE;
-    a.asrc = AS_QUANT;
-    a.K = K;
-    a.M = mm;
-    a.q = q;
-    a.seg[0] = GemvSeg{d_packed, scale, N, 0};
-    a.nseg = 1;
-    a.P = P;
-    a.waves = 4;
-    a.out = d_C + (size_t)m0 * N;
-    a.ldo = N;
-    if (int rc = launch_gemv(a, st)) return rc;
-  }
-  return MS_OK;
+  const QuantRows q = quant_rows_view(buf, M, K);
+  RowSrc r{};
+  r.x = d_A;
+  r.ld = K;
+  r.pre_scale = 1.f;
+  if (int rc = launch_quant_rows(r, M, K, q, st)) return rc;
+  GemvArgs a{};
+  a.epi = accumulate ? EPI_ACCUMULATE : EPI_STORE;
+  a.asrc = AS_QUANT;
+  a.K = K;
+  a.M = M;
+  a.q = q;
+  a.seg[0] = GemvSeg{d_packed, scale, N, 0};
+  a.nseg = 1;
+  a.out = d_C;
+  a.ldo = N;
+  return launch_gemv(a, st);
 }
 
 static int q4_matmul_check(int M, int K, int N) {
