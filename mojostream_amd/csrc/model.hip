@@ -120,14 +120,13 @@ struct ms_model {
   void *quant = nullptr;
   int quant_k = 0;
   // kpend: a split projection whose parts the next one's quantization combines
-  // (RowSrc::ks), where kdefer allows it; its operand's shifts and sums in kshift
+  // (RowSrc::ks), where launch_proj's caller allows it; its operand's shifts and sums in kshift
   // and kxsum
   struct {
     int ks;
     const float *resid;
     float scale;
   } kpend = {0, nullptr, 0.f};
-  bool kdefer = false;
   int32_t *kshift = nullptr;
   int64_t *kxsum = nullptr;
   int64_t *kpart = nullptr;  // sums of the K parts of a short prompt's O and Down
@@ -288,11 +287,14 @@ static int launch_gemv_rec(const GemvArgs &a, hipStream_t st) {
 // One row of one sequence with the row quantized per wave (AS_WAVES) when the
 // shapes fit (K = waves * 640), else launch_proj.
 static int launch_proj_row(ms_model *m, const RunCfg &rc, GemvArgs a, const RowSrc &r,
-                           int waves, int waves_row, hipStream_t st);
+                           int waves, int waves_row, bool defer, hipStream_t st);
 
 constexpr size_t kLdsLimit = 150 * 1024;  // LDS of a GEMV launch with its limb rows
 
-static int launch_proj(ms_model *m, GemvArgs a, const RowSrc &r, int waves, hipStream_t st) {
+// defer: the result (a.out) is read by the next projection's quantization and by nothing
+// else, so that a split GEMM may leave its parts for that one to combine.
+static int launch_proj(ms_model *m, GemvArgs a, const RowSrc &r, int waves, bool defer,
+                       hipStream_t st) {
   if (a.M > kGemvMaxM) {
     // prefill rows: quantize every row once (three limbs), then the MFMA GEMM
     GemmArgs g{};
@@ -326,7 +328,7 @@ static int launch_proj(ms_model *m, GemvArgs a, const RowSrc &r, int waves, hipS
     // Parts only: the operand's shifts and sums must outlive the next operand.  Rows of
     // up to 4096 values: E4B prompts of 17, 77, 250 tokens 3575, 4306, 6506 -> 3422,
     // 4152, 6428 us; longer rows (14B class, 30, 100, 300 tokens) gain nothing.
-    if (g.ksplit > 1 && m->kdefer && a.ldo <= 4096) {
+    if (g.ksplit > 1 && defer && a.ldo <= 4096) {
       g.parts_only = 1;
       g.a.shift = m->kshift;
       g.a.xsum = m->kxsum;
@@ -365,7 +367,7 @@ static int launch_proj(ms_model *m, GemvArgs a, const RowSrc &r, int waves, hipS
 // the LDS; otherwise launch_proj.  (At two to four rows the per-row prologue
 // of launch_proj is faster.)
 static int launch_proj_row(ms_model *m, const RunCfg &rc, GemvArgs a, const RowSrc &r,
-                           int waves, int waves_row, hipStream_t st) {
+                           int waves, int waves_row, bool defer, hipStream_t st) {
   if (rc.one_row && a.M == 1 && !r.gamma && !r.x_out) {
     GemvArgs w = a;
     w.asrc = AS_WAVES;
@@ -388,7 +390,7 @@ static int launch_proj_row(ms_model *m, const RunCfg &rc, GemvArgs a, const RowS
     w.waves = waves_row;
     if (wave_shape_ok(w) && gemv_lds_need(w) <= kLdsLimit) return launch_gemv_rec(w, st);
   }
-  return launch_proj(m, a, r, waves, st);
+  return launch_proj(m, a, r, waves, defer, st);
 }
 
 // Rows entering layer l: the previous layer's output or the call's input rows.
@@ -497,7 +499,7 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
       w.pf.rope_cur = m->rope_cur;
       if (int rc2 = launch_gemv_rec(w, st)) return rc2;
     } else {
-      if (int rc2 = launch_proj_row(m, rc, a, r, 8, 4, st)) return rc2;
+      if (int rc2 = launch_proj_row(m, rc, a, r, 8, 4, false, st)) return rc2;
       if (use_part)
         if (int rc2 = launch_rope_cur(attn, st)) return rc2;
     }
@@ -561,8 +563,6 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
     a.nseg = 1;
     a.P = 1;
     a.out = m->x2;
-    // (x2 is read by the next projection's quantization only)
-    m->kdefer = true;
     a.ldo = D;
     a.resid = m->xn;
     ProfScope ps(PC_O, (double)d.q_dim * D / 2, st);
@@ -577,7 +577,8 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
       a.q = quant_rows_view(m->quant, M, d.q_dim);
       if (int rc2 = launch_merge_quant(o_src, M, d.q_dim, a.q, st)) return rc2;
       if (int rc2 = launch_gemv_rec(a, st)) return rc2;
-    } else if (int rc2 = launch_proj_row(m, rc, a, r, 8, 8, st)) {
+    } else if (int rc2 = launch_proj_row(m, rc, a, r, 8, 8, true, st)) {
+      // (x2: only Gate|Up's rows)
       return rc2;
     }
   }
@@ -600,7 +601,7 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
     a.sw_out = m->aF;
     a.ldo_sw = F;
     ProfScope ps(PC_GATEUP, (double)D * F, st);
-    if (int rc2 = launch_proj_row(m, rc, a, r, 4, 4, st)) return rc2;
+    if (int rc2 = launch_proj_row(m, rc, a, r, 4, 4, false, st)) return rc2;
   }
   // 5. x_out = x2n + ffn . Wd (residual epilogue): the layer output
   {
@@ -618,12 +619,12 @@ static int enqueue_layer(ms_model *m, int l, const RunCfg &rc, hipStream_t st) {
     a.out = m->xs;
     // the layer's output: the next layer's quantization is its only reader inside a
     // run without taps
-    m->kdefer = l + 1 < rc.first_layer + rc.n_layers && !rc.hidden && !rc.tap_last;
+    const bool defer = l + 1 < rc.first_layer + rc.n_layers && !rc.hidden && !rc.tap_last;
     a.ldo = D;
     a.resid = m->x2n;
     if (rc.hidden) a.out2 = rc.hidden + (size_t)(l - rc.first_layer) * M * D;
     ProfScope ps(PC_DOWN, (double)F * D / 2, st);
-    if (int rc2 = launch_proj_row(m, rc, a, r, 16, 16, st)) return rc2;
+    if (int rc2 = launch_proj_row(m, rc, a, r, 16, 16, defer, st)) return rc2;
   }
   return MS_OK;
 }
