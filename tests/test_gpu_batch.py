@@ -138,3 +138,50 @@ def test_attention_sweep_of_each_decode_path(gpu, kind, B):
             ms.prof_sweep(other, "attention")  # nothing recorded: its launches are gone
         finally:
             other.close()
+
+
+# heads, kv heads, head dim, circular cache of 64: one to three and six to eight query
+# heads per kv head, the most heads and the longest rows of the merge in O's quantization
+SHAPES = [(2, 2, 128, 0), (4, 2, 128, 1), (6, 2, 128, 0), (12, 2, 128, 1), (14, 2, 128, 0),
+          (16, 2, 128, 0), (48, 8, 128, 0), (2, 2, 256, 0), (2, 1, 256, 1), (3, 1, 256, 0),
+          (1, 1, 512, 0), (2, 1, 512, 0), (3, 1, 512, 1), (16, 4, 512, 0)]
+
+
+@pytest.mark.parametrize("B", [1, 3, 6, 16])
+@pytest.mark.parametrize("nh,nkv,hd,circ", SHAPES)
+def test_decode_attention_shapes(gpu, nh, nkv, hd, circ, B):
+    """One layer, row by row, against the float64 statement of it: sequences at positions
+    of their own, 0 to past 128 (below 64 one launch, past it chunks and their merge; with
+    five rows or more the merge is in O's quantization).  Q4 rows carry 31 bits, everything
+    else is fp32: a row is within 2e-6 of 64 bits, as the other layers' tests hold it."""
+    from tests.golden.layer_ref import RefLayer
+    ms = gpu
+    say(f"decode attention nh={nh} nkv={nkv} hd={hd} circular={circ} B={B}")
+    D, n = 256, 133
+    desc = ms.LayerDesc(q_dim=nh * hd, kv_dim=nkv * hd, head_dim=hd, n_heads=nh, n_kv_heads=nkv,
+                        rot_dim=hd // 2, theta=1e4, cache_kind=circ,
+                        cache_len=64 if circ else 160, clamp_reads=0)
+    arch = ms.Arch("one", D, D, [desc])
+    rng = np.random.default_rng(nh * hd + B)
+    w = [rng.integers(1, 16, (k, c // 2 * 2)).astype(np.uint8) for k, c in arch.matrix_shapes(0)]
+    w = [(a[:, 0::2] | (a[:, 1::2] << 4)).astype(np.uint8) for a in w]
+    sc = [np.float32(1 / (4.3 * np.sqrt(k))) for k, _ in arch.matrix_shapes(0)]
+    m = ms.Model(arch, max_seqs=B, max_rows=1, max_pos=160)
+    for i in range(7):
+        m.set_matrix(0, i, w[i], float(sc[i]))
+    m.set_ple(0, 1.0)
+    x = rng.standard_normal((B, n, D)).astype(np.float32)
+    lag = [5 * b % 31 for b in range(B)]
+    got = np.zeros((B, n, D), np.float32)
+    for t in range(n):
+        # (a sequence that lags repeats its first row, which writes the same keys)
+        pos = [max(0, t - s) for s in lag]
+        out = m.layer_forward(0, np.stack([x[b, p] for b, p in enumerate(pos)]), pos, 1)
+        for b, p in enumerate(pos):
+            got[b, p] = out[b]
+    m.close()
+    for b in {0, B // 2, B - 1}:
+        k = n - lag[b]
+        ref = RefLayer(desc, D, D, w, sc, 1.0).forward(x[b, :k].astype(np.float64), 0)
+        err = np.linalg.norm(got[b, :k] - ref, axis=1) / np.linalg.norm(ref, axis=1)
+        assert err.max() < 2e-6, (b, int(err.argmax()), err.max())
