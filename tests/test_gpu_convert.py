@@ -91,6 +91,27 @@ def test_q4_quantize_tile_edges(gpu, oracle, dt, shape):
     assert s == s_want == np.float32(2.0 ** -6)
     assert np.array_equal(got, want)
 
+@pytest.mark.parametrize("top", [7.0e-7, 0.0317, 0.25, 1.0, 3.3, 1.7e5, 9.1e22, 3.4e38])
+def test_q4_quantize_quotients(gpu, top):
+    """The codes are those of a correctly rounded fp32 quotient: two million weights
+    within eight units in the last place of every tie, and random ones, for scales
+    from near the smallest to the largest."""
+    ms = gpu
+    say(f"q4_quantize quotients, maximum {top}")
+    n_out, n_in = 512, 4096
+    rng = np.random.default_rng(int(np.float32(top).view(np.uint32)))
+    s = np.float32(float(np.float32(top)) / 7.0)
+    with np.errstate(over="ignore"):
+        tie = ((rng.integers(-7, 7, (n_out, n_in)) + 0.5) * float(s)).astype(np.float32)
+    w = (tie.view(np.int32) + rng.integers(-8, 9, tie.shape, np.int32)).view(np.float32)
+    w[::4] = (rng.uniform(-1, 1, w[::4].shape) * float(np.float32(top))).astype(np.float32)
+    w = np.clip(w, -np.float32(top), np.float32(top))
+    w[3, 5] = np.float32(top)
+    got, s_got = device_quantize(ms, w, ms.Q4_DTYPES["F32"], n_out, n_in)
+    assert np.float32(s_got) == s
+    q = (np.clip(np.rint(w / s), -8, 7) + 8).astype(np.uint8).T
+    assert np.array_equal(got, q[:, 0::2] | (q[:, 1::2] << 4))
+
 
 def test_q4_quantize_grid_ties_and_tiny_blocks(gpu, oracle):
     ms = gpu
