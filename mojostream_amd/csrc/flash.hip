@@ -37,16 +37,16 @@
 // Error against 64 bits (relative 2-norm, normal q, k and v, scores up to 0.3 to 3 times
 // sqrt(hd)): 0.6e-7 to 1.2e-6 at 300 to 2048 rows, 0.5e-7 to 2.0e-7 at 17 rows, below
 // that of an fp32 MFMA kernel with one running sum in each of 18 cells (1.2e-7 to 1.8e-6,
-// 0.6e-7 to 4.6e-7).  The two fp16 parts took 0.7 of this kernel's time, 1.0e-7 to 1.3e-6
+// 0.6e-7 to 4.6e-7).  The two fp16 parts took two thirds of this kernel's time, 1.0e-7 to 1.3e-6
 // on these inputs, 0.8e-7 to 3.2e-7 at 17 rows, and 1e-5 to 5e-5 in rows or dims beside
 // values 2^24 times theirs.
 //
-// Measured (E4B, 2048 rows; the fp32 kernel before): sliding layer 64 to 70 + 16 (prep)
-// against 135 + 17 us (RoPE and append launches), full layer 263 to 295 + 40 + 13.5
-// (merge) against 515 + 29; 14B class, 1000 rows, one layer: 81 + 17.5 against 5.0 ms of
-// chunk launches.  Bound by the fragment reads of one wave per SIMD and by its softmax:
-// the matrix cores are busy 38% of the time at head dim 256.  A short prompt by latency
-// (77 rows: 14.5 + 6.3 against 22.5 + 9.5 us).
+// Measured (E4B, 2048 rows; the fp32 kernel on the same card): sliding layer 63 + 16
+// (prep) against 124 + 15 us (RoPE and append launches), full layer 257 + 40 + 13 (merge)
+// against 471 + 15 + 12 (a slower card: 70 + 17 and 291 + 40 + 13); 14B class, 1000 rows,
+// one layer: 85 + 18 us against 5.0 ms of chunk launches.  Bound by the fragment reads of
+// one wave per SIMD and by its softmax: the matrix cores are busy 38% of the time at head
+// dim 256.  A short prompt by latency (77 rows: 14.7 + 7.1 against 22.5 + 9.5 us).
 #include <algorithm>
 #include <cmath>
 

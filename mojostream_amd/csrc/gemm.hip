@@ -30,10 +30,11 @@
 // What bounds it: at 2048 rows the operand traffic and the instructions between
 // the MFMAs.  A loop of the same MFMAs, LDS reads, unpacking and operand loads
 // runs at 3.14 POP/s on this card (3.76 without the operand loads, 4.33 MFMAs
-// alone; the nominal 5.0 is not reached).  Measured (E4B, 2048 rows; the one-row-
-// tile kernel with compiler scheduling before it): Gate|Up 240 us, 2.68 POP/s
-// (266 us); Down 135 (139), sliding Q|K|V 43.8 (49), full Q|K|V 79 (87); 14B
-// class, 1000 rows: Gate|Up 335 (404), Down 181 (193).
+// alone; the nominal 5.0 is not reached).  Measured in the trace of a whole prefill
+// (E4B, 2048 rows; the one-row-tile kernel with compiler scheduling on the same
+// card): Gate|Up 243 us, 2.65 POP/s (271 us); Down 136 (143), sliding Q|K|V 42.6
+// (48.5), full Q|K|V 79 (88); 14B class, 1000 rows: Gate|Up 361 (396), Down 188
+// (197).  On a slower card Gate|Up takes 263 us, 2.45 POP/s.
 //
 // Short prompts leave most CUs idle where the matrix is narrow (O, Down: 20
 // column tiles): gemm_ksplit splits K over blocks, whose exact int64 sums
