@@ -521,7 +521,9 @@ int ms_runner_run_pipeline(ms_runner *r, float *d_C, const float *d_A, int M,
 /* ---- profiling ------------------------------------------------------------ */
 /* When enabled, ms_decode_run (eager mode) records HIP events around every
  * launch of each kernel class on the library stream; ms_prof_get returns
- * launch counts and total milliseconds per class. */
+ * launch counts and total milliseconds per class.  Enabling starts a new
+ * recording: ms_prof_sweep takes launches recorded since, and none of a model
+ * that was destroyed. */
 #define MS_PROF_CLASSES 8
 int ms_prof_enable(int on);
 int ms_prof_get(int cls, const char **name, long *launches, double *total_ms,

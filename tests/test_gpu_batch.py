@@ -140,11 +140,11 @@ def test_attention_sweep_of_each_decode_path(gpu, kind, B):
             other.close()
 
 
-# heads, kv heads, head dim, circular cache of 64: one to three and six to eight query
+# heads, kv heads, head dim, length of a circular cache (0: linear): one to three and six to eight query
 # heads per kv head, the most heads and the longest rows of the merge in O's quantization
-SHAPES = [(2, 2, 128, 0), (4, 2, 128, 1), (6, 2, 128, 0), (12, 2, 128, 1), (14, 2, 128, 0),
-          (16, 2, 128, 0), (48, 8, 128, 0), (2, 2, 256, 0), (2, 1, 256, 1), (3, 1, 256, 0),
-          (1, 1, 512, 0), (2, 1, 512, 0), (3, 1, 512, 1), (16, 4, 512, 0)]
+SHAPES = [(2, 2, 128, 0), (4, 2, 128, 64), (6, 2, 128, 0), (12, 2, 128, 50), (14, 2, 128, 0),
+          (16, 2, 128, 0), (48, 8, 128, 100), (2, 2, 256, 0), (2, 1, 256, 64), (3, 1, 256, 0),
+          (1, 1, 512, 0), (2, 1, 512, 0), (3, 1, 512, 77), (16, 4, 512, 0)]
 
 
 @pytest.mark.parametrize("B", [1, 3, 6, 16])
@@ -159,8 +159,8 @@ def test_decode_attention_shapes(gpu, nh, nkv, hd, circ, B):
     say(f"decode attention nh={nh} nkv={nkv} hd={hd} circular={circ} B={B}")
     D, n = 256, 133
     desc = ms.LayerDesc(q_dim=nh * hd, kv_dim=nkv * hd, head_dim=hd, n_heads=nh, n_kv_heads=nkv,
-                        rot_dim=hd // 2, theta=1e4, cache_kind=circ,
-                        cache_len=64 if circ else 160, clamp_reads=0)
+                        rot_dim=hd // 2, theta=1e4, cache_kind=int(circ > 0),
+                        cache_len=circ or 141, clamp_reads=0)
     arch = ms.Arch("one", D, D, [desc])
     rng = np.random.default_rng(nh * hd + B)
     w = [rng.integers(1, 16, (k, c // 2 * 2)).astype(np.uint8) for k, c in arch.matrix_shapes(0)]
