@@ -37,9 +37,9 @@
 // Error against 64 bits (relative 2-norm, normal q, k and v, scores up to 0.3 to 3 times
 // sqrt(hd)): 0.6e-7 to 1.2e-6 at 300 to 2048 rows, 0.5e-7 to 2.0e-7 at 17 rows, below
 // that of an fp32 MFMA kernel with one running sum in each of 18 cells (1.2e-7 to 1.8e-6,
-// 0.6e-7 to 4.6e-7).  The two fp16 parts took two thirds of this kernel's time, 1.0e-7 to 1.3e-6
-// on these inputs, 0.8e-7 to 3.2e-7 at 17 rows, and 1e-5 to 5e-5 in rows or dims beside
-// values 2^24 times theirs.
+// 0.6e-7 to 4.6e-7).  The two fp16 parts took two thirds of this kernel's time; 1.0e-7 to
+// 1.3e-6 on these inputs, 0.8e-7 to 3.2e-7 at 17 rows, and 1e-5 to 5e-5 in rows or dims
+// beside values 2^24 times theirs.
 //
 // Measured (E4B, 2048 rows; the fp32 kernel on the same card): sliding layer 63 + 16
 // (prep) against 124 + 15 us (RoPE and append launches), full layer 257 + 40 + 13 (merge)
@@ -324,7 +324,8 @@ __device__ inline float whole(const __bf16 *p, int j) {
 // The queries of one wave over key tiles t0 .. t1, key by key in fp32: for blocks whose
 // tiles hold values that are not finite.  There the products of parts, and those with
 // the weights of masked keys (0 NaN), would reach rows that do not attend to the value.
-// Lanes take 64 keys for the scores and HD / 64 dims each for the output.
+// Lanes take 64 keys for the scores and HD / 64 dims each for the output.  Not tuned: with
+// such a value in every key tile a sliding layer of 2048 rows takes 7.5 ms, a full one 33.
 template <int HD, class Store>
 __device__ inline void flash_plain(const AttnArgs &a, const FlashBuf &f, int h, int q0, int t0,
                                    int t1, int lane, Store store) {
