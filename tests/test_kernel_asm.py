@@ -76,8 +76,8 @@ def _in_flight_at_barriers(lines):
     return list(found.values())
 
 
-def test_checker_counts():
-    """The checker on hand-written blocks: a read before a barrier, one behind a wait,
+def test_in_flight_counts():
+    """The count on hand-written blocks: a read before a barrier, one behind a wait,
     one that reaches the barrier around a loop only."""
     assert _in_flight_at_barriers(["ds_read_b128 v[0:3], v4", "s_barrier"]) == [1]
     assert _in_flight_at_barriers(["ds_read_b128 v[0:3], v4", "ds_read_b128 v[0:3], v4",
