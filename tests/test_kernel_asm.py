@@ -7,7 +7,7 @@ import subprocess
 
 import pytest
 
-HERE = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HERE = os.path.dirname(os.path.dirname(os.path.realpath(__file__)))
 PKG = os.path.join(HERE, "mojostream_amd")
 
 
